@@ -1,0 +1,77 @@
+"""Every tiling of the prefill GEMMs at ragged edges, against FP64 on the GPU.
+
+The dispatch chooses a tiling per shape by a time model; the shapes below reach
+each candidate (largest tiles down to the smallest) with partial token tiles,
+partial row tiles, K that is not whole stages or chunks, and the fallbacks of
+operands that the split form does not take. Bound per output (fp32 sums of
+exact products, one fp16 rounding): 0.5 ulp16(exact) + 2^-19 sum_k |x_k w_k|.
+"""
+
+import pytest
+import torch
+
+from helpers import guarded_out, random_q8
+from venturi_amd import Q8RowSplitWeight
+
+pytestmark = pytest.mark.gpu
+
+
+def ulp16(v):
+    return torch.exp2(torch.floor(torch.log2(v.abs().clamp_min(2.0**-14))) - 10)
+
+
+def assert_bound(got, x, w):
+    """got [T, N] fp16 against x [T, K] @ w[N, K]^T in FP64 (all on the GPU)."""
+    exact, magnitude = x @ w.T, x.abs() @ w.abs().T
+    error = (got.double() - exact).abs()
+    assert bool((error <= 0.5 * ulp16(exact) + 2.0**-19 * magnitude).all())
+
+
+def values(codes, scales, k):
+    n, padded = codes.shape
+    group = padded // scales.shape[1]
+    return (codes.view(n, -1, group).double() * scales.double().unsqueeze(-1)).view(n, padded)[:, :k]
+
+
+def activations(tokens, k, device, seed):
+    return torch.randn(tokens, k, generator=torch.Generator().manual_seed(seed)).half().to(device)
+
+
+# (tokens, rows, columns): 256 x 128, 128 x 128, 64 x 128, 80 x 64, 64 x 64, 48 x 64, 32 x 64 and 32 x 32 tiles.
+Q8_SHAPES = [(257, 14003, 136), (513, 7001, 136), (1025, 7001, 136), (300, 10001, 264), (97, 14003, 136),
+             (33, 20001, 520), (129, 7001, 1032), (81, 14003, 1000), (160, 4100, 1032), (113, 7001, 1032),
+             (79, 14003, 136), (300, 4100, 136), (33, 14003, 136), (65, 10001, 200), (33, 257, 136), (97, 31, 3976)]
+
+
+@pytest.mark.parametrize("tokens,n,k", Q8_SHAPES)
+def test_q8_tilings(backend, device, tokens, n, k):
+    print(f"case q8 prefill tiling tokens={tokens} n={n} k={k}", flush=True)
+    codes, scales = (t.to(device) for t in random_q8(n, k, 31 + n + tokens))
+    x = activations(tokens, k, device, tokens)
+    plan = backend.upload_linear(Q8RowSplitWeight(codes, scales, k), dtype=torch.float16, device=device).prepare(
+        tokens=tokens, route="mfma")
+    guard, out = guarded_out(tokens, n, torch.float16, device)
+    plan.run(x, out=out)
+    assert guard[0] == 47 and guard[-1] == 47
+    assert_bound(out, x.double(), values(codes, scales, k))
+    aligned = torch.empty(tokens, n, dtype=torch.float16, device=device)
+    plan.run(x, out=aligned)  # 16-byte stores where n allows them: the same bits
+    assert torch.equal(aligned, out)
+
+
+@pytest.mark.parametrize("tokens,n,k,shift", [(40, 70, 8, 0), (70, 33, 40, 0), (33, 64, 120, 0), (40, 300, 1000, 1),
+                                              (130, 64, 4096, 1), (33, 3, (1 << 22) + 8, 0)])
+def test_q8_operands_outside_the_split_form(backend, device, tokens, n, k, shift):
+    # Fewer than 128 columns, scales aligned to 2 bytes only, rows past the 32-bit lane offsets.
+    print(f"case q8 prefill fallback tokens={tokens} n={n} k={k} shift={shift}", flush=True)
+    codes, scales = (t.to(device) for t in random_q8(n, k, 5 + n + tokens))
+    padded = codes.shape[1]
+    moved = torch.empty(scales.numel() + shift, dtype=torch.float16, device=device)[shift:].view(scales.shape)
+    moved.copy_(scales)
+    x = activations(tokens, k, device, 9)
+    guard, out = guarded_out(tokens, n, torch.float16, device)
+    lib = backend._native
+    lib.check(lib.venturi_q8_prefill_run(x.data_ptr(), codes.data_ptr(), moved.data_ptr(), out.data_ptr(), tokens, n, k,
+                                         padded, 0, torch.cuda.current_stream(device).cuda_stream))
+    assert guard[0] == 47 and guard[-1] == 47
+    assert_bound(out, x.double(), values(codes, scales, k))

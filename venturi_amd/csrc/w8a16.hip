@@ -6,163 +6,209 @@
 // Each 32-column group's D is one v_mfma_f32_16x16x32_f16 on the fp16
 // activations and the int8 codes converted to fp16 exactly (every x * code
 // product is exact in fp32); the group scale is one fp32 FMA per (t, n, g),
-// groups summed in natural order, so outputs agree with the canonical order
-// (blocks.cu:306-321) to fp32 association, like the decode route.
+// each wave's groups summed in natural order and the waves that split K
+// afterwards, so outputs agree with the canonical order (blocks.cu:306-321) to
+// fp32 association, like the decode route.
 //
-// Tiling: a workgroup of WM x WN waves computes (WM*TI*16) tokens x
-// (WN*TJ*16) rows, each wave TI x TJ tiles of 16 x 16. GS groups are staged at
-// a time in two LDS buffers: the tile's activation rows (32 GS halves each)
-// and weight rows (32 GS codes converted to fp16 once per workgroup) plus the
-// weight scales. Global loads run PF stages ahead in registers; one barrier
-// per stage. LDS rows are 4 GS 16-byte units XOR-swizzled by (row >> 1) so
-// that 16 consecutive rows' fragment reads fall on distinct banks. The output
-// tile leaves through LDS as 16-byte row units.
-#include "common.hpp"
+// Two forms (prefill.hpp), chosen per shape by a measured time model:
+// * cooperative (q8_prefill): WT x WN x WK waves compute (WT*TI*16) tokens x
+//   (WN*TJ*16) rows; a stage is WK groups, staged in two LDS buffers
+//   (activations as fp16, codes biased to unsigned), one group per K wave, one
+//   barrier per stage. For grids that fill the chip.
+// * split (q8_prefill_split): each of WK waves computes the whole TI*16 x TJ*16
+//   tile over its own 128-column chunks through its own LDS region; no barrier
+//   before the sum. For the small grids of short prompts, where it fills the
+//   CUs with K instead of tiles.
+//
+// What binds them is instruction issue: per 16 x 16 tile and group one MFMA
+// (16 cycles of the matrix cores) and four scaling FMAs (16 cycles of the
+// VALU), plus a tile row's share of the code conversion. So both forms issue a
+// tile's MFMA four tiles before its FMAs, replace each activation fragment by
+// the next group's as soon as its last MFMA is issued, and pin that order with
+// scheduling barriers; LDS, memory and matrix work then overlap within a wave.
+// Measured on MI355X against one workgroup of 8 waves with a barrier per group
+// (the form this replaces), us:
+//   tokens x [7168 x 5120]:  64: 74.6 -> 17.0, 200: 76.5 -> 33.3, 512: 77.3 -> 55,
+//     1024: 137 -> 101; [5120 x 17408]: 64: 255 -> 43, 512: 267 -> 178;
+//   [34816 x 5120], 2048 tokens: 1210 -> 1030 (710 TFLOP/s; the wave's VALU and
+//     MFMA issue alone would take about 640).
+#include "prefill.hpp"
 
 #include <algorithm>
 
 namespace vt {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
-// Sixteen int8 codes -> sixteen fp16 values, exactly (u = c + 128 as the
-// mantissa of 1024 + u, then -1152).
-__device__ __forceinline__ void codes16_to_fp16(const uint4 w, uint4& lo, uint4& hi) {
+// Eight biased codes u = c + 128 (one MFMA B fragment of a lane) -> fp16 c.
+__device__ __forceinline__ half8 codes8_to_fp16(const uint2 w) {
     const half2v bias = {static_cast<_Float16>(-1152.0f), static_cast<_Float16>(-1152.0f)};
-    std::uint32_t h[8];
-    const std::uint32_t words[4] = {w.x, w.y, w.z, w.w};
+    const std::uint32_t words[2] = {w.x, w.y};
+    half8 h;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const std::uint32_t u = words[i] ^ 0x80808080u;
-        const half2v a = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, u, 0x05010400u)) + bias;
-        const half2v b = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, u, 0x05030402u)) + bias;
-        h[2 * i] = __builtin_bit_cast(std::uint32_t, a);
-        h[2 * i + 1] = __builtin_bit_cast(std::uint32_t, b);
+    for (int i = 0; i < 2; ++i) {
+        const half2v a = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, words[i], 0x05010400u)) + bias;
+        const half2v b = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, words[i], 0x05030402u)) + bias;
+        h[4 * i] = a[0]; h[4 * i + 1] = a[1]; h[4 * i + 2] = b[0]; h[4 * i + 3] = b[1];
     }
-    lo = make_uint4(h[0], h[1], h[2], h[3]);
-    hi = make_uint4(h[4], h[5], h[6], h[7]);
+    return h;
 }
 
-// XOR swizzle of the 16-byte units of a staged row of U units (4 or 8), so
-// that 16 consecutive rows' fragment reads fall on distinct banks.
-template <int U>
-__device__ __forceinline__ int swizzle(int row) { return (row >> 1) & (U - 1); }
-
-// GS groups of 32 columns per stage.
-template <int WM, int WN, int TI, int TJ, int GS>
+template <int WT, int WN, int WK, int TI, int TJ>
 struct PrefillGeom {
-    static constexpr int kThreads = WM * WN * 64;
-    static constexpr int kTM = WM * TI * 16;      // tokens per workgroup
-    static constexpr int kTN = WN * TJ * 16;      // weight rows per workgroup
-    static constexpr int kU = 4 * GS;             // 16-byte fp16 units per staged row
-    static constexpr int kAUnits = kTM * kU;      // 16-byte activation loads per stage
-    static constexpr int kBUnits = kTN * 2 * GS;  // 16-byte code loads per stage (32 codes a row a group)
+    static constexpr int kThreads = WT * WN * WK * 64;
+    static constexpr int kTM = WT * TI * 16;   // tokens per workgroup
+    static constexpr int kTN = WN * TJ * 16;   // weight rows per workgroup
+    static constexpr int kGroups = WK;         // groups of 32 columns per stage, one per wave of a K set
+    static constexpr int kAU = 4 * kGroups;    // 16-byte units of a staged activation row (fp16)
+    static constexpr int kBU = 2 * kGroups;    // 16-byte units of a staged weight row (int8 codes)
+    static constexpr int kAUnits = kTM * kAU;
+    static constexpr int kBUnits = kTN * kBU;
+    static constexpr int kSUnits = kTN * kGroups;  // scales of a stage
     static constexpr int kAPer = (kAUnits + kThreads - 1) / kThreads;
     static constexpr int kBPer = (kBUnits + kThreads - 1) / kThreads;
-    static_assert(kAUnits % kThreads == 0 || kAUnits < kThreads, "whole loads per thread");
-    static_assert(kBUnits % kThreads == 0 || kBUnits < kThreads, "whole loads per thread");
-    static_assert(kTN * GS <= kThreads, "one scale per thread");
+    static constexpr int kSPer = (kSUnits + kThreads - 1) / kThreads;
+    // A buffer holds whole rounds of the threads' stores, so no store is guarded.
+    static constexpr int kABytes = kAPer * kThreads * 16, kBBytes = kBPer * kThreads * 16, kSBytes = kSPer * kThreads * 4;
+    static constexpr int kStageBytes = kABytes + kBBytes + kSBytes;
+    // Output: the WK partial sums of OI token tiles of every wave at a time, fp32 rows of kTN + 4.
+    static constexpr int kPitch = kTN + 4;
+    static constexpr int out_bytes(int oi) { return WK * WT * oi * 16 * kPitch * 4; }
+    static constexpr int kOI = out_bytes(TI) <= 2 * kStageBytes   ? TI
+                               : TI % 2 == 0 && out_bytes(TI / 2) <= 2 * kStageBytes ? TI / 2
+                               : TI % 4 == 0 && out_bytes(TI / 4) <= 2 * kStageBytes ? TI / 4
+                                                                                      : 1;
+    static constexpr int kLds = 2 * kStageBytes > out_bytes(kOI) ? 2 * kStageBytes : out_bytes(kOI);
+    static_assert(TI % kOI == 0 && kLds <= 160 * 1024, "prefill tile exceeds LDS");
 };
 
-template <int WM, int WN, int TI, int TJ, int GS>
-struct PrefillStage {
-    using G = PrefillGeom<WM, WN, TI, TJ, GS>;
-    uint4 a[G::kAPer];
-    uint4 b[G::kBPer];
-    unsigned short ws;
-};
-
-template <int WM, int WN, int TI, int TJ, int PF, int GS>
-__global__ __launch_bounds__(WM * WN * 64) void q8_prefill(const __half* __restrict__ x,
-                                                          const std::int8_t* __restrict__ codes,
-                                                          const __half* __restrict__ scales, __half* __restrict__ out,
-                                                          int tokens, int n, int k, int padded, int groups) {
-    using G = PrefillGeom<WM, WN, TI, TJ, GS>;
-    using Stage = PrefillStage<WM, WN, TI, TJ, GS>;
-    constexpr int TM = G::kTM, TN = G::kTN, T = G::kThreads, U = G::kU;
-    constexpr int kStageBytes = 2 * (TM + TN) * U * 16 + 2 * GS * TN * 4;
-    constexpr int kPitch = TN + 8;  // halves per token row of the output tile
-    constexpr int kBytes = kStageBytes > TM * kPitch * 2 ? kStageBytes : TM * kPitch * 2;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kBytes];
-    auto* a_lds = reinterpret_cast<uint4(*)[TM * U]>(lds);
-    auto* b_lds = reinterpret_cast<uint4(*)[TN * U]>(lds + 2 * TM * U * 16);
-    auto* ws_lds = reinterpret_cast<float(*)[GS][TN]>(lds + 2 * (TM + TN) * U * 16);
-    const int stages = (groups + GS - 1) / GS;
-
+// PF stages are in flight in registers; Off is the type of the lane offsets
+// (32 bits up to kNarrowK columns).
+template <int WT, int WN, int WK, int TI, int TJ, int PF, class Off>
+__global__ __launch_bounds__(WT * WN * WK * 64, 2) void q8_prefill(const __half* __restrict__ x,
+                                                                  const std::int8_t* __restrict__ codes,
+                                                                  const __half* __restrict__ scales,
+                                                                  __half* __restrict__ out, int tokens, int n, int k,
+                                                                  int padded, int groups, TileOrder order) {
+    using G = PrefillGeom<WT, WN, WK, TI, TJ>;
+    constexpr int TM = G::kTM, TN = G::kTN, T = G::kThreads, AU = G::kAU, BU = G::kBU, KG = G::kGroups;
+    extern __shared__ uint4 q8p_lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
+    const int wk = wave % WK, wn = (wave / WK) % WN, wt = wave / (WK * WN);
     const int q = lane >> 4, r = lane & 15;
-    const int t0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-
-    // Stage s covers groups GS*s .. GS*s + GS - 1 (columns 32 GS s ..). Activation
-    // load u of a thread: unit i = tid + u*T, token i / U of the tile, columns
-    // 8 * (i % U) .. +8 of the stage (zero past k or past the last token: the
-    // address is clamped and the value replaced at the store).
-    const __half* a_src[G::kAPer];
-    int a_col[G::kAPer];
-    bool a_row_ok[G::kAPer];
+    const int tile = tile_of(order);
+    if (tile < 0) return;
+    const int t0 = tile % order.token_tiles * TM, n0 = tile / order.token_tiles * TN;
+    const int stages = (groups + KG - 1) / KG;
+    auto* lds = reinterpret_cast<unsigned char*>(q8p_lds);
+    Off a_off[G::kAPer], b_off[G::kBPer], s_off[G::kSPer];
+    const auto* a_base = reinterpret_cast<const char*>(x + static_cast<std::int64_t>(t0) * k);
+    const auto* b_base = reinterpret_cast<const char*>(codes + static_cast<std::int64_t>(n0) * padded);
+    const auto* s_base = reinterpret_cast<const char*>(scales + static_cast<std::int64_t>(n0) * (padded / 32));
 #pragma unroll
     for (int u = 0; u < G::kAPer; ++u) {
         const int i = tid + u * T;
-        const int tok = i / U;
-        a_row_ok[u] = t0 + tok < tokens;
-        a_src[u] = x + static_cast<std::int64_t>(min(t0 + tok, tokens - 1)) * k;
-        a_col[u] = 8 * (i % U);
+        a_off[u] = 2u * (static_cast<Off>(min(i / AU, tokens - 1 - t0)) * k + 8 * (i % AU));
     }
-    // Code load u: unit i, row i / (2 GS), code bytes 16 * (i % (2 GS)) of the stage.
-    const std::int8_t* b_src[G::kBPer];
 #pragma unroll
     for (int u = 0; u < G::kBPer; ++u) {
         const int i = tid + u * T;
-        b_src[u] = codes + static_cast<std::int64_t>(min(n0 + min(i / (2 * GS), TN - 1), n - 1)) * padded +
-                   16 * (i % (2 * GS));
+        b_off[u] = static_cast<Off>(min(i / BU, n - 1 - n0)) * padded + 16 * (i % BU);
     }
-    // Scale slot sid = T - 1 - tid (staged by the last threads): row sid % TN,
-    // group sid / TN of the stage.
-    const int sid = T - 1 - tid;
-    const int s_grp = sid / TN;
-    const __half* ws_src = scales + static_cast<std::int64_t>(min(n0 + sid % TN, n - 1)) * (padded / 32);
-
-    auto load = [&](int st, Stage& s) __attribute__((always_inline)) {
-        const int c0 = st * 32 * GS;
+#pragma unroll
+    for (int u = 0; u < G::kSPer; ++u) {
+        const int i = tid + u * T;
+        s_off[u] = 2u * (static_cast<Off>(min(i / KG, n - 1 - n0)) * (padded / 32) + i % KG);
+    }
+    // The columns run in stages of 32 KG. When K is not whole stages, the
+    // partial one comes first, so that only the prologue masks and clamps:
+    // stage 0 then starts at the last column base, stage s > 0 at s - 1.
+    constexpr int KC = 32 * KG;
+    const int whole = k / KC, first = whole < stages ? whole : 0, shift = whole < stages ? 1 : 0;
+    uint4 st_a[PF][G::kAPer], st_b[PF][G::kBPer];  // PF stages in flight
+    unsigned short st_s[PF][G::kSPer];
+    // Loads stage columns [c0, c0 + KC), all of them real ones.
+    auto load = [&](int base, auto slot) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < G::kAPer; ++u)
-            if (G::kAUnits >= T || tid < G::kAUnits)
-                s.a[u] = *reinterpret_cast<const uint4*>(a_src[u] + min(c0 + a_col[u], k - 8));
+            st_a[slot][u] = *reinterpret_cast<const uint4*>(a_base + static_cast<std::int64_t>(base) * (2 * KC) + lane_offset(a_off[u]));
 #pragma unroll
         for (int u = 0; u < G::kBPer; ++u)
-            if (G::kBUnits >= T || tid < G::kBUnits)
-                s.b[u] = *reinterpret_cast<const uint4*>(b_src[u] + min(c0, padded - 32 * GS));
-        s.ws = __half_as_ushort(ws_src[min(st * GS + (s_grp < GS ? s_grp : 0), groups - 1)]);
+            st_b[slot][u] = *reinterpret_cast<const uint4*>(b_base + static_cast<std::int64_t>(base) * KC + lane_offset(b_off[u]));
+#pragma unroll
+        for (int u = 0; u < G::kSPer; ++u)
+            st_s[slot][u] = *reinterpret_cast<const unsigned short*>(s_base + static_cast<std::int64_t>(base) * (2 * KG) +
+                                                               lane_offset(s_off[u]));
     };
-    auto store = [&](const Stage& s, int st, int buf) __attribute__((always_inline)) {
-        const int c0 = st * 32 * GS;
+    auto load_edge = [&](int base, auto slot) __attribute__((always_inline)) {
+        const int c0 = base * KC;
 #pragma unroll
         for (int u = 0; u < G::kAPer; ++u) {
-            const int i = tid + u * T;
-            if (G::kAUnits < T && i >= G::kAUnits) break;
-            const int tok = i / U;
-            const bool ok = a_row_ok[u] && c0 + a_col[u] < k;  // k % 8 == 0: a unit is all in or all out
-            a_lds[buf][tok * U + ((i % U) ^ swizzle<U>(tok))] = ok ? s.a[u] : make_uint4(0u, 0u, 0u, 0u);
+            const int col = 8 * ((tid + u * T) % AU);
+            const uint4 v = *reinterpret_cast<const uint4*>(a_base + a_off[u] + 2 * static_cast<std::int64_t>(min(c0, k - 8 - col)));
+            st_a[slot][u] = c0 + col < k ? v : make_uint4(0u, 0u, 0u, 0u);  // k % 8 == 0: a unit is all in or all out
         }
 #pragma unroll
         for (int u = 0; u < G::kBPer; ++u) {
-            const int i = tid + u * T;
-            if (G::kBUnits < T && i >= G::kBUnits) break;
-            const int row = i / (2 * GS), piece = i % (2 * GS);
-            uint4 lo, hi;
-            codes16_to_fp16(s.b[u], lo, hi);
-            b_lds[buf][row * U + ((2 * piece) ^ swizzle<U>(row))] = lo;
-            b_lds[buf][row * U + ((2 * piece + 1) ^ swizzle<U>(row))] = hi;
+            const int col = 16 * ((tid + u * T) % BU);
+            st_b[slot][u] = *reinterpret_cast<const uint4*>(b_base + b_off[u] + static_cast<std::int64_t>(min(c0, padded - 16 - col)));
         }
-        // A group past the last one (groups % GS != 0) carries scale 0.
-        if (sid < TN * GS)
-            ws_lds[buf][s_grp][sid % TN] = st * GS + s_grp < groups ? __half2float(__ushort_as_half(s.ws)) : 0.0f;
+#pragma unroll
+        for (int u = 0; u < G::kSPer; ++u) {
+            const int g = (tid + u * T) % KG;
+            const unsigned short v = *reinterpret_cast<const unsigned short*>(s_base + s_off[u] + 2 * static_cast<std::int64_t>(min(base * KG, groups - 1 - g)));
+            st_s[slot][u] = base * KG + g < groups ? v : 0;  // groups past the last one carry scale 0
+        }
+    };
+    // LDS offsets: a store unit's, and those of the lane's fragments (rows 16
+    // apart share a swizzle, so tiles are whole strides apart).
+    std::uint32_t a_put[G::kAPer], b_put[G::kBPer], s_put[G::kSPer];
+#pragma unroll
+    for (int u = 0; u < G::kAPer; ++u) {
+        const int i = tid + u * T, row = i / AU;
+        a_put[u] = 16 * (row * AU + ((i % AU) ^ swizzle<AU>(row)));
+    }
+#pragma unroll
+    for (int u = 0; u < G::kBPer; ++u) {
+        const int i = tid + u * T, row = i / BU;
+        b_put[u] = G::kABytes + 16 * (row * BU + ((i % BU) ^ swizzle<BU>(row)));
+    }
+#pragma unroll
+    for (int u = 0; u < G::kSPer; ++u) {
+        const int i = tid + u * T;
+        s_put[u] = G::kABytes + G::kBBytes + 4 * (i < G::kSUnits ? (i % KG) * TN + i / KG : i);
+    }
+    const std::uint32_t a_get = 16 * ((wt * TI * 16 + r) * AU + ((4 * wk + q) ^ swizzle<AU>(r)));
+    const std::uint32_t b_get =
+        G::kABytes + 16 * ((wn * TJ * 16 + r) * BU + ((2 * wk + (q >> 1)) ^ swizzle<BU>(r))) + 8 * (q & 1);
+    const std::uint32_t s_get = G::kABytes + G::kBBytes + 4 * (wk * TN + wn * TJ * 16 + r);
+    auto store = [&](int buf, auto slot) __attribute__((always_inline)) {
+        unsigned char* base = lds + buf * G::kStageBytes;
+#pragma unroll
+        for (int u = 0; u < G::kAPer; ++u) *reinterpret_cast<uint4*>(base + a_put[u]) = st_a[slot][u];
+#pragma unroll
+        for (int u = 0; u < G::kBPer; ++u) {
+            const uint4 v = st_b[slot][u];  // biased: code + 128
+            *reinterpret_cast<uint4*>(base + b_put[u]) =
+                make_uint4(v.x ^ 0x80808080u, v.y ^ 0x80808080u, v.z ^ 0x80808080u, v.w ^ 0x80808080u);
+        }
+#pragma unroll
+        for (int u = 0; u < G::kSPer; ++u)
+            *reinterpret_cast<float*>(base + s_put[u]) = __half2float(__ushort_as_half(st_s[slot][u]));
+    };
+    half8 fa[TI];
+    uint2 rb[TJ];
+    float ws[TJ];
+    auto read_a = [&](int buf, int i) __attribute__((always_inline)) {
+        fa[i] = *reinterpret_cast<const half8*>(lds + buf * G::kStageBytes + a_get + i * 256 * AU);
+    };
+    auto read_b = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            rb[j] = *reinterpret_cast<const uint2*>(lds + buf * G::kStageBytes + b_get + j * 256 * BU);
+            ws[j] = *reinterpret_cast<const float*>(lds + buf * G::kStageBytes + s_get + j * 64);
+        }
     };
 
     float4v y[TI][TJ];
@@ -171,129 +217,315 @@ __global__ __launch_bounds__(WM * WN * 64) void q8_prefill(const __half* __restr
 #pragma unroll
         for (int j = 0; j < TJ; ++j) y[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // A stage's fragments, read from LDS before the next stage is converted
-    // into the other buffer, so the conversion covers the read latency.
-    struct Frag {
-        half8 fa[GS][TI];
-        half8 fb[GS][TJ];
-        float wsv[GS][TJ];
-    };
-    auto read = [&](int buf, Frag& f) __attribute__((always_inline)) {
+    // Stage s is multiplied from registers while stage s + 1 is read from LDS
+    // (each activation fragment as soon as its register is free), stage s + 2
+    // is written to LDS and stage s + 3 is requested from memory.
+    const int last = max(whole - 1, 0);  // the last whole stage's column base
+    load_edge(first, Slot<0>{});
+    store(0, Slot<0>{});
+    if (whole == 0) {
+        // The partial stage is the only one: the loop's requests (never
+        // consumed) stay on column 0 of their rows.
 #pragma unroll
-        for (int gg = 0; gg < GS; ++gg) {
+        for (int u = 0; u < G::kAPer; ++u) a_off[u] -= 16u * ((tid + u * T) % AU);
+#pragma unroll
+        for (int u = 0; u < G::kBPer; ++u) b_off[u] -= 16u * ((tid + u * T) % BU);
+#pragma unroll
+        for (int u = 0; u < G::kSPer; ++u) s_off[u] -= 2u * ((tid + u * T) % KG);
+    }
+    if (stages > 1) {
+        load(1 - shift, Slot<0>{});
+        store(1, Slot<0>{});
+    }
+    each_slot<PF>([&](auto p) __attribute__((always_inline)) { load(min(2 + p - shift, last), p); });
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TI; ++i) read_a(0, i);
+    read_b(0);
+    __syncthreads();
+    constexpr int kTiles = TI * TJ, kAhead = kTiles < 4 ? 1 : 4;
+    constexpr int kStoreAt = kTiles / 4, kLoadAt = kTiles / 4 + 2, kReadB = TJ + kTiles / 4;
+    auto step = [&](int sg, auto slot) __attribute__((always_inline)) {
+        const int next = (sg + 1) & 1;
+        const float4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        half8 fb[TJ];
+        float wj[TJ];
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) wj[j] = ws[j];
+        // Tile t's MFMA is issued kAhead tiles before its four scaling FMAs, so
+        // the matrix cores run under the wave's own VALU work.
+        float4v d[kAhead];
+#pragma unroll
+        for (int t = 0; t < kTiles + kAhead; ++t) {
+            if (t >= kAhead) {
+                const int f = t - kAhead, i = f / TJ, j = f % TJ;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[i][j][e] = fmaf(d[f % kAhead][e], wj[j], y[i][j][e]);
+            }
+            if (t < TJ) fb[t] = codes8_to_fp16(rb[t]);
+            if (t < kTiles) {
+                d[t % kAhead] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[t / TJ], fb[t % TJ], zero, 0, 0, 0);
+                if (t % TJ == TJ - 1) read_a(next, t / TJ);
+            }
+            if (t == kStoreAt) store(sg & 1, slot);
+            if (t == kLoadAt) load(min(sg + 2 + PF - shift, last), slot);
+            if (t == kReadB) read_b(next);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+    };
+    int sg = 0;
+    for (; sg + PF <= stages; sg += PF) {
+        each_slot<PF>([&](auto p) __attribute__((always_inline)) { step(sg + p, p); });
+    }
+    each_slot<PF - 1>([&](auto p) __attribute__((always_inline)) {
+        if (sg + p < stages) step(sg + p, p);
+    });
+
+    // The partial sums of the WK waves through LDS, OI token tiles of every
+    // wave at a time.
+    auto* o_lds = reinterpret_cast<float*>(q8p_lds);
+    constexpr int OI = G::kOI, P = G::kPitch, kRows = WT * OI * 16;
+#pragma unroll
+    for (int c = 0; c < TI / OI; ++c) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < OI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    o_lds[(wk * kRows + (wt * OI + i) * 16 + 4 * q + e) * P + wn * TJ * 16 + j * 16 + r] = y[c * OI + i][j][e];
+        __syncthreads();
+        store_partials<WK, kRows, TN, P, T>(o_lds, out, tokens, n, n0, [&](int row) {
+            return t0 + (row / (OI * 16)) * TI * 16 + c * OI * 16 + row % (OI * 16);
+        });
+    }
+}
+
+template <int WT, int WN, int WK, int TI, int TJ, int PF, class Off = std::uint32_t>
+void launch_prefill(const __half* x, const std::int8_t* codes, const __half* scales, __half* out, int tokens, int n,
+                    int k, int padded, hipStream_t stream) {
+    using G = PrefillGeom<WT, WN, WK, TI, TJ>;
+    const auto kernel = q8_prefill<WT, WN, WK, TI, TJ, PF, Off>;
+    const TileOrder order = tile_order(tokens, G::kTM, n, G::kTN);
+    static const bool raised = (raise_lds(kernel, G::kLds), true);
+    static_cast<void>(raised);
+    kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(x, codes, scales, out, tokens, n, k, padded,
+                                                               (k + 31) / 32, order);
+}
+
+template <int WK, int TI, int TJ>
+struct SplitGeom {
+    static constexpr int kThreads = WK * 64;
+    static constexpr int kTM = TI * 16, kTN = TJ * 16;
+    static constexpr int kA = 2 * TI;                   // 16-byte activation loads of a lane per step (64 columns)
+    static constexpr int kB = TJ;                       // 16-byte code loads of a lane per step
+    static constexpr int kABytes = kTM * 128, kBBytes = kTN * 64, kSBytes = 4 * 64 * 4;
+    static constexpr int kWave = kABytes + kBBytes + kSBytes;
+    static constexpr int kPitch = kTN + 4;
+    static constexpr int kOut = WK * kTM * kPitch * 4;
+    static constexpr int kLds = WK * kWave > kOut ? WK * kWave : kOut;
+    static_assert(kTN <= 64 && kLds <= 160 * 1024, "split tile exceeds LDS");
+};
+
+template <int WK, int TI, int TJ>
+__global__ __launch_bounds__(WK * 64, 2) void q8_prefill_split(const __half* __restrict__ x,
+                                                              const std::int8_t* __restrict__ codes,
+                                                              const __half* __restrict__ scales,
+                                                              __half* __restrict__ out, int tokens, int n, int k,
+                                                              int padded, int groups, TileOrder order) {
+    using G = SplitGeom<WK, TI, TJ>;
+    constexpr int TM = G::kTM, TN = G::kTN;
+    extern __shared__ uint4 q8p_lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = lane >> 4, r = lane & 15;
+    const int tile = tile_of(order);
+    if (tile < 0) return;
+    const int t0 = tile % order.token_tiles * TM, n0 = tile / order.token_tiles * TN;
+    const int chunks = padded / 128;
+    auto* lds = reinterpret_cast<unsigned char*>(q8p_lds) + wave * G::kWave;
+
+    float4v y[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) y[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+
+    if (wave < chunks) {
+        // Lane offsets of the loads: activation unit u is row lane / 8 + 8 u of
+        // the tile, 16-byte unit lane % 8 of its 128 bytes; code unit u row
+        // lane / 4 + 16 u, unit lane % 4 of its 64 bytes; scales row lane.
+        std::uint32_t a_off[G::kA], b_off[G::kB], s_off;
+        const auto* a_base = reinterpret_cast<const char*>(x + static_cast<std::int64_t>(t0) * k);
+        const auto* b_base = reinterpret_cast<const char*>(codes + static_cast<std::int64_t>(n0) * padded);
+        const auto* s_base = reinterpret_cast<const char*>(scales + static_cast<std::int64_t>(n0) * (padded / 32));
+#pragma unroll
+        for (int u = 0; u < G::kA; ++u)
+            a_off[u] = 2u * (static_cast<std::uint32_t>(min(lane / 8 + 8 * u, tokens - 1 - t0)) * k + 8 * (lane % 8));
+#pragma unroll
+        for (int u = 0; u < G::kB; ++u)
+            b_off[u] = static_cast<std::uint32_t>(min(lane / 4 + 16 * u, n - 1 - n0)) * padded + 16 * (lane % 4);
+        s_off = 2u * static_cast<std::uint32_t>(min(lane, n - 1 - n0)) * (padded / 32);
+        uint4 st_a[G::kA], st_b[G::kB];
+        uint2 st_s;
+        // Step `sub` (64 columns) of chunk c, all of them real columns.
+        auto load = [&](int c, auto sub) __attribute__((always_inline)) {
+            const std::int64_t c0 = static_cast<std::int64_t>(c) * 128 + sub * 64;
+#pragma unroll
+            for (int u = 0; u < G::kA; ++u) st_a[u] = *reinterpret_cast<const uint4*>(a_base + 2 * c0 + lane_offset(a_off[u]));
+#pragma unroll
+            for (int u = 0; u < G::kB; ++u) st_b[u] = *reinterpret_cast<const uint4*>(b_base + c0 + lane_offset(b_off[u]));
+            if constexpr (sub == 0)
+                st_s = *reinterpret_cast<const uint2*>(s_base + 8 * static_cast<std::int64_t>(c) + lane_offset(s_off));
+        };
+        // The same for the last chunk: columns past k are zero (k % 8 == 0: a
+        // unit is all in or all out), groups past the last one carry scale 0.
+        auto load_edge = [&](int c, auto sub) __attribute__((always_inline)) {
+            load(0, sub);
+            const int c0 = c * 128 + sub * 64, col = c0 + 8 * (lane % 8);
+#pragma unroll
+            for (int u = 0; u < G::kA; ++u) {
+                const uint4 v = *reinterpret_cast<const uint4*>(
+                    a_base + a_off[u] + 2 * static_cast<std::int64_t>(min(c0, k - 8 - 8 * (lane % 8))));
+                st_a[u] = col < k ? v : make_uint4(0u, 0u, 0u, 0u);
+            }
+#pragma unroll
+            for (int u = 0; u < G::kB; ++u) st_b[u] = *reinterpret_cast<const uint4*>(b_base + c0 + b_off[u]);
+            if constexpr (sub == 0) {
+                const uint2 v = *reinterpret_cast<const uint2*>(s_base + 8 * static_cast<std::int64_t>(c) + s_off);
+                const int real = groups - 4 * c;  // 1 .. 4
+                st_s.x = real >= 2 ? v.x : v.x & 0xffffu;
+                st_s.y = real >= 4 ? v.y : real == 3 ? v.y & 0xffffu : 0u;
+            }
+        };
+        const std::uint32_t a_put = 16 * ((lane / 8) * 8 + ((lane % 8) ^ swizzle<8>(lane / 8)));
+        const std::uint32_t a_put_odd = 16 * ((lane / 8) * 8 + ((lane % 8) ^ swizzle<8>(lane / 8 + 8)));
+        const std::uint32_t b_put = G::kABytes + 16 * ((lane / 4) * 4 + ((lane % 4) ^ swizzle<4>(lane / 4)));
+        const std::uint32_t s_put = G::kABytes + G::kBBytes + 4 * lane;
+        std::uint32_t a_get[2], b_get[2];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            a_get[g] = 16 * (r * 8 + ((4 * g + q) ^ swizzle<8>(r)));
+            b_get[g] = G::kABytes + 16 * (r * 4 + ((2 * g + (q >> 1)) ^ swizzle<4>(r))) + 8 * (q & 1);
+        }
+        const std::uint32_t s_get = G::kABytes + G::kBBytes + 4 * r;
+        auto store = [&](auto sub) __attribute__((always_inline)) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int u = 0; u < G::kA; ++u)
+                *reinterpret_cast<uint4*>(lds + (u & 1 ? a_put_odd : a_put) + u * 1024) = st_a[u];
+#pragma unroll
+            for (int u = 0; u < G::kB; ++u) {
+                const uint4 v = st_b[u];  // biased: code + 128
+                *reinterpret_cast<uint4*>(lds + b_put + u * 1024) =
+                    make_uint4(v.x ^ 0x80808080u, v.y ^ 0x80808080u, v.z ^ 0x80808080u, v.w ^ 0x80808080u);
+            }
+            if constexpr (sub == 0) {
+                const float f[4] = {half_lo(st_s.x), half_hi(st_s.x), half_lo(st_s.y), half_hi(st_s.y)};
+#pragma unroll
+                for (int g = 0; g < 4; ++g) *reinterpret_cast<float*>(lds + s_put + 256 * g) = f[g];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        };
+        half8 fa[TI];
+        uint2 rb[TJ];
+        float ws[TJ];
+        auto read_a = [&](int g, int i) __attribute__((always_inline)) {
+            fa[i] = *reinterpret_cast<const half8*>(lds + a_get[g & 1] + i * 2048);
+        };
+        auto read_b = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < TJ; ++j) {
-                const int row = wn * TJ * 16 + j * 16 + r;
-                f.fb[gg][j] = __builtin_bit_cast(half8, b_lds[buf][row * U + ((4 * gg + q) ^ swizzle<U>(row))]);
-                f.wsv[gg][j] = ws_lds[buf][gg][row];
+                rb[j] = *reinterpret_cast<const uint2*>(lds + b_get[g & 1] + j * 1024);
+                ws[j] = *reinterpret_cast<const float*>(lds + s_get + 256 * g + j * 64);
             }
-#pragma unroll
-            for (int i = 0; i < TI; ++i) {
-                const int tok = wm * TI * 16 + i * 16 + r;
-                f.fa[gg][i] = __builtin_bit_cast(half8, a_lds[buf][tok * U + ((4 * gg + q) ^ swizzle<U>(tok))]);
-            }
+        };
+
+        // The wave's chunks run from the last one down, so only the prologue
+        // sees the edge; requests past the wave's last chunk go to chunk 0 and
+        // are never consumed.
+        int c = chunks - 1 - wave;
+        if (c == chunks - 1) {
+            load_edge(c, Slot<0>{});
+            store(Slot<0>{});
+            load_edge(c, Slot<1>{});
+        } else {
+            load(c, Slot<0>{});
+            store(Slot<0>{});
+            load(c, Slot<1>{});
         }
-    };
-    // Groups in natural order; each tile's MFMA is followed by the scaling of
-    // an earlier tile (the schedule below pins the interleave, so the matrix
-    // cores run under the wave's own VALU work instead of the epilogue being
-    // gathered after the stage's barrier).
-    auto math = [&](const Frag& f) __attribute__((always_inline)) {
-        const float4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int gg = 0; gg < GS; ++gg)
+        for (int i = 0; i < TI; ++i) read_a(0, i);
+        read_b(0);
+        constexpr int kTiles = TI * TJ, kAhead = kTiles < 5 ? 2 : 4;
+        for (; c >= 0; c -= WK) {
+            const int next = max(c - WK, 0);
+            each_slot<4>([&](auto g) __attribute__((always_inline)) {
+                // Group g of the chunk is multiplied from registers; each
+                // activation fragment is replaced by the next group's as soon
+                // as it is free. The LDS holds one step (two groups): after the
+                // last reads of a step the next one is written over it (a
+                // wave's LDS accesses stay in order, and no other wave sees
+                // its region), and the one after that is requested.
+                const float4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                half8 fb[TJ];
+                float wj[TJ];
 #pragma unroll
-            for (int i = 0; i < TI; ++i)
+                for (int j = 0; j < TJ; ++j) wj[j] = ws[j];
+                float4v d[kAhead];
 #pragma unroll
-                for (int j = 0; j < TJ; ++j) {
-                    const float4v d = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.fa[gg][i], f.fb[gg][j], zero, 0, 0, 0);
+                for (int t = 0; t < kTiles + kAhead; ++t) {
+                    if (t >= kAhead) {
+                        const int f = t - kAhead, i = f / TJ, j = f % TJ;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) y[i][j][e] = fmaf(d[e], f.wsv[gg][j], y[i][j][e]);
+                        for (int e = 0; e < 4; ++e) y[i][j][e] = fmaf(d[f % kAhead][e], wj[j], y[i][j][e]);
+                    }
+                    if (t < TJ) fb[t] = codes8_to_fp16(rb[t]);
+                    if (t == 0 && g == 1) {
+                        store(Slot<1>{});
+                        load(next, Slot<0>{});
+                    }
+                    if (t == 0 && g == 3) {
+                        store(Slot<0>{});
+                        load(next, Slot<1>{});
+                    }
+                    if (t < kTiles) {
+                        d[t % kAhead] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[t / TJ], fb[t % TJ], zero, 0, 0, 0);
+                        if (t % TJ == TJ - 1) read_a(g + 1, t / TJ);
+                    }
+                    if (t == TJ) read_b((g + 1) & 3);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-#pragma unroll
-        for (int t = 0; t < GS * TI * TJ; ++t) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
+            });
         }
-    };
+    }
 
-    // Stage s is loaded PF stages ahead into register stage s % PF, converted
-    // into LDS buffer s % 2 while stage s - 1 is multiplied out, and consumed
-    // after the barrier that ends that step. Full rounds of PF steps have no
-    // branch on the stage index (loads and stores past the last stage are
-    // clamped and never consumed); the last partial round is guarded.
-    static_assert(PF % 2 == 0, "the buffer parity of a step is fixed within a round");
-    Stage st[PF];
-#pragma unroll
-    for (int s = 0; s < PF; ++s) load(min(s, stages - 1), st[s]);
-    store(st[0], 0, 0);
-    load(min(PF, stages - 1), st[0]);
+    // The partial sums of the waves through LDS.
+    auto* o_lds = reinterpret_cast<float*>(q8p_lds);
+    constexpr int P = G::kPitch;
     __syncthreads();
-    int g0 = 0;
-    for (; g0 + PF <= stages; g0 += PF) {
-#pragma unroll
-        for (int s = 0; s < PF; ++s) {
-            Frag f;
-            read(s & 1, f);
-            const int nxt = min(g0 + s + 1, stages - 1);
-            store(st[(s + 1) % PF], nxt, (s + 1) & 1);
-            load(min(g0 + s + 1 + PF, stages - 1), st[(s + 1) % PF]);
-            math(f);
-            __syncthreads();
-        }
-    }
-    if (g0 < stages) {
-#pragma unroll
-        for (int s = 0; s < PF; ++s) {
-            if (g0 + s < stages) {
-                Frag f;
-                read(s & 1, f);
-                store(st[(s + 1) % PF], min(g0 + s + 1, stages - 1), (s + 1) & 1);
-                math(f);
-                __syncthreads();
-            }
-        }
-    }
-
-    // Output tile: fp16 through LDS (token rows padded by 8 halves so the four
-    // token quads of a wave's 2-byte writes fall on distinct banks), then
-    // 16-byte row units to HBM.
-    auto* o_lds = reinterpret_cast<__half*>(lds);
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                o_lds[(wm * TI * 16 + i * 16 + 4 * q + e) * kPitch + wn * TJ * 16 + j * 16 + r] =
-                    from_f32<__half>(y[i][j][e]);
+            for (int e = 0; e < 4; ++e) o_lds[(wave * TM + i * 16 + 4 * q + e) * P + j * 16 + r] = y[i][j][e];
     __syncthreads();
-    const bool vec = (n % 8) == 0 && (reinterpret_cast<std::uintptr_t>(out) & 15) == 0;
-    constexpr int kUnits = TM * TN / 8;
-#pragma unroll
-    for (int u = tid; u < kUnits; u += T) {
-        const int tok = u / (TN / 8), c = (u % (TN / 8)) * 8;
-        const int t = t0 + tok, col = n0 + c;
-        if (t >= tokens || col >= n) continue;
-        const __half* src = o_lds + tok * kPitch + c;
-        __half* dst = out + static_cast<std::int64_t>(t) * n + col;
-        if (vec) {
-            *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
-        } else {
-            for (int e = 0; e < 8 && col + e < n; ++e) dst[e] = src[e];
-        }
-    }
+    store_partials<WK, TM, TN, P, G::kThreads>(o_lds, out, tokens, n, n0, [&](int row) { return t0 + row; });
 }
 
-template <int WM, int WN, int TI, int TJ, int PF, int GS = 1>
-void launch_prefill(const __half* x, const std::int8_t* codes, const __half* scales, __half* out, int tokens, int n,
-                    int k, int padded, hipStream_t stream) {
-    using G = PrefillGeom<WM, WN, TI, TJ, GS>;
-    const int groups = (k + 31) / 32;
-    const dim3 grid((n + G::kTN - 1) / G::kTN, (tokens + G::kTM - 1) / G::kTM);
-    require(grid.y <= 65535, "token tiles exceed the launch grid");
-    q8_prefill<WM, WN, TI, TJ, PF, GS><<<grid, G::kThreads, 0, stream>>>(x, codes, scales, out, tokens, n, k,
-                                                                        padded, groups);
+template <int WK, int TI, int TJ>
+void launch_split(const __half* x, const std::int8_t* codes, const __half* scales, __half* out, int tokens, int n,
+                  int k, int padded, hipStream_t stream) {
+    using G = SplitGeom<WK, TI, TJ>;
+    const auto kernel = q8_prefill_split<WK, TI, TJ>;
+    const TileOrder order = tile_order(tokens, G::kTM, n, G::kTN);
+    static const bool raised = (raise_lds(kernel, G::kLds), true);
+    static_cast<void>(raised);
+    kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(x, codes, scales, out, tokens, n, k, padded,
+                                                               (k + 31) / 32, order);
 }
 
 // The exact two-term fp16 form of Q8 weights, for the dense route: row j of
@@ -365,24 +597,34 @@ void q8_prefill_launch(const void* x, const std::int8_t* codes, const __half* sc
     require(dtype == kF16, "the Q8 prefill GEMM takes FP16 activations");
     require(k % 8 == 0 && aligned(x, 16), "the Q8 prefill GEMM needs k % 8 == 0 and 16-byte aligned x");
     require(aligned(codes, 16) && aligned(scales, 2) && aligned(out, 2), "misaligned Q8 operand");
-    // Four tilings of 8 waves: 256 x 128 (waves of 64 x 64), 128 x 160
-    // (32 x 80), 128 x 224 (32 x 112), each one workgroup per CU, and
-    // 128 x 128 with two groups per stage (the small grids' tiling). The
-    // launch takes the one with the least time over whole tile rounds on the
-    // CUs, from their measured rates per unit of work (1 : 0.76 : 0.89 :
-    // 0.80): small grids take 128 x 128 as before; at M = 2048,
-    // 7168 rows take 128 x 224 (512 tiles, two rounds), 5120 rows 128 x 160
-    // (512 tiles), 34816 rows 256 x 128 (config-2 W8A16 QKV / o_proj / gate+up
-    // / down 303 / 306 / 1225 / 818 -> 297 / 256 / 1225 / 685 us; same bits
-    // in every tiling, the groups being summed in natural order).
     const auto* xp = static_cast<const __half*>(x);
     auto* op = static_cast<__half*>(out);
-    constexpr GemmTiling kTilings[4] = {{256, 128, 1.0}, {128, 160, 0.76}, {128, 224, 0.89}, {128, 128, 0.80}};
-    const int best = pick_tiling(tokens, n, kTilings);
-    if (best == 0) launch_prefill<4, 2, 4, 4, 2, 1>(xp, codes, scales, op, tokens, n, k, padded, stream);
-    else if (best == 1) launch_prefill<4, 2, 2, 5, 2, 1>(xp, codes, scales, op, tokens, n, k, padded, stream);
-    else if (best == 2) launch_prefill<4, 2, 2, 7, 2, 1>(xp, codes, scales, op, tokens, n, k, padded, stream);
-    else launch_prefill<2, 4, 4, 2, 2, 2>(xp, codes, scales, op, tokens, n, k, padded, stream);
+    if (k > kNarrowK) {  // rows too long for 32-bit lane offsets
+        launch_prefill<1, 2, 4, 4, 4, 1, std::uint64_t>(xp, codes, scales, op, tokens, n, k, padded, stream);
+        return;
+    }
+    // The tiling with the least predicted time; the constants are a fit to 115
+    // shapes (33-2048 tokens, 1024-34816 rows, 1024-25600 columns; each
+    // candidate timed on each shape on MI355X): the choice is within 8% of the
+    // fastest candidate on every one of them and 0.4% on average.
+    constexpr PrefillTiling kTilings[8] = {
+        {256, 128, 1, 0.0, 6.67, 18.50, 18.50}, {128, 128, 1, 0.0, 6.84, 9.59, 9.59}, {64, 128, 1, 0.3, 4.87, 5.93, 5.93},
+        {80, 64, 2, 0.0, 6.93, 3.75, 9.03},     {64, 64, 2, 2.2, 3.33, 3.42, 7.26},   {48, 64, 2, 2.6, 2.48, 2.80, 6.13},
+        {32, 64, 2, 2.9, 1.04, 2.51, 5.16},     {32, 32, 1, 2.3, 0.45, 1.88, 1.88}};
+    int best = fastest_tiling(kTilings, tokens, n, k);
+    // The split form reads a chunk's four scales as one 8-byte word and needs
+    // one whole chunk.
+    if (best >= 3 && (k < 128 || !aligned(scales, 8))) best = 2;
+    switch (best) {
+        case 0: launch_prefill<2, 2, 2, 8, 4, 1>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 1: launch_prefill<1, 2, 4, 8, 4, 1>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 2: launch_prefill<1, 2, 4, 4, 4, 2>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 3: launch_split<4, 5, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 4: launch_split<4, 4, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 5: launch_split<4, 3, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 6: launch_split<4, 2, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        default: launch_split<8, 2, 2>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+    }
 }
 
 }  // namespace vt
