@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from helpers import guarded_out, random_q8
-from venturi_amd import Q8RowSplitWeight
+from venturi_amd import Q8RowSplitWeight, prepare_q8_dp4a
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +75,57 @@ def test_q8_operands_outside_the_split_form(backend, device, tokens, n, k, shift
                                          padded, 0, torch.cuda.current_stream(device).cuda_stream))
     assert guard[0] == 47 and guard[-1] == 47
     assert_bound(out, x.double(), values(codes, scales, k))
+
+
+def represented(workspace, tokens, k, passes):
+    """FP64 values of the quantized activations in an A8 workspace."""
+    groups = (k + 31) // 32
+    count = tokens * groups
+    codes = workspace[: count * 32 * passes].view(torch.int8).view(passes, tokens, groups, 32).double()
+    scales = workspace[count * 32 * passes :].view(torch.float32).view(passes, tokens, groups, 1).double()
+    return (codes * scales).sum(0).view(tokens, groups * 32)[:, :k]
+
+
+# 256 x 128, 128 x 128, 64 x 128, 64 x 64 (eight and four K waves), 48 x 64 (four and eight), 32 x 64 and 32 x 32
+# tiles; whole and partial stages and chunks (K % 128), K below one chunk, one and two passes.
+A8_SHAPES = [(257, 14003, 136, 1), (513, 7001, 128, 2), (129, 14003, 136, 1), (257, 7001, 300, 1), (65, 10001, 136, 1),
+             (33, 14003, 256, 1), (97, 7001, 520, 1), (160, 4100, 520, 2), (97, 14003, 4104, 1), (200, 7001, 2056, 2),
+             (65, 10001, 1032, 1), (79, 10001, 519, 2), (33, 14003, 136, 2), (97, 4100, 520, 1), (33, 4100, 1032, 1),
+             (47, 4100, 520, 2), (65, 257, 136, 1), (33, 257, 129, 2), (81, 31, 3971, 1), (65, 70, 31, 2), (40, 33, 127, 1)]
+
+
+@pytest.mark.parametrize("tokens,n,k,passes", A8_SHAPES)
+def test_a8_tilings(backend, device, tokens, n, k, passes):
+    print(f"case a8 prefill tiling tokens={tokens} n={n} k={k} passes={passes}", flush=True)
+    codes, scales = (t.to(device) for t in random_q8(n, k, 57 + n + tokens))
+    x = activations(tokens, k, device, tokens + 1)
+    x[3, min(k - 1, 40)] = float("inf")  # that group: zero codes, NaN scale; the token's outputs are NaN
+    plan = prepare_q8_dp4a(backend.upload_linear(Q8RowSplitWeight(codes, scales, k), dtype=torch.float16, device=device),
+                           tokens=tokens, residual_compensation=passes == 2, route="mfma")
+    workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=device)
+    guard, out = guarded_out(tokens, n, torch.float16, device)
+    plan.run(x, out=out, workspace=workspace)
+    assert guard[0] == 47 and guard[-1] == 47
+    keep = torch.arange(tokens, device=device) != 3
+    assert bool(torch.isnan(out[3]).all())
+    assert_bound(out[keep], represented(workspace, tokens, k, passes)[keep], values(codes, scales, k))
+    aligned = torch.empty(tokens, n, dtype=torch.float16, device=device)
+    plan.project(out=aligned, workspace=workspace)  # 16-byte stores where n allows them: the same bits
+    assert torch.equal(aligned[keep], out[keep])
+
+
+@pytest.mark.parametrize("tokens,n,k,passes", [(130, 300, 1000, 1), (70, 64, 4096, 2)])
+def test_a8_scales_aligned_to_two_bytes(backend, device, tokens, n, k, passes):
+    print(f"case a8 prefill fallback tokens={tokens} n={n} k={k}", flush=True)
+    codes, scales = (t.to(device) for t in random_q8(n, k, 5 + n + tokens))
+    moved = torch.empty(scales.numel() + 1, dtype=torch.float16, device=device)[1:].view(scales.shape)
+    moved.copy_(scales)
+    x = activations(tokens, k, device, 9)
+    lib, stream = backend._native, torch.cuda.current_stream(device).cuda_stream
+    workspace = torch.empty(lib.venturi_q8_dp4a_bytes(tokens, k, passes), dtype=torch.uint8, device=device)
+    lib.check(lib.venturi_q8_dp4a_quantize(x.data_ptr(), workspace.data_ptr(), workspace.numel(), tokens, k, passes, stream))
+    guard, out = guarded_out(tokens, n, torch.float16, device)
+    lib.check(lib.venturi_q8_a8_gemm_run(workspace.data_ptr(), workspace.numel(), codes.data_ptr(), moved.data_ptr(),
+                                         out.data_ptr(), tokens, n, k, codes.shape[1], passes, stream))
+    assert guard[0] == 47 and guard[-1] == 47
+    assert_bound(out, represented(workspace, tokens, k, passes), values(codes, scales, k))

@@ -1,341 +1,562 @@
-// W8A8 projection for many tokens on matrix cores with a free fp32 order
-// (the "mfma" A8 route).
+// W8A8 projection for many tokens on int8 matrix cores with a free fp32 order
+// (the "mfma" A8 route above the decode kernels).
 //
-// out[t][n] = fp16( sum_g d[t][n][g] * (ws[n][g] * as[t][g]) )   (one pass)
+// out[t][n] = fp16( sum_p sum_g d[p][t][n][g] * ws[n][g] * as[p][t][g] )
 //
-// d is the exact integer dot of the group's 32 activation and weight codes:
-// int8 codes are exact in fp16, every product of two codes is an integer
-// below 2^14 and every partial sum of 32 of them an integer below 2^19, so
-// v_mfma_f32_16x16x32_f16 returns d exactly as fp32 (the int32 accumulator
-// of the reference, q8_dp4a.cuh:47-58). The group scaling is the reference's
-// (one fp32 product ws*as, one FMA), but groups are accumulated in natural
-// order into one fp32 sum per output instead of the reference's 32 lane
-// slots and shuffle tree (q8_dp4a.cuh:59-70), so outputs agree with the
-// reference to fp32 association, not bit for bit. With two passes (the
-// residual profile) the group term is (d0 * as0 + d1 * as1) * ws.
+// d is the exact integer dot of the group's 32 activation and weight codes
+// (q8_dp4a.cuh:47-58), one v_mfma_i32_16x16x32_i8 on the codes as they are
+// stored. The accumulator starts at the bit pattern of 1.5 * 2^23, so its 32
+// bits read as a float are exactly 1.5 * 2^23 + d (|d| < 2^19) without a
+// conversion, and one FMA with ws takes the offset off again:
+//   t = fma(1.5 * 2^23 + d, ws, -1.5 * 2^23 * ws) = round(d * ws),
+// because 1.5 * 2^23 * ws is exact (an 11-bit significand times 3); then
+// y = fma(t, as, y). Two VALU instructions per output and group, as the
+// reference's product and FMA (q8_dp4a.cuh:59-70), with one fp32 rounding
+// besides the sum's as there. Groups are summed in natural order per wave and
+// the waves that split K afterwards, so outputs agree with the reference to
+// fp32 association, not bit for bit. The second pass of the residual profile
+// is a second run over the same weight columns. (A row with a non-finite
+// weight scale, which the format excludes, gives NaN.)
 //
-// Tiling: a workgroup of WM x WN waves computes (WM*TI*16) tokens x
-// (WN*TJ*16) rows; each wave computes TI x TJ MFMA tiles of 16 x 16. Groups
-// are staged one at a time in two LDS buffers: the group's codes (converted
-// to fp16 once per workgroup) and scales. Global loads run two groups ahead
-// in registers; one barrier per group. LDS rows are 32 halves (four 16-byte
-// units) with the units of row t XOR-swizzled by (t >> 1) & 3, so the
-// 16-byte fragment reads of 16 consecutive rows fall on distinct banks. The
-// output tile leaves through LDS as 16-byte row units.
-#include "common.hpp"
+// What binds it is VALU issue: eight instructions (32 cycles) per 16 x 16 tile
+// and group against one MFMA of 16 cycles. So the two forms (cooperative and
+// split, prefill.hpp) keep everything else off the VALU: codes go from memory
+// through LDS into the MFMA unconverted, an operand is replaced by the next
+// group's as soon as its last use is issued, and a tile's MFMA is issued four
+// tiles before its VALU work. Measured on MI355X against the form this
+// replaces (codes converted to fp16 once per workgroup, one 8-wave workgroup
+// per 128- or 256-token tile, a barrier per group), us:
+//   tokens x [7168 x 5120]: 64: 114 -> 18, 200: 119 -> 38, 512: 129 -> 66;
+//   [5120 x 17408]: 64: 395 -> 54, 512: 422 -> 175;
+//   [34816 x 5120], 2048 tokens: 1794 -> 1135 (643 TOP/s; the VALU work alone
+//     would take about 700 us).
+#include "prefill.hpp"
 
 #include <algorithm>
-#include <utility>
 
 namespace vt {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float float4v __attribute__((ext_vector_type(4)));
+typedef int int4v __attribute__((ext_vector_type(4)));
+typedef std::uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte load at 4-byte alignment
 
-// Sixteen int8 codes -> sixteen fp16 values, exactly (u = c + 128 as the
-// mantissa of 1024 + u, then -1152).
-__device__ __forceinline__ void codes16_to_half(const uint4 w, uint4& lo, uint4& hi) {
-    typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-    const half2v bias = {static_cast<_Float16>(-1152.0f), static_cast<_Float16>(-1152.0f)};
-    std::uint32_t h[8];
-    const std::uint32_t words[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const std::uint32_t u = words[i] ^ 0x80808080u;
-        const half2v a = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, u, 0x05010400u)) + bias;
-        const half2v b = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, u, 0x05030402u)) + bias;
-        h[2 * i] = __builtin_bit_cast(std::uint32_t, a);
-        h[2 * i + 1] = __builtin_bit_cast(std::uint32_t, b);
-    }
-    lo = make_uint4(h[0], h[1], h[2], h[3]);
-    hi = make_uint4(h[4], h[5], h[6], h[7]);
-}
+constexpr int kMagicBits = 0x4B400000;         // 1.5 * 2^23
+constexpr float kMagic = 12582912.0f;
 
-__device__ __forceinline__ int swz(int row) { return (row >> 1) & 3; }
+// A wave's TI x TJ tiles of 16 tokens x 16 rows. The MFMA's rows are weight
+// rows and its columns tokens: lane (r, q) holds token r and rows 4q .. 4q + 3
+// of a tile, its activation scale is one register per token tile and its
+// weight scales four per row tile.
+template <int TI, int TJ>
+struct A8Tile {
+    static constexpr int kTiles = TI * TJ, kAhead = kTiles < 5 ? 2 : 4;
+    float4v y[TJ][TI];
+    long fa[TI], fb[TJ];
+    float as[TI];
+    float4 ws[TJ];
 
-template <int P, int WM, int WN, int TI, int TJ>
-struct FastGeom {
-    static constexpr int kThreads = WM * WN * 64;
-    static constexpr int kTM = WM * TI * 16;  // tokens per workgroup
-    static constexpr int kTN = WN * TJ * 16;  // rows per workgroup
-    static constexpr int kAUnits = P * kTM * 2;  // 16-byte code loads per group (activations)
-    static constexpr int kBUnits = kTN * 2;      // 16-byte code loads per group (weights)
-    static constexpr int kAPer = (kAUnits + kThreads - 1) / kThreads;
-    static constexpr int kBPer = (kBUnits + kThreads - 1) / kThreads;
-    static_assert(kAUnits % kThreads == 0 || kAUnits < kThreads, "whole loads per thread");
-    static_assert(kBUnits % kThreads == 0 || kBUnits < kThreads, "whole loads per thread");
-    static_assert(P * kTM <= kThreads && kTN <= kThreads, "one scale per thread");
-};
-
-template <int P, int WM, int WN, int TI, int TJ>
-struct FastStage {
-    using G = FastGeom<P, WM, WN, TI, TJ>;
-    uint4 a[G::kAPer];
-    uint4 b[G::kBPer];
-    float as;
-    unsigned short ws;
-};
-
-template <int P, int WM, int WN, int TI, int TJ>
-struct FastLds {
-    using G = FastGeom<P, WM, WN, TI, TJ>;
-    static constexpr int kA = P * G::kTM * 4;   // 16-byte units of one activation buffer
-    static constexpr int kB = G::kTN * 4;       // 16-byte units of one weight buffer
-    static constexpr int kStage = 2 * (kA + kB) * 16 + 2 * (P * G::kTM + G::kTN) * 4;
-    static constexpr int kPitch = G::kTN + 8;   // halves per token row of the output tile
-    static constexpr int kOut = G::kTM * kPitch * 2;
-    static constexpr int kBytes = kStage > kOut ? kStage : kOut;
-};
-
-template <int P, int WM, int WN, int TI, int TJ>
-__global__ __launch_bounds__(WM * WN * 64) void a8_gemm_fast(const std::int8_t* __restrict__ acodes,
-                                                            const float* __restrict__ ascales,
-                                                            const std::int8_t* __restrict__ wcodes,
-                                                            const __half* __restrict__ wscales,
-                                                            __half* __restrict__ out, int tokens, int n, int padded,
-                                                            int groups) {
-    using G = FastGeom<P, WM, WN, TI, TJ>;
-    using L = FastLds<P, WM, WN, TI, TJ>;
-    using Stage = FastStage<P, WM, WN, TI, TJ>;
-    constexpr int TM = G::kTM, TN = G::kTN, T = G::kThreads;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[L::kBytes];
-    auto* a_lds = reinterpret_cast<uint4(*)[L::kA]>(lds);
-    auto* b_lds = reinterpret_cast<uint4(*)[L::kB]>(lds + 2 * L::kA * 16);
-    auto* as_lds = reinterpret_cast<float(*)[P * TM]>(lds + 2 * (L::kA + L::kB) * 16);
-    auto* ws_lds = reinterpret_cast<float(*)[TN]>(lds + 2 * (L::kA + L::kB) * 16 + 2 * P * TM * 4);
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
-    const int q = lane >> 4, r = lane & 15;
-    const int t0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-    const std::int64_t count = static_cast<std::int64_t>(tokens) * groups;
-
-    // Staging sources. Activation load u of a thread: unit i = tid + u*T,
-    // pass i / (2*TM), token (i / 2) % TM, half i % 2 of the group's 32 bytes.
-    const std::int8_t* a_src[G::kAPer];
-#pragma unroll
-    for (int u = 0; u < G::kAPer; ++u) {
-        const int i = tid + u * T;
-        const int p = i / (2 * TM), tok = (i / 2) % TM;
-        a_src[u] = acodes + (min(p, P - 1) * count + static_cast<std::int64_t>(min(t0 + tok, tokens - 1)) * groups) * 32 +
-                   16 * (i & 1);
-    }
-    const std::int8_t* b_src[G::kBPer];
-#pragma unroll
-    for (int u = 0; u < G::kBPer; ++u) {
-        const int i = tid + u * T;
-        b_src[u] = wcodes + static_cast<std::int64_t>(min(n0 + min(i / 2, TN - 1), n - 1)) * padded + 16 * (i & 1);
-    }
-    // Scales are staged by the last threads of the workgroup (the weight codes,
-    // fewer than the activation codes, are staged by the first ones).
-    const int sid = T - 1 - tid;
-    const int s_pass = min(sid / TM, P - 1);
-    const float* as_src =
-        ascales + s_pass * count + static_cast<std::int64_t>(min(t0 + sid % TM, tokens - 1)) * groups;
-    const __half* ws_src = wscales + static_cast<std::int64_t>(min(n0 + sid % TN, n - 1)) * (padded / 32);
-
-    // Group g's operands into registers (g is clamped by the caller, so a load
-    // past the last group re-reads it and is never consumed).
-    auto load = [&](int g, Stage& s) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < G::kAPer; ++u)
-            if (G::kAUnits >= T || tid < G::kAUnits) s.a[u] = *reinterpret_cast<const uint4*>(a_src[u] + g * 32);
-#pragma unroll
-        for (int u = 0; u < G::kBPer; ++u)
-            if (G::kBUnits >= T || tid < G::kBUnits) s.b[u] = *reinterpret_cast<const uint4*>(b_src[u] + g * 32);
-        s.as = as_src[g];
-        s.ws = __half_as_ushort(ws_src[g]);
-    };
-    auto store = [&](const Stage& s, int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < G::kAPer; ++u) {
-            const int i = tid + u * T;
-            if (G::kAUnits < T && i >= G::kAUnits) break;
-            const int row = i / 2;  // pass-major row p*TM + token
-            const int tok = row % TM;
-            uint4 lo, hi;
-            codes16_to_half(s.a[u], lo, hi);
-            a_lds[buf][row * 4 + ((2 * (i & 1)) ^ swz(tok))] = lo;
-            a_lds[buf][row * 4 + ((2 * (i & 1) + 1) ^ swz(tok))] = hi;
-        }
-#pragma unroll
-        for (int u = 0; u < G::kBPer; ++u) {
-            const int i = tid + u * T;
-            if (G::kBUnits < T && i >= G::kBUnits) break;
-            const int row = i / 2;
-            uint4 lo, hi;
-            codes16_to_half(s.b[u], lo, hi);
-            b_lds[buf][row * 4 + ((2 * (i & 1)) ^ swz(row))] = lo;
-            b_lds[buf][row * 4 + ((2 * (i & 1) + 1) ^ swz(row))] = hi;
-        }
-        if (sid < P * TM) as_lds[buf][sid] = s.as;
-        if (sid < TN) ws_lds[buf][sid] = __half2float(__ushort_as_half(s.ws));
-    };
-
-    float4v y[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) y[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-
-    struct Frag {
-        half8 fa[P][TI];
-        half8 fb[TJ];
-        float4 asv[P][TI];
-        float wsv[TJ];
-    };
-    auto read = [&](int buf, Frag& f) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-            const int row = wn * TJ * 16 + j * 16 + r;
-            f.fb[j] = __builtin_bit_cast(half8, b_lds[buf][row * 4 + (q ^ swz(row))]);
-            f.wsv[j] = ws_lds[buf][row];
-        }
-#pragma unroll
-        for (int i = 0; i < TI; ++i) {
-            const int tok = wm * TI * 16 + i * 16 + r;
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                f.fa[p][i] = __builtin_bit_cast(half8, a_lds[buf][(p * TM + tok) * 4 + (q ^ swz(tok))]);
-                f.asv[p][i] = *reinterpret_cast<const float4*>(&as_lds[buf][p * TM + wm * TI * 16 + i * 16 + 4 * q]);
-            }
-        }
-    };
-    // One group: each tile's MFMA is followed by the scaling of an earlier
-    // tile, so one wave's matrix-core work runs under its own VALU epilogue
-    // (the schedule below pins that interleave: the epilogue may not be
-    // gathered after the group's barrier, where both waves of a SIMD would
-    // run their VALU work at once).
-    constexpr int kEpi = P == 1 ? 8 : 12;  // VALU instructions per tile
-    auto math = [&](const Frag& f) __attribute__((always_inline)) {
-        const float4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int j = 0; j < TJ; ++j) {
-                if constexpr (P == 1) {
-                    const float4v d = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.fa[0][i], f.fb[j], zero, 0, 0, 0);
-                    const float a4[4] = {f.asv[0][i].x, f.asv[0][i].y, f.asv[0][i].z, f.asv[0][i].w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[i][j][e] = fmaf(d[e], f.wsv[j] * a4[e], y[i][j][e]);
-                } else {
-                    const float4v d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.fa[0][i], f.fb[j], zero, 0, 0, 0);
-                    const float4v d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.fa[1][i], f.fb[j], zero, 0, 0, 0);
-                    const float a0[4] = {f.asv[0][i].x, f.asv[0][i].y, f.asv[0][i].z, f.asv[0][i].w};
-                    const float a1[4] = {f.asv[1][i].x, f.asv[1][i].y, f.asv[1][i].z, f.asv[1][i].w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float t = fmaf(d1[e], a1[e], d0[e] * a0[e]);
-                        y[i][j][e] = fmaf(t, f.wsv[j], y[i][j][e]);
-                    }
-                }
-            }
-#pragma unroll
-        for (int t = 0; t < TI * TJ; ++t) {
-            __builtin_amdgcn_sched_group_barrier(0x008, P, 0);     // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, kEpi, 0);  // VALU
-        }
-    };
-
-    // Pipeline over groups, two LDS buffers and two register stages: while
-    // group g is multiplied out of buffer g % 2, group g + 1 (loaded two
-    // groups earlier) is converted into the other buffer and group g + 3 is
-    // requested; one barrier per group. The body of a step has no branches
-    // on g, so the scheduler sees the fragment reads, the conversion and the
-    // interleaved MFMA / VALU work as one region.
-    Stage st0, st1;
-    load(0, st0);
-    load(min(1, groups - 1), st1);
-    store(st0, 0);
-    load(min(2, groups - 1), st0);
-    __syncthreads();
-    int g = 0;
-    for (; g + 1 < groups; g += 2) {
-        Frag f;
-        read(0, f);
-        store(st1, 1);
-        load(min(g + 3, groups - 1), st1);
-        math(f);
-        __syncthreads();
-        read(1, f);
-        store(st0, 0);
-        load(min(g + 4, groups - 1), st0);
-        math(f);
-        __syncthreads();
-    }
-    if (g < groups) {
-        Frag f;
-        read(0, f);
-        math(f);
-        __syncthreads();
-    }
-
-    // Output tile: fp16 through LDS (token rows of TN halves, padded by 8 so
-    // the four token quads of a wave's 2-byte writes fall on distinct banks),
-    // then 16-byte row units to HBM.
-    auto* o_lds = reinterpret_cast<__half*>(lds);
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
+    __device__ __forceinline__ void clear() {
 #pragma unroll
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                o_lds[(wm * TI * 16 + i * 16 + 4 * q + e) * L::kPitch + wn * TJ * 16 + j * 16 + r] =
-                    from_f32<__half>(y[i][j][e]);
-    __syncthreads();
-    const bool vec = (n % 8) == 0 && (reinterpret_cast<std::uintptr_t>(out) & 15) == 0;
-    constexpr int kUnits = TM * TN / 8;
+            for (int i = 0; i < TI; ++i) y[j][i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    // Reads all operands of a group.
+    template <class Source>
+    __device__ __forceinline__ void fill(const Source& src) {
 #pragma unroll
-    for (int u = tid; u < kUnits; u += T) {
-        const int tok = u / (TN / 8), c = (u % (TN / 8)) * 8;
-        const int t = t0 + tok, col = n0 + c;
-        if (t >= tokens || col >= n) continue;
-        const __half* src = o_lds + tok * L::kPitch + c;
-        __half* dst = out + static_cast<std::int64_t>(t) * n + col;
-        if (vec) {
-            *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
-        } else {
-            for (int e = 0; e < 8 && col + e < n; ++e) dst[e] = src[e];
+        for (int i = 0; i < TI; ++i) {
+            fa[i] = src.a(i);
+            as[i] = src.a_scale(i);
+        }
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            fb[j] = src.b(j);
+            ws[j] = src.b_scale(j);
         }
     }
+    // Multiplies the group in registers and replaces every operand by the next
+    // group's as soon as its last use is issued. Tiles run down the tokens of a
+    // row tile; a tile's MFMA is issued kAhead tiles before its eight VALU
+    // instructions. hook(t) runs before tile t.
+    template <class Source, class Hook>
+    __device__ __forceinline__ void group(const Source& next, Hook&& hook) {
+        const int4v magic = {kMagicBits, kMagicBits, kMagicBits, kMagicBits};
+        int4v d[kAhead];
+        float4 nm;
+#pragma unroll
+        for (int t = 0; t < kTiles + kAhead; ++t) {
+            hook(t);
+            if (t >= kAhead) {
+                const int f = t - kAhead, j = f / TI, i = f % TI;
+                if (i == 0) nm = make_float4(-kMagic * ws[j].x, -kMagic * ws[j].y, -kMagic * ws[j].z, -kMagic * ws[j].w);
+                const float s[4] = {ws[j].x, ws[j].y, ws[j].z, ws[j].w}, m[4] = {nm.x, nm.y, nm.z, nm.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    y[j][i][e] = fmaf(fmaf(__int_as_float(d[f % kAhead][e]), s[e], m[e]), as[i], y[j][i][e]);
+                if (j == TJ - 1) as[i] = next.a_scale(i);
+                if (i == TI - 1) ws[j] = next.b_scale(j);
+            }
+            if (t < kTiles) {
+                const int j = t / TI, i = t % TI;
+                d[t % kAhead] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fb[j], fa[i], magic, 0, 0, 0);
+                if (j == TJ - 1) fa[i] = next.a(i);
+                if (i == TI - 1) fb[j] = next.b(j);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // Partial sums of token tiles [I0, I0 + N) as fp32 rows of P floats.
+    template <int I0, int N, int P>
+    __device__ __forceinline__ void put(float* rows, int r, int q) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+                *reinterpret_cast<float4v*>(rows + (i * 16 + r) * P + j * 16 + 4 * q) = y[j][I0 + i];
+    }
+};
+
+// Where a wave's operands of one group lie in LDS (byte addresses of its lane).
+struct A8Source {
+    const unsigned char *pa, *pb, *psa, *psb;
+    int a_stride, b_stride;  // bytes between tiles of 16 rows
+    __device__ __forceinline__ long a(int i) const { return *reinterpret_cast<const long*>(pa + i * a_stride); }
+    __device__ __forceinline__ long b(int j) const { return *reinterpret_cast<const long*>(pb + j * b_stride); }
+    __device__ __forceinline__ float a_scale(int i) const { return *reinterpret_cast<const float*>(psa + i * 64); }
+    __device__ __forceinline__ float4 b_scale(int j) const { return *reinterpret_cast<const float4*>(psb + j * 64); }
+};
+
+template <int WT, int WN, int WK, int TI, int TJ>
+struct A8Geom {
+    static constexpr int kThreads = WT * WN * WK * 64;
+    static constexpr int kTM = WT * TI * 16, kTN = WN * TJ * 16;
+    static constexpr int kGroups = WK;      // groups per stage, one per K wave
+    static constexpr int kU = 2 * kGroups;  // 16-byte units of a staged row of codes
+    static constexpr int kAPer = (kTM * kU + kThreads - 1) / kThreads, kBPer = (kTN * kU + kThreads - 1) / kThreads;
+    static constexpr int kAsPer = (kTM * kGroups + kThreads - 1) / kThreads;
+    static constexpr int kWsPer = (kTN * kGroups + kThreads - 1) / kThreads;
+    // A buffer holds whole rounds of the threads' stores, so no store is guarded.
+    static constexpr int kB = kAPer * kThreads * 16, kAs = kB + kBPer * kThreads * 16, kWs = kAs + kAsPer * kThreads * 4;
+    static constexpr int kStage = kWs + kWsPer * kThreads * 4;
+    static constexpr int kPitch = kTN + 4;
+    static constexpr int out_bytes(int oi) { return WK * WT * oi * 16 * kPitch * 4; }
+    static constexpr int kOI = out_bytes(TI) <= 140 * 1024       ? TI
+                               : TI % 2 == 0 && out_bytes(TI / 2) <= 140 * 1024 ? TI / 2
+                               : TI % 4 == 0                                   ? TI / 4
+                                                                               : 1;
+    static constexpr int kLds = 2 * kStage > out_bytes(kOI) ? 2 * kStage : out_bytes(kOI);
+    static_assert(TI % kOI == 0 && kLds <= 160 * 1024, "prefill tile exceeds LDS");
+};
+
+// Cooperative form: stages of WK groups in two LDS buffers, one group per K
+// wave. While a stage is multiplied, the next one's operands are read, the one
+// after is written to LDS and the one after that is requested.
+template <int WT, int WN, int WK, int TI, int TJ, class Off>
+__global__ __launch_bounds__(WT * WN * WK * 64, 2) void a8_prefill(const std::int8_t* __restrict__ acodes,
+                                                                  const float* __restrict__ ascales,
+                                                                  const std::int8_t* __restrict__ wcodes,
+                                                                  const __half* __restrict__ wscales,
+                                                                  __half* __restrict__ out, int tokens, int n,
+                                                                  int padded, int groups, int passes, TileOrder order) {
+    using G = A8Geom<WT, WN, WK, TI, TJ>;
+    constexpr int TM = G::kTM, TN = G::kTN, T = G::kThreads, U = G::kU, KG = G::kGroups;
+    extern __shared__ uint4 a8p_lds[];
+    auto* lds = reinterpret_cast<unsigned char*>(a8p_lds);
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave % WK, wn = (wave / WK) % WN, wt = wave / (WK * WN);
+    const int q = lane >> 4, r = lane & 15;
+    const int tile = tile_of(order);
+    if (tile < 0) return;
+    const int t0 = tile % order.token_tiles * TM, n0 = tile / order.token_tiles * TN;
+
+    const std::int64_t count = static_cast<std::int64_t>(tokens) * groups;  // groups of one pass
+    const auto* a_base = reinterpret_cast<const char*>(acodes) + static_cast<std::int64_t>(t0) * groups * 32;
+    const auto* as_base = reinterpret_cast<const char*>(ascales + static_cast<std::int64_t>(t0) * groups);
+    const auto* b_base = reinterpret_cast<const char*>(wcodes + static_cast<std::int64_t>(n0) * padded);
+    const auto* ws_base = reinterpret_cast<const char*>(wscales + static_cast<std::int64_t>(n0) * (padded / 32));
+    Off a_off[G::kAPer], b_off[G::kBPer], as_off[G::kAsPer], ws_off[G::kWsPer];
+    std::uint32_t a_put[G::kAPer], b_put[G::kBPer], as_put[G::kAsPer], ws_put[G::kWsPer];
+#pragma unroll
+    for (int u = 0; u < G::kAPer; ++u) {
+        const int i = tid + u * T, row = i / U;
+        a_off[u] = static_cast<Off>(min(row, tokens - 1 - t0)) * (groups * 32) + 16 * (i % U);
+        a_put[u] = 16 * (row * U + ((i % U) ^ swizzle<U>(row)));
+    }
+#pragma unroll
+    for (int u = 0; u < G::kBPer; ++u) {
+        const int i = tid + u * T, row = i / U;
+        b_off[u] = static_cast<Off>(min(row, n - 1 - n0)) * padded + 16 * (i % U);
+        b_put[u] = G::kB + 16 * (row * U + ((i % U) ^ swizzle<U>(row)));
+    }
+#pragma unroll
+    for (int u = 0; u < G::kAsPer; ++u) {
+        const int i = tid + u * T;
+        as_off[u] = 4u * (static_cast<Off>(min(i / KG, tokens - 1 - t0)) * groups + i % KG);
+        as_put[u] = G::kAs + 4 * (i < TM * KG ? (i % KG) * TM + i / KG : i);
+    }
+#pragma unroll
+    for (int u = 0; u < G::kWsPer; ++u) {
+        const int i = tid + u * T;
+        ws_off[u] = 2u * (static_cast<Off>(min(i / KG, n - 1 - n0)) * (padded / 32) + i % KG);
+        ws_put[u] = G::kWs + 4 * (i < TN * KG ? (i % KG) * TN + i / KG : i);
+    }
+
+    // Stage order: the partial stage of each pass first (when the groups are
+    // not whole stages), so that only the prologue clamps, then the whole
+    // stages of pass 0 and of pass 1.
+    const int whole = groups / KG, edges = whole * KG < groups ? passes : 0;
+    const int stages = edges + passes * whole;
+    u32x4 st_a[G::kAPer], st_b[G::kBPer];
+    float st_as[G::kAsPer];
+    unsigned short st_ws[G::kWsPer];
+    auto load = [&](int stage) __attribute__((always_inline)) {
+        const int w = min(max(stage - edges, 0), max(passes * whole - 1, 0));
+        const int pass = w >= whole && w > 0 ? 1 : 0;
+        const std::int64_t base = w - pass * whole;
+        const char* ap = a_base + pass * count * 32 + base * (32 * KG);
+        const char* sp = as_base + pass * count * 4 + base * (4 * KG);
+        const char* bp = b_base + base * (32 * KG);
+        const char* wp = ws_base + base * (2 * KG);
+#pragma unroll
+        for (int u = 0; u < G::kAPer; ++u) st_a[u] = *reinterpret_cast<const u32x4*>(ap + lane_offset(a_off[u]));
+#pragma unroll
+        for (int u = 0; u < G::kBPer; ++u) st_b[u] = *reinterpret_cast<const u32x4*>(bp + lane_offset(b_off[u]));
+#pragma unroll
+        for (int u = 0; u < G::kAsPer; ++u) st_as[u] = *reinterpret_cast<const float*>(sp + lane_offset(as_off[u]));
+#pragma unroll
+        for (int u = 0; u < G::kWsPer; ++u)
+            st_ws[u] = *reinterpret_cast<const unsigned short*>(wp + lane_offset(ws_off[u]));
+    };
+    // The partial stage of a pass: groups past the last one carry scale 0 (their codes are clamped, finite).
+    auto load_edge = [&](int pass) __attribute__((always_inline)) {
+        const int g0 = whole * KG;
+#pragma unroll
+        for (int u = 0; u < G::kAPer; ++u) {
+            const int unit = (tid + u * T) % U;
+            st_a[u] = *reinterpret_cast<const u32x4*>(
+                a_base + pass * count * 32 + a_off[u] + 16 * static_cast<std::int64_t>(min(2 * g0, 2 * groups - 1 - unit)));
+        }
+#pragma unroll
+        for (int u = 0; u < G::kBPer; ++u) {
+            const int unit = (tid + u * T) % U;
+            st_b[u] = *reinterpret_cast<const u32x4*>(
+                b_base + b_off[u] + 16 * static_cast<std::int64_t>(min(2 * g0, 2 * groups - 1 - unit)));
+        }
+#pragma unroll
+        for (int u = 0; u < G::kAsPer; ++u) {
+            const int g = (tid + u * T) % KG;
+            const float v = *reinterpret_cast<const float*>(as_base + pass * count * 4 + as_off[u] +
+                                                            4 * static_cast<std::int64_t>(min(g0, groups - 1 - g)));
+            st_as[u] = g0 + g < groups ? v : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < G::kWsPer; ++u) {
+            const int g = (tid + u * T) % KG;
+            const unsigned short v = *reinterpret_cast<const unsigned short*>(
+                ws_base + ws_off[u] + 2 * static_cast<std::int64_t>(min(g0, groups - 1 - g)));
+            st_ws[u] = g0 + g < groups ? v : 0;
+        }
+    };
+    auto store = [&](int buf) __attribute__((always_inline)) {
+        unsigned char* base = lds + buf * G::kStage;
+#pragma unroll
+        for (int u = 0; u < G::kAPer; ++u) *reinterpret_cast<u32x4*>(base + a_put[u]) = st_a[u];
+#pragma unroll
+        for (int u = 0; u < G::kBPer; ++u) *reinterpret_cast<u32x4*>(base + b_put[u]) = st_b[u];
+#pragma unroll
+        for (int u = 0; u < G::kAsPer; ++u) *reinterpret_cast<float*>(base + as_put[u]) = st_as[u];
+#pragma unroll
+        for (int u = 0; u < G::kWsPer; ++u)
+            *reinterpret_cast<float*>(base + ws_put[u]) = __half2float(__ushort_as_half(st_ws[u]));
+    };
+    const std::uint32_t a_get = 16 * ((wt * TI * 16 + r) * U + ((2 * wk + (q >> 1)) ^ swizzle<U>(r))) + 8 * (q & 1);
+    const std::uint32_t b_get =
+        G::kB + 16 * ((wn * TJ * 16 + r) * U + ((2 * wk + (q >> 1)) ^ swizzle<U>(r))) + 8 * (q & 1);
+    const std::uint32_t as_get = G::kAs + 4 * (wk * TM + wt * TI * 16 + r);
+    const std::uint32_t ws_get = G::kWs + 4 * (wk * TN + wn * TJ * 16 + 4 * q);
+    auto source = [&](int buf) __attribute__((always_inline)) {
+        const unsigned char* base = lds + buf * G::kStage;
+        return A8Source{base + a_get, base + b_get, base + as_get, base + ws_get, 256 * U, 256 * U};
+    };
+
+    A8Tile<TI, TJ> m;
+    m.clear();
+    if (edges > 0) {
+        load_edge(0);
+        store(0);
+    } else {
+        load(0);
+        store(0);
+    }
+    if (edges > 1) {
+        load_edge(1);
+        store(1);
+    } else if (stages > 1) {
+        load(1);
+        store(1);
+    }
+    if (whole == 0) {  // no whole stage: the loop's requests (never consumed) stay on group 0 of their rows
+#pragma unroll
+        for (int u = 0; u < G::kAPer; ++u) a_off[u] -= 16 * ((tid + u * T) % U);
+#pragma unroll
+        for (int u = 0; u < G::kBPer; ++u) b_off[u] -= 16 * ((tid + u * T) % U);
+#pragma unroll
+        for (int u = 0; u < G::kAsPer; ++u) as_off[u] -= 4 * ((tid + u * T) % KG);
+#pragma unroll
+        for (int u = 0; u < G::kWsPer; ++u) ws_off[u] -= 2 * ((tid + u * T) % KG);
+    }
+    load(2);
+    __syncthreads();
+    m.fill(source(0));
+    __syncthreads();
+    constexpr int kStoreAt = TI * TJ / 4, kLoadAt = TI * TJ / 4 + 2;
+    for (int sg = 0; sg < stages; ++sg) {
+        m.group(source((sg + 1) & 1), [&](int t) __attribute__((always_inline)) {
+            if (t == kStoreAt) store(sg & 1);
+            if (t == kLoadAt) load(sg + 3);
+        });
+        __syncthreads();
+    }
+
+    auto* o_lds = reinterpret_cast<float*>(lds);
+    constexpr int OI = G::kOI, P = G::kPitch, kRows = WT * OI * 16;
+    each_slot<TI / OI>([&](auto c) __attribute__((always_inline)) {
+        __syncthreads();
+        m.template put<c * OI, OI, P>(o_lds + (wk * kRows + wt * OI * 16) * P + wn * TJ * 16, r, q);
+        __syncthreads();
+        store_partials<WK, kRows, TN, P, T>(o_lds, out, tokens, n, n0, [&](int row) {
+            return t0 + (row / (OI * 16)) * TI * 16 + c * OI * 16 + row % (OI * 16);
+        });
+    });
 }
 
-template <int P, int WM, int WN, int TI, int TJ>
-void launch_fast(const std::int8_t* acodes, const float* ascales, const std::int8_t* codes, const __half* scales,
-                 __half* out, int tokens, int n, int padded, int groups, hipStream_t stream) {
-    using G = FastGeom<P, WM, WN, TI, TJ>;
-    const dim3 grid((n + G::kTN - 1) / G::kTN, (tokens + G::kTM - 1) / G::kTM);
-    require(grid.y <= 65535, "token tiles exceed the launch grid");
-    a8_gemm_fast<P, WM, WN, TI, TJ><<<grid, G::kThreads, 0, stream>>>(acodes, ascales, codes, scales, out, tokens, n,
-                                                                     padded, groups);
+template <int WK, int TI, int TJ>
+struct A8SplitGeom {
+    static constexpr int kThreads = WK * 64;
+    static constexpr int kTM = TI * 16, kTN = TJ * 16;
+    static constexpr int kAsPer = (kTM + 63) / 64;
+    static constexpr int kB = kTM * 128, kAs = kB + kTN * 128, kWs = kAs + 4 * kAsPer * 64 * 4;
+    static constexpr int kWave = kWs + 4 * 64 * 4;
+    static constexpr int kPitch = kTN + 4;
+    static constexpr int kOut = WK * kTM * kPitch * 4;
+    static constexpr int kLds = WK * kWave > kOut ? WK * kWave : kOut;
+    static_assert(kTN <= 64 && kLds <= 160 * 1024, "split tile exceeds LDS");
+};
+
+// Split form: every wave computes the whole tile over its own 128-column
+// chunks through its own LDS region (a wave's LDS accesses stay in order), so
+// there is no barrier before the final sum.
+template <int WK, int TI, int TJ>
+__global__ __launch_bounds__(WK * 64, 2) void a8_prefill_split(const std::int8_t* __restrict__ acodes,
+                                                              const float* __restrict__ ascales,
+                                                              const std::int8_t* __restrict__ wcodes,
+                                                              const __half* __restrict__ wscales,
+                                                              __half* __restrict__ out, int tokens, int n, int padded,
+                                                              int groups, int passes, TileOrder order) {
+    using G = A8SplitGeom<WK, TI, TJ>;
+    constexpr int TM = G::kTM, TN = G::kTN, kA = 2 * TI, kB = 2 * TJ;
+    static_assert(WK >= 2, "the last chunk of each pass is a wave's first");
+    extern __shared__ uint4 a8p_lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = lane >> 4, r = lane & 15;
+    const int tile = tile_of(order);
+    if (tile < 0) return;
+    const int t0 = tile % order.token_tiles * TM, n0 = tile / order.token_tiles * TN;
+    auto* lds = reinterpret_cast<unsigned char*>(a8p_lds) + wave * G::kWave;
+
+    // Chunk order: the last chunk of each pass (it may be partial) first, then
+    // the others of pass 0 and of pass 1; wave w takes every WK-th from w.
+    const int chunks = padded / 128, inner = chunks - 1, total = passes * chunks;
+    A8Tile<TI, TJ> m;
+    m.clear();
+    if (wave < total) {
+        const std::int64_t count = static_cast<std::int64_t>(tokens) * groups;
+        const auto* a_base = reinterpret_cast<const char*>(acodes) + static_cast<std::int64_t>(t0) * groups * 32;
+        const auto* as_base = reinterpret_cast<const char*>(ascales + static_cast<std::int64_t>(t0) * groups);
+        const auto* b_base = reinterpret_cast<const char*>(wcodes + static_cast<std::int64_t>(n0) * padded);
+        const auto* ws_base = reinterpret_cast<const char*>(wscales + static_cast<std::int64_t>(n0) * (padded / 32));
+        // Code unit u of a lane: row lane / 8 + 8 u, unit lane % 8 of its 128 bytes.
+        std::uint32_t a_off[kA], b_off[kB], as_off[G::kAsPer], ws_off;
+#pragma unroll
+        for (int u = 0; u < kA; ++u)
+            a_off[u] = static_cast<std::uint32_t>(min(lane / 8 + 8 * u, tokens - 1 - t0)) * (groups * 32) + 16 * (lane % 8);
+#pragma unroll
+        for (int u = 0; u < kB; ++u)
+            b_off[u] = static_cast<std::uint32_t>(min(lane / 8 + 8 * u, n - 1 - n0)) * padded + 16 * (lane % 8);
+#pragma unroll
+        for (int u = 0; u < G::kAsPer; ++u)
+            as_off[u] = 4u * static_cast<std::uint32_t>(min(lane + 64 * u, tokens - 1 - t0)) * groups;
+        ws_off = 2u * static_cast<std::uint32_t>(min(lane, n - 1 - n0)) * (padded / 32);
+        u32x4 st_a[kA], st_b[kB];
+        float4u st_as[G::kAsPer];
+        uint2 st_ws;
+        // A chunk of four whole groups (inner chunks; past the end, chunk 0 of pass 0, never consumed).
+        auto load = [&](int v) __attribute__((always_inline)) {
+            const int w = v < total ? v - passes : 0;
+            const int pass = w >= inner && w > 0 ? 1 : 0;
+            const std::int64_t c = w - pass * inner;
+            const char* ap = a_base + pass * count * 32 + c * 128;
+            const char* sp = as_base + pass * count * 4 + c * 16;
+#pragma unroll
+            for (int u = 0; u < kA; ++u) st_a[u] = *reinterpret_cast<const u32x4*>(ap + lane_offset(a_off[u]));
+#pragma unroll
+            for (int u = 0; u < kB; ++u) st_b[u] = *reinterpret_cast<const u32x4*>(b_base + c * 128 + lane_offset(b_off[u]));
+#pragma unroll
+            for (int u = 0; u < G::kAsPer; ++u) st_as[u] = *reinterpret_cast<const float4u*>(sp + lane_offset(as_off[u]));
+            st_ws = *reinterpret_cast<const uint2*>(ws_base + c * 8 + lane_offset(ws_off));
+        };
+        // The last chunk of a pass: groups past the last one carry scale 0 (their codes are clamped, finite).
+        auto load_edge = [&](int pass) __attribute__((always_inline)) {
+            const int real = groups - 4 * inner;  // 1 .. 4
+            const int unit = min(8 * inner, 2 * groups - 1 - lane % 8);
+#pragma unroll
+            for (int u = 0; u < kA; ++u)
+                st_a[u] = *reinterpret_cast<const u32x4*>(a_base + pass * count * 32 + a_off[u] + 16 * static_cast<std::int64_t>(unit));
+#pragma unroll
+            for (int u = 0; u < kB; ++u)
+                st_b[u] = *reinterpret_cast<const u32x4*>(b_base + b_off[u] + 16 * static_cast<std::int64_t>(unit));
+#pragma unroll
+            for (int u = 0; u < G::kAsPer; ++u)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float v = *reinterpret_cast<const float*>(
+                        as_base + pass * count * 4 + as_off[u] + 4 * static_cast<std::int64_t>(min(4 * inner + g, groups - 1)));
+                    st_as[u][g] = g < real ? v : 0.0f;
+                }
+            const uint2 v = *reinterpret_cast<const uint2*>(ws_base + ws_off + 8 * static_cast<std::int64_t>(inner));
+            st_ws.x = real >= 2 ? v.x : v.x & 0xffffu;
+            st_ws.y = real >= 4 ? v.y : real == 3 ? v.y & 0xffffu : 0u;
+        };
+        // Rows 8 apart alternate between two swizzles.
+        std::uint32_t put[2];
+#pragma unroll
+        for (int odd = 0; odd < 2; ++odd) put[odd] = 16 * ((lane / 8) * 8 + ((lane % 8) ^ swizzle<8>(lane / 8 + 8 * odd)));
+        auto store = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int u = 0; u < kA; ++u) *reinterpret_cast<u32x4*>(lds + put[u & 1] + u * 1024) = st_a[u];
+#pragma unroll
+            for (int u = 0; u < kB; ++u) *reinterpret_cast<u32x4*>(lds + G::kB + put[u & 1] + u * 1024) = st_b[u];
+#pragma unroll
+            for (int u = 0; u < G::kAsPer; ++u)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<float*>(lds + G::kAs + 4 * ((g * G::kAsPer + u) * 64 + lane)) = st_as[u][g];
+            const float f[4] = {half_lo(st_ws.x), half_hi(st_ws.x), half_lo(st_ws.y), half_hi(st_ws.y)};
+#pragma unroll
+            for (int g = 0; g < 4; ++g) *reinterpret_cast<float*>(lds + G::kWs + 4 * (64 * g + lane)) = f[g];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        };
+        std::uint32_t get[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) get[g] = 16 * (r * 8 + ((2 * g + (q >> 1)) ^ swizzle<8>(r))) + 8 * (q & 1);
+        auto source = [&](int g) __attribute__((always_inline)) {
+            return A8Source{lds + get[g], lds + G::kB + get[g], lds + G::kAs + 4 * (g * G::kAsPer * 64 + r),
+                            lds + G::kWs + 4 * (64 * g + 4 * q), 2048, 2048};
+        };
+        if (wave < passes) {
+            load_edge(wave);
+            store();
+        } else {
+            load(wave);
+            store();
+        }
+        load(wave + WK);
+        m.fill(source(0));
+        for (int v = wave; v < total; v += WK) {
+            each_slot<4>([&](auto g) __attribute__((always_inline)) {
+                m.group(source((g + 1) % 4), [&](int t) __attribute__((always_inline)) {
+                    if (g == 3 && t == 0) {  // every read of this chunk is issued
+                        store();
+                        load(v + 2 * WK);
+                    }
+                });
+            });
+        }
+    }
+
+    auto* o_lds = reinterpret_cast<float*>(a8p_lds);
+    constexpr int P = G::kPitch;
+    __syncthreads();
+    m.template put<0, TI, P>(o_lds + wave * TM * P, r, q);
+    __syncthreads();
+    store_partials<WK, TM, TN, P, G::kThreads>(o_lds, out, tokens, n, n0, [&](int row) { return t0 + row; });
+}
+
+struct A8Operands {
+    const std::int8_t* acodes;
+    const float* ascales;
+    const std::int8_t* codes;
+    const __half* scales;
+    __half* out;
+    int tokens, n, padded, groups, passes;
+};
+
+template <int WT, int WN, int WK, int TI, int TJ, class Off = std::uint32_t>
+void launch_coop(const A8Operands& o, hipStream_t stream) {
+    using G = A8Geom<WT, WN, WK, TI, TJ>;
+    const auto kernel = a8_prefill<WT, WN, WK, TI, TJ, Off>;
+    const TileOrder order = tile_order(o.tokens, G::kTM, o.n, G::kTN);
+    static const bool raised = (raise_lds(kernel, G::kLds), true);
+    static_cast<void>(raised);
+    kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(o.acodes, o.ascales, o.codes, o.scales, o.out, o.tokens,
+                                                               o.n, o.padded, o.groups, o.passes, order);
+}
+
+template <int WK, int TI, int TJ>
+void launch_split(const A8Operands& o, hipStream_t stream) {
+    using G = A8SplitGeom<WK, TI, TJ>;
+    const auto kernel = a8_prefill_split<WK, TI, TJ>;
+    const TileOrder order = tile_order(o.tokens, G::kTM, o.n, G::kTN);
+    static const bool raised = (raise_lds(kernel, G::kLds), true);
+    static_cast<void>(raised);
+    kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(o.acodes, o.ascales, o.codes, o.scales, o.out, o.tokens,
+                                                               o.n, o.padded, o.groups, o.passes, order);
 }
 
 }  // namespace
 
 void a8_fast_launch(const void* workspace, const std::int8_t* codes, const __half* scales, void* out, int tokens, int n,
                     int k, int padded, int passes, hipStream_t stream) {
-    const int groups = (k + 31) / 32;
-    const std::int64_t count = static_cast<std::int64_t>(tokens) * groups;
-    const auto* acodes = static_cast<const std::int8_t*>(workspace);
-    const auto* ascales = reinterpret_cast<const float*>(acodes + count * 32 * passes);
-    auto* y = static_cast<__half*>(out);
-    if (passes == 2) {
-        launch_fast<2, 4, 2, 2, 4>(acodes, ascales, codes, scales, y, tokens, n, padded, groups, stream);
+    A8Operands o{};
+    o.tokens = tokens; o.n = n; o.padded = padded; o.groups = (k + 31) / 32; o.passes = passes;
+    const std::int64_t count = static_cast<std::int64_t>(tokens) * o.groups;
+    o.acodes = static_cast<const std::int8_t*>(workspace);
+    o.ascales = reinterpret_cast<const float*>(o.acodes + count * 32 * passes);
+    o.codes = codes; o.scales = scales; o.out = static_cast<__half*>(out);
+    if (k > kNarrowK) {  // rows too long for 32-bit lane offsets
+        launch_coop<1, 2, 4, 4, 4, std::uint64_t>(o, stream);
         return;
     }
-    // One pass: 256 x 128, 128 x 160 or 128 x 224 tiles (waves of 64 x 64,
-    // 32 x 80, 32 x 112), whichever leaves the fewest tile rounds on the CUs
-    // at the measured rates (config 3 at M = 2048 on MI355X: QKV / o_proj /
-    // gate+up / down 457 / 435 / 1781 / 1162 -> 408 / 389 / 1781 / 1038 us;
-    // same bits in every tiling, the groups being summed in natural order).
-    constexpr GemmTiling kTilings[3] = {{256, 128, 1.0}, {128, 160, 0.76}, {128, 224, 0.89}};
-    const int best = pick_tiling(tokens, n, kTilings);
-    if (best == 0) launch_fast<1, 4, 2, 4, 4>(acodes, ascales, codes, scales, y, tokens, n, padded, groups, stream);
-    else if (best == 1) launch_fast<1, 4, 2, 2, 5>(acodes, ascales, codes, scales, y, tokens, n, padded, groups, stream);
-    else launch_fast<1, 4, 2, 2, 7>(acodes, ascales, codes, scales, y, tokens, n, padded, groups, stream);
+    // The tiling with the least predicted time (the passes run one after the
+    // other over K); the constants are a fit to 105 shapes (33-2048 tokens,
+    // 1024-34816 rows, 1024-25600 columns, one and two passes; each candidate
+    // timed on each shape on MI355X): the choice is within 9% of the fastest
+    // candidate on every one of them and 0.5% on average.
+    constexpr PrefillTiling kTilings[9] = {
+        {256, 128, 1, 0.0, 6.12, 21.59, 21.59}, {128, 128, 1, 0.0, 7.25, 10.83, 10.83}, {64, 128, 1, 0.9, 4.39, 7.05, 7.05},
+        {64, 64, 1, 0.8, 5.99, 3.22, 3.22},     {64, 64, 2, 3.1, 4.02, 3.66, 6.34},     {48, 64, 2, 3.5, 2.78, 3.14, 5.40},
+        {48, 64, 1, 1.2, 4.84, 2.70, 2.70},     {32, 64, 1, 1.5, 3.74, 2.23, 2.23},     {32, 32, 1, 2.9, 0.72, 1.71, 1.71}};
+    int best = fastest_tiling(kTilings, tokens, n, static_cast<double>(k) * passes);
+    // The split form reads a chunk's four weight scales as one 8-byte word and
+    // needs one whole chunk.
+    if (best >= 3 && (k < 128 || !aligned(scales, 8))) best = 2;
+    switch (best) {
+        case 0: launch_coop<2, 2, 2, 8, 4>(o, stream); break;
+        case 1: launch_coop<1, 2, 4, 8, 4>(o, stream); break;
+        case 2: launch_coop<1, 2, 4, 4, 4>(o, stream); break;
+        case 3: launch_split<8, 4, 4>(o, stream); break;
+        case 4: launch_split<4, 4, 4>(o, stream); break;
+        case 5: launch_split<4, 3, 4>(o, stream); break;
+        case 6: launch_split<8, 3, 4>(o, stream); break;
+        case 7: launch_split<8, 2, 4>(o, stream); break;
+        default: launch_split<8, 2, 2>(o, stream); break;
+    }
 }
 
 }  // namespace vt

@@ -56,7 +56,7 @@ struct PrefillTiling {
     double base, round, solo, full;
 };
 
-inline double tiling_time(const PrefillTiling& t, int tokens, int n, int k) {
+inline double tiling_time(const PrefillTiling& t, int tokens, int n, double k) {
     const std::int64_t tiles = static_cast<std::int64_t>((tokens + t.tm - 1) / t.tm) * ((n + t.tn - 1) / t.tn);
     const std::int64_t slots = static_cast<std::int64_t>(device_cus()) * t.per_cu;
     const std::int64_t whole = tiles / slots, rest = tiles % slots;
@@ -66,7 +66,7 @@ inline double tiling_time(const PrefillTiling& t, int tokens, int n, int k) {
 }
 
 template <int N>
-inline int fastest_tiling(const PrefillTiling (&tilings)[N], int tokens, int n, int k) {
+inline int fastest_tiling(const PrefillTiling (&tilings)[N], int tokens, int n, double k) {
     int best = 0;
     for (int i = 1; i < N; ++i)
         if (tiling_time(tilings[i], tokens, n, k) < tiling_time(tilings[best], tokens, n, k)) best = i;
