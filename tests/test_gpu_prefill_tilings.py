@@ -12,6 +12,7 @@ import torch
 
 from helpers import guarded_out, random_q8
 from venturi_amd import Q8RowSplitWeight, prepare_q8_dp4a
+from venturi_amd.weights import Q4RowSplitWeight
 
 pytestmark = pytest.mark.gpu
 
@@ -129,3 +130,33 @@ def test_a8_scales_aligned_to_two_bytes(backend, device, tokens, n, k, passes):
                                          out.data_ptr(), tokens, n, k, codes.shape[1], passes, stream))
     assert guard[0] == 47 and guard[-1] == 47
     assert_bound(out, represented(workspace, tokens, k, passes), values(codes, scales, k))
+
+
+# 128 x 128, 64 x 128, 64 x 64 (eight and four K waves), 48 x 64 (four and eight), 32 x 64 and 32 x 32 tiles, the wide
+# tiles of the large grids, K below one chunk, and the first token count of the route.
+Q4_SHAPES = [(300, 10001, 264), (129, 7001, 520), (97, 7001, 1032), (113, 14003, 2056), (65, 14003, 520),
+             (97, 4100, 1032), (47, 4100, 1032), (65, 257, 136), (32, 33, 3976), (33, 70, 40), (40, 300, 120),
+             (1025, 14003, 264), (513, 14003, 136), (1025, 10001, 136), (700, 7001, 2056), (65, 10001, 136), (200, 2049, 1000), (513, 1000, 2056)]
+
+
+@pytest.mark.parametrize("tokens,n,k", Q4_SHAPES)
+def test_q4_tilings(backend, device, tokens, n, k):
+    print(f"case q4 prefill tiling tokens={tokens} n={n} k={k}", flush=True)
+    gen = torch.Generator().manual_seed(3 + n + tokens)
+    padded = (k + 127) // 128 * 128
+    codes = torch.randint(0, 256, (n, padded // 2), dtype=torch.uint8, generator=gen).to(device)
+    scales = (torch.rand(n, padded // 64, generator=gen) * 0.05).half().to(device)
+    low, high = codes & 15, codes >> 4
+    signed = torch.stack((low, high), -1).view(n, padded).to(torch.int8)
+    signed = torch.where(signed > 7, signed - 16, signed)
+    x = activations(tokens, k, device, tokens + 2)
+    plan = backend.upload_linear(Q4RowSplitWeight(codes, scales, k), dtype=torch.float16, device=device).prepare(
+        tokens=tokens, route="mfma")
+    guard, out = guarded_out(tokens, n, torch.float16, device)
+    plan.run(x, out=out)
+    assert guard[0] == 47 and guard[-1] == 47
+    weights = values(signed, scales, k).half().double()  # the contract's fp16(q * scale)
+    assert_bound(out, x.double(), weights)
+    aligned = torch.empty(tokens, n, dtype=torch.float16, device=device)
+    plan.run(x, out=aligned)  # 16-byte stores where n allows them: the same bits
+    assert torch.equal(aligned, out)

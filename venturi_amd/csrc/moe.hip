@@ -26,6 +26,11 @@
 #include <type_traits>
 
 namespace vt {
+
+// w4a16.hip: false where the wide tiles of row_prefill are the faster ones.
+bool q4_prefill_launch(const __half* x, const std::uint8_t* codes, const __half* scales, __half* out, int tokens, int n,
+                       int k, int padded, hipStream_t stream);
+
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -1387,8 +1392,9 @@ void row_decode_dispatch(const __half* x, const std::uint8_t* codes, const std::
 // GEMM reads each weight once per 16 or 32 tokens).
 constexpr int kRowPrefillMinTokens = 32;
 
-// Prefill tiles. Below 256 tokens: 128 tokens x 128 rows (8 waves of 32 x 64).
-// From 256 tokens: 256 tokens x 32*TJ rows, 8 waves of 64 x 16*TJ (one
+// Prefill tiles. Q4 runs the kernels of w4a16.hip except where these are the
+// faster ones. Q5 and Q6, below 256 tokens: 128 tokens x 128 rows (8 waves of
+// 32 x 64). Otherwise: 256 tokens x 32*TJ rows, 8 waves of 64 x 16*TJ (one
 // workgroup per CU by LDS), TJ in {5, 6, 7} picked for the fewest tile rounds
 // over the CUs weighted by the wider tiles' higher rate (fewer LDS bytes per
 // MFMA): at M = 2048 on MI355X, 5120 rows take TJ = 5 (256 tiles, one round),
@@ -1398,7 +1404,9 @@ constexpr int kRowPrefillMinTokens = 32;
 template <int HB>
 void row_prefill_dispatch(const __half* x, const std::uint8_t* codes, const std::uint8_t* high, const __half* scales,
                           __half* out, int tokens, int n, int k, int padded, hipStream_t stream) {
-    if (tokens < 256) {
+    if constexpr (HB == 0) {
+        if (q4_prefill_launch(x, codes, scales, out, tokens, n, k, padded, stream)) return;
+    } else if (tokens < 256) {
         launch_row_prefill<HB, 4, 2, 2, 4, 2>(x, codes, high, scales, out, tokens, n, k, padded, stream);
         return;
     }
