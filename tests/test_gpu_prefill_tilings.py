@@ -160,3 +160,31 @@ def test_q4_tilings(backend, device, tokens, n, k):
     aligned = torch.empty(tokens, n, dtype=torch.float16, device=device)
     plan.run(x, out=aligned)  # 16-byte stores where n allows them: the same bits
     assert torch.equal(aligned, out)
+
+
+# The split form over the tiled planes: one, two and three row blocks per workgroup, four K waves past 768 blocks;
+# K below one chunk, partial chunks, odd group counts; up to 16 tokens where the activations exceed the decode LDS.
+A8_TILED_SHAPES = [(17, 4096, 1000, 1), (32, 70, 31, 2), (31, 33, 97, 1), (20, 500, 4000, 2), (24, 5120, 519, 1),
+                   (32, 7167, 2056, 2), (17, 11702, 391, 2), (32, 12300, 136, 1), (25, 20001, 264, 2),
+                   (16, 300, 16392, 2), (12, 5000, 17408, 2), (16, 13000, 5120, 2), (9, 17000, 12296, 1)]
+
+
+@pytest.mark.parametrize("tokens,n,k,passes", A8_TILED_SHAPES)
+def test_a8_tiled_split(backend, device, tokens, n, k, passes):
+    print(f"case a8 tiled split tokens={tokens} n={n} k={k} passes={passes}", flush=True)
+    codes, scales = (t.to(device) for t in random_q8(n, k, 91 + n + tokens))
+    x = activations(tokens, k, device, tokens + 4)
+    x[1, min(k - 1, 40)] = float("nan")  # that group: zero codes, NaN scale; the token's outputs are NaN
+    plan = prepare_q8_dp4a(backend.upload_linear(Q8RowSplitWeight(codes, scales, k), dtype=torch.float16, device=device),
+                           tokens=tokens, residual_compensation=passes == 2)
+    assert plan.kernel == "tiled"
+    workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=device)
+    guard, out = guarded_out(tokens, n, torch.float16, device)
+    plan.run(x, out=out, workspace=workspace)
+    assert guard[0] == 47 and guard[-1] == 47
+    keep = torch.arange(tokens, device=device) != 1
+    assert bool(torch.isnan(out[1]).all())
+    assert_bound(out[keep], represented(workspace, tokens, k, passes)[keep], values(codes, scales, k))
+    again = torch.empty(tokens, n, dtype=torch.float16, device=device)
+    plan.project(out=again, workspace=workspace)
+    assert torch.equal(again[keep], out[keep])

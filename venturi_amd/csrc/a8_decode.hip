@@ -22,10 +22,12 @@
 // [2 groups]), and its activation scales are the two of its own token. B
 // fragments are 8 bytes of the token's group codes at [group][8q ..].
 //
-// Three forms share that arithmetic:
+// Three forms share that arithmetic (17-32 tokens, and fewer whose activations
+// exceed the LDS of these forms, run the split form of the prefill GEMM over
+// the tiled planes, a8_fast.hip):
 // * a8_tiled_decode reads a filled A8 workspace ([pass][token][group][32]
 //   codes, then fp32 scales [pass][token][group]) from global memory, each
-//   lane its own B fragments (up to 32 tokens);
+//   lane its own B fragments (up to 16 tokens);
 // * a8_tiled_lds<STAGE = true> copies a filled workspace into LDS once per
 //   workgroup (up to 16 tokens where the copy fits one round of loads and the
 //   LDS keeps the shape's workgroups resident), and its waves read their B
@@ -52,6 +54,10 @@
 #include <type_traits>
 
 namespace vt {
+
+void a8_tiled_split_launch(const void* workspace, const void* codes, const void* scales, void* out, int tokens, int n,
+                           int k, int padded, int passes, hipStream_t stream);
+
 namespace {
 
 typedef int int4v __attribute__((ext_vector_type(4)));
@@ -88,16 +94,16 @@ __device__ __forceinline__ void run_pipeline(int batches, Batch (&buf)[NBUF], Fe
         if (i + NBUF + j < batches) consume(buf[j], std::true_type{});
 }
 
-template <int RB, int NB, int P>
+template <int RB, int P>
 struct A8Batch {
     uint4 w[RB];              // 16 weight code bytes per block (groups 2c and 2c + 1)
     uint4 ws[RB];             // four rows' scale pairs (fp16)
-    uint2 ac[P][NB][2];       // 8 activation code bytes of groups 2c and 2c + 1
-    float as[P][NB][2];       // the token's activation scales of the two groups
+    uint2 ac[P][2];           // 8 activation code bytes of groups 2c and 2c + 1
+    float as[P][2];           // the token's activation scales of the two groups
     bool pair;                // group 2c + 1 exists (false only in the last chunk of an odd group count)
 };
 
-template <int W, int RB, int NB, int P, int NBUF>
+template <int W, int RB, int P, int NBUF>
 __global__ __launch_bounds__(W * 64) void a8_tiled_decode(const std::int8_t* __restrict__ acodes,
                                                           const float* __restrict__ ascales,
                                                           const uint4* __restrict__ codes,
@@ -105,7 +111,7 @@ __global__ __launch_bounds__(W * 64) void a8_tiled_decode(const std::int8_t* __r
                                                           int tokens, int n, int groups, int chunks, int blocks) {
     // chunks: the plane's chunk stride (padded / 64); the wave loop covers only
     // the ceil(groups / 2) chunks that hold a group of the workspace.
-    __shared__ float4v partial[W][RB * NB][64];
+    __shared__ float4v partial[W][RB][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, r = lane & 15;
@@ -118,16 +124,14 @@ __global__ __launch_bounds__(W * 64) void a8_tiled_decode(const std::int8_t* __r
 
     // Activation sources of this lane's token (absent tokens read the last
     // token's codes and feed only outputs that are never stored).
-    const std::int8_t* arow[P][NB];
-    const float* srow[P][NB];
+    const std::int8_t* arow[P];
+    const float* srow[P];
 #pragma unroll
-    for (int p = 0; p < P; ++p)
-#pragma unroll
-        for (int tb = 0; tb < NB; ++tb) {
-            const std::int64_t t = min(16 * tb + r, tokens - 1);
-            arow[p][tb] = acodes + (p * count + t * groups) * 32 + 8 * q;
-            srow[p][tb] = ascales + p * count + t * groups;
-        }
+    for (int p = 0; p < P; ++p) {
+        const std::int64_t t = min(r, tokens - 1);
+        arow[p] = acodes + (p * count + t * groups) * 32 + 8 * q;
+        srow[p] = ascales + p * count + t * groups;
+    }
     const uint4* wsrc[RB];
     const uint4* ssrc[RB];
 #pragma unroll
@@ -142,7 +146,7 @@ __global__ __launch_bounds__(W * 64) void a8_tiled_decode(const std::int8_t* __r
     // not the workspace's: its loads re-read the last group and its term is
     // skipped (the weight codes and scales of padded groups are not read into
     // any output, as in the reference, which stops at the last group).
-    auto fetch = [&](int i, A8Batch<RB, NB, P>& t) {
+    auto fetch = [&](int i, A8Batch<RB, P>& t) {
         const int ch = min(c0 + i, c1 - 1);
         t.pair = 2 * ch + 1 < groups;
 #pragma unroll
@@ -152,26 +156,22 @@ __global__ __launch_bounds__(W * 64) void a8_tiled_decode(const std::int8_t* __r
         }
         const int ga = min(2 * ch, groups - 1), gb = min(2 * ch + 1, groups - 1);
 #pragma unroll
-        for (int p = 0; p < P; ++p)
-#pragma unroll
-            for (int tb = 0; tb < NB; ++tb) {
-                t.ac[p][tb][0] = *reinterpret_cast<const uint2*>(arow[p][tb] + ga * 32);
-                t.ac[p][tb][1] = *reinterpret_cast<const uint2*>(arow[p][tb] + gb * 32);
-                t.as[p][tb][0] = srow[p][tb][ga];
-                t.as[p][tb][1] = srow[p][tb][gb];
-            }
+        for (int p = 0; p < P; ++p) {
+            t.ac[p][0] = *reinterpret_cast<const uint2*>(arow[p] + ga * 32);
+            t.ac[p][1] = *reinterpret_cast<const uint2*>(arow[p] + gb * 32);
+            t.as[p][0] = srow[p][ga];
+            t.as[p][1] = srow[p][gb];
+        }
     };
 
-    float4v y[RB][NB];
+    float4v y[RB];
 #pragma unroll
-    for (int b = 0; b < RB; ++b)
-#pragma unroll
-        for (int tb = 0; tb < NB; ++tb) y[b][tb] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int b = 0; b < RB; ++b) y[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
     const int4v zero = {0, 0, 0, 0};
 
     // Only a wave's last chunk can lack its second group, and it is one of the
     // loop's tail multiplies: the loop body takes the group unconditionally.
-    auto consume = [&](const A8Batch<RB, NB, P>& t, auto last) {
+    auto consume = [&](const A8Batch<RB, P>& t, auto last) {
         const bool second = !decltype(last)::value || t.pair;
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
@@ -179,60 +179,51 @@ __global__ __launch_bounds__(W * 64) void a8_tiled_decode(const std::int8_t* __r
             const long wb = static_cast<long>(static_cast<unsigned long>(t.w[b].z) | (static_cast<unsigned long>(t.w[b].w) << 32));
             // Rows 4q + e: scale pairs (group a, group b) in the 32-bit words of t.ws[b].
             const std::uint32_t pair[4] = {t.ws[b].x, t.ws[b].y, t.ws[b].z, t.ws[b].w};
+            int4v da[P], db[P];
 #pragma unroll
-            for (int tb = 0; tb < NB; ++tb) {
-                int4v da[P], db[P];
+            for (int p = 0; p < P; ++p) {
+                const long xa =
+                    static_cast<long>(static_cast<unsigned long>(t.ac[p][0].x) | (static_cast<unsigned long>(t.ac[p][0].y) << 32));
+                const long xb =
+                    static_cast<long>(static_cast<unsigned long>(t.ac[p][1].x) | (static_cast<unsigned long>(t.ac[p][1].y) << 32));
+                da[p] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wa, xa, zero, 0, 0, 0);
+                db[p] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, xb, zero, 0, 0, 0);
+            }
 #pragma unroll
-                for (int p = 0; p < P; ++p) {
-                    const long xa = static_cast<long>(static_cast<unsigned long>(t.ac[p][tb][0].x) |
-                                                      (static_cast<unsigned long>(t.ac[p][tb][0].y) << 32));
-                    const long xb = static_cast<long>(static_cast<unsigned long>(t.ac[p][tb][1].x) |
-                                                      (static_cast<unsigned long>(t.ac[p][tb][1].y) << 32));
-                    da[p] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wa, xa, zero, 0, 0, 0);
-                    db[p] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, xb, zero, 0, 0, 0);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float wsa = half_lo(pair[e]), wsb = half_hi(pair[e]);
-                    if constexpr (P == 1) {
-                        y[b][tb][e] = fmaf(static_cast<float>(da[0][e]), wsa * t.as[0][tb][0], y[b][tb][e]);
-                        if (second)
-                            y[b][tb][e] = fmaf(static_cast<float>(db[0][e]), wsb * t.as[0][tb][1], y[b][tb][e]);
-                    } else {
-                        const float ta = fmaf(static_cast<float>(da[1][e]), t.as[1][tb][0],
-                                              static_cast<float>(da[0][e]) * t.as[0][tb][0]);
-                        const float tbv = fmaf(static_cast<float>(db[1][e]), t.as[1][tb][1],
-                                               static_cast<float>(db[0][e]) * t.as[0][tb][1]);
-                        y[b][tb][e] = fmaf(ta, wsa, y[b][tb][e]);
-                        if (second) y[b][tb][e] = fmaf(tbv, wsb, y[b][tb][e]);
-                    }
+            for (int e = 0; e < 4; ++e) {
+                const float wsa = half_lo(pair[e]), wsb = half_hi(pair[e]);
+                if constexpr (P == 1) {
+                    y[b][e] = fmaf(static_cast<float>(da[0][e]), wsa * t.as[0][0], y[b][e]);
+                    if (second) y[b][e] = fmaf(static_cast<float>(db[0][e]), wsb * t.as[0][1], y[b][e]);
+                } else {
+                    const float ta = fmaf(static_cast<float>(da[1][e]), t.as[1][0], static_cast<float>(da[0][e]) * t.as[0][0]);
+                    const float tbv = fmaf(static_cast<float>(db[1][e]), t.as[1][1], static_cast<float>(db[0][e]) * t.as[0][1]);
+                    y[b][e] = fmaf(ta, wsa, y[b][e]);
+                    if (second) y[b][e] = fmaf(tbv, wsb, y[b][e]);
                 }
             }
         }
     };
 
     if (batches > 0) {
-        A8Batch<RB, NB, P> buf[NBUF];
+        A8Batch<RB, P> buf[NBUF];
 #pragma unroll
         for (int j = 0; j < NBUF; ++j) fetch(j, buf[j]);
         run_pipeline<NBUF>(batches, buf, fetch, consume);
     }
 #pragma unroll
-    for (int b = 0; b < RB; ++b)
-#pragma unroll
-        for (int tb = 0; tb < NB; ++tb) partial[wave][b * NB + tb][lane] = y[b][tb];
+    for (int b = 0; b < RB; ++b) partial[wave][b][lane] = y[b];
     __syncthreads();
-    for (int p = wave; p < RB * NB; p += W) {
-        const int b = p / NB, tb = p % NB;
-        float4v sum = partial[0][p][lane];
+    for (int b = wave; b < RB; b += W) {
+        float4v sum = partial[0][b][lane];
         for (int w = 1; w < W; ++w) {
-            const float4v v = partial[w][p][lane];
+            const float4v v = partial[w][b][lane];
 #pragma unroll
             for (int e = 0; e < 4; ++e) sum[e] += v[e];
         }
-        const int blk = block0 + b, t = 16 * tb + r;
-        if (blk >= blocks || t >= tokens) continue;
-        __half* o = out + static_cast<std::int64_t>(t) * n + 16 * blk + 4 * q;
+        const int blk = block0 + b;
+        if (blk >= blocks || r >= tokens) continue;
+        __half* o = out + static_cast<std::int64_t>(r) * n + 16 * blk + 4 * q;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (16 * blk + 4 * q + e < n) o[e] = from_f32<__half>(sum[e]);
@@ -539,17 +530,15 @@ __global__ __launch_bounds__(W * 64) void a8_tiled_lds(const __half* x, const st
 }
 
 // Workgroup shape of both kernels (unsplit K): W waves over RB row blocks,
-// NBUF batches in flight per wave. Two token blocks take 8 waves over two row
-// blocks (the other shapes spill); one token block takes 16 waves over one
-// row block up to 256 blocks, over two up to 511 (grids of at most 256
-// workgroups, one per CU), else 8 waves over three.
+// NBUF batches in flight per wave: 16 waves over one row block up to 256
+// blocks, over two up to 511 (grids of at most 256 workgroups, one per CU),
+// else 8 waves over three.
 struct A8Shape {
     int waves, rb, nbuf;
     int ks = 1;  // workgroups splitting K (2: the staged form's halves, exchanging through slots)
 };
 
-A8Shape a8_shape(int token_blocks, int blocks) {
-    if (token_blocks == 2) return {8, 2, 2};
+A8Shape a8_shape(int blocks) {
     return blocks <= 256 ? A8Shape{16, 1, 2} : blocks <= 511 ? A8Shape{16, 2, 2} : A8Shape{8, 3, 2};
 }
 
@@ -573,17 +562,15 @@ void visit_one_block_shape(const A8Shape& sh, F&& f) {
     visit_shape<ShapeTag<16, 1, 2>, ShapeTag<16, 2, 2>, ShapeTag<8, 3, 2>>(sh, f);
 }
 
-template <int NB, int P>
+template <int P>
 void dispatch_a8_tiled(const std::int8_t* acodes, const float* ascales, const uint4* codes, const uint4* scales,
                        __half* out, int tokens, int n, int groups, int chunks, int blocks, hipStream_t stream) {
     auto launch = [&](auto tag) {
         using T = decltype(tag);
-        a8_tiled_decode<T::waves, T::rb, NB, P, T::nbuf><<<(blocks + T::rb - 1) / T::rb, T::waves * 64, 0, stream>>>(
+        a8_tiled_decode<T::waves, T::rb, P, T::nbuf><<<(blocks + T::rb - 1) / T::rb, T::waves * 64, 0, stream>>>(
             acodes, ascales, codes, scales, out, tokens, n, groups, chunks, blocks);
     };
-    const A8Shape sh = a8_shape(NB, blocks);
-    if constexpr (NB == 2) visit_shape<ShapeTag<8, 2, 2>>(sh, launch);
-    else visit_one_block_shape(sh, launch);
+    visit_one_block_shape(a8_shape(blocks), launch);
 }
 
 // LDS bytes of a8_tiled_lds: the activation rows of the workgroup's groups
@@ -658,7 +645,7 @@ struct A8TiledPlan {
 
 A8TiledPlan a8_tiled_plan(int tokens, int n, int k, int passes) {
     const int groups = (k + 31) / 32, blocks = (n + 15) / 16;
-    A8Shape sh = a8_shape(tokens <= 16 ? 1 : 2, blocks);
+    A8Shape sh = a8_shape(blocks);
     if (tokens > 16) return {false, sh, 0};
     std::size_t lds = a8_lds_bytes(tokens, groups, passes, sh);
     if (sh.waves == 8 && lds > kA8StageLdsMax / 2) {
@@ -679,7 +666,7 @@ A8TiledPlan a8_tiled_plan(int tokens, int n, int k, int passes) {
     const bool fits = lds <= (sh.waves == 16 ? kA8StageLdsMax : kA8StageLdsMax / 2) &&
                       2 * rows_groups <= kA8StageUnits * threads && rows_groups <= kA8StageScales * threads;
     if (fits) return {true, sh, lds};
-    return {false, a8_shape(1, blocks), 0};
+    return {false, a8_shape(blocks), 0};
 }
 
 }  // namespace
@@ -717,13 +704,20 @@ void a8_tiled_launch(const void* workspace, std::uint64_t available, const void*
                                      k, groups, chunks, blocks, plan.lds, stream);
         return;
     }
-    if (tokens <= 16) {
-        if (passes == 1) dispatch_a8_tiled<1, 1>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
-        else dispatch_a8_tiled<1, 2>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
-    } else {
-        if (passes == 1) dispatch_a8_tiled<2, 1>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
-        else dispatch_a8_tiled<2, 2>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
-    }
+    // Past 16 tokens, and where one token block's activations exceed the LDS of
+    // the forms above, the split form of the prefill GEMM reads the tiled
+    // planes. (Between 513 and 768 row blocks the register form stays the
+    // faster one at 9-16 tokens: 15232 columns x 732 blocks at 12 tokens, two
+    // passes, 59 against 65 us; 1088 blocks against it 72 -> 67, 320 blocks 63
+    // -> 49. Where the one-launch form could also serve the call, both steps
+    // keep its order of sums.)
+    const bool one_launch = a8_lds_bytes(tokens, groups, passes, a8_shape(blocks)) <= kA8FusedLdsMax;
+    if (tokens > 16 || (!one_launch && (blocks <= 512 || blocks > 768)))
+        a8_tiled_split_launch(workspace, codes, scales, out, tokens, n, k, padded, passes, stream);
+    else if (passes == 1)
+        dispatch_a8_tiled<1>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
+    else
+        dispatch_a8_tiled<2>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
 }
 
 void a8_tiled_linear_launch(const void* x, void* workspace, std::uint64_t available, const void* codes,
@@ -734,7 +728,7 @@ void a8_tiled_linear_launch(const void* x, void* workspace, std::uint64_t availa
     const int groups = (k + 31) / 32, chunks = padded / 64, blocks = (n + 15) / 16;
     // The fused kernel: one token block, whole 16-byte activation pieces, its
     // LDS within the default limit and every quantizer task in its one round.
-    const A8Shape sh = a8_shape(1, blocks);
+    const A8Shape sh = a8_shape(blocks);
     const std::size_t lds = a8_lds_bytes(tokens, groups, passes, sh);
     if (tokens > 16 || k % 8 != 0 || !aligned(x, 16) || lds > kA8FusedLdsMax ||
         4L * tokens * groups > static_cast<long>(kA8FusedTasks) * sh.waves * 64) {

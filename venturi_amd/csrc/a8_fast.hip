@@ -488,6 +488,183 @@ __global__ __launch_bounds__(WK * 64, 2) void a8_prefill_split(const std::int8_t
     store_partials<WK, TM, TN, P, G::kThreads>(o_lds, out, tokens, n, n0, [&](int row) { return t0 + row; });
 }
 
+// The split form over the tiled Q8 planes (the decode route's copy: codes
+// [row block][64-column chunk][lane 16q + m][two groups' 8 bytes], scales
+// [row block][chunk][row][2]), for 17-32 tokens and for fewer whose
+// activations exceed the decode kernels' LDS. A lane's 16 code bytes are its
+// fragments of a chunk's two groups and its 16 scale bytes the four rows'
+// pairs, so weights go straight to registers in 1 KB wave loads; activations
+// travel through the wave's LDS region as in the row-major form.
+template <int WK, int TI, int TJ>
+struct A8TiledGeom {
+    static constexpr int kThreads = WK * 64;
+    static constexpr int kTM = TI * 16, kTN = TJ * 16;
+    static constexpr int kAs = kTM * 128, kWave = kAs + 4 * 64 * 4;
+    static constexpr int kPitch = kTN + 4;
+    static constexpr int kOut = WK * kTM * kPitch * 4;
+    static constexpr int kLds = WK * kWave > kOut ? WK * kWave : kOut;
+    static_assert(kTM <= 64 && kLds <= 160 * 1024, "tiled split tile exceeds LDS");
+};
+
+template <int TJ>
+struct A8TiledSource {
+    const unsigned char *pa, *psa;
+    const u32x4 *codes, *scales;  // [TJ] of the 64-column chunk that holds the group
+    int odd;                      // second group of the chunk
+    __device__ __forceinline__ long a(int i) const { return *reinterpret_cast<const long*>(pa + i * 2048); }
+    __device__ __forceinline__ float a_scale(int i) const { return *reinterpret_cast<const float*>(psa + i * 64); }
+    __device__ __forceinline__ long b(int j) const {
+        return static_cast<long>(static_cast<std::uint64_t>(codes[j][2 * odd]) |
+                                 static_cast<std::uint64_t>(codes[j][2 * odd + 1]) << 32);
+    }
+    __device__ __forceinline__ float4 b_scale(int j) const {
+        const u32x4 s = scales[j];
+        return odd ? make_float4(half_hi(s[0]), half_hi(s[1]), half_hi(s[2]), half_hi(s[3]))
+                   : make_float4(half_lo(s[0]), half_lo(s[1]), half_lo(s[2]), half_lo(s[3]));
+    }
+};
+
+template <int WK, int TI, int TJ>
+__global__ __launch_bounds__(WK * 64, WK > 8 ? WK / 4 : 2) void a8_tiled_split(
+    const std::int8_t* __restrict__ acodes, const float* __restrict__ ascales, const u32x4* __restrict__ wcodes,
+    const u32x4* __restrict__ wscales, __half* __restrict__ out, int tokens, int n, int padded, int groups, int passes) {
+    using G = A8TiledGeom<WK, TI, TJ>;
+    constexpr int TM = G::kTM, TN = G::kTN, kA = 2 * TI;
+    static_assert(WK >= 2, "the last chunk of each pass is a wave's first");
+    extern __shared__ uint4 a8p_lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = lane >> 4, r = lane & 15;
+    const int block0 = blockIdx.x * TJ, blocks = (n + 15) / 16;
+    auto* lds = reinterpret_cast<unsigned char*>(a8p_lds) + wave * G::kWave;
+
+    const int chunks = padded / 128, inner = chunks - 1, total = passes * chunks;
+    A8Tile<TI, TJ> m;
+    m.clear();
+    if (wave < total) {
+        const std::int64_t count = static_cast<std::int64_t>(tokens) * groups;
+        // Activation unit u of a lane: row lane / 8 + 8 u, unit lane % 8 of the
+        // chunk's 128 bytes; scales: row lane. Where the only chunk is partial,
+        // the requests that are never consumed stay inside the first row.
+        const std::int8_t* a_src[kA];
+        const bool whole = inner > 0 || groups >= 4;
+#pragma unroll
+        for (int u = 0; u < kA; ++u)
+            a_src[u] = acodes + static_cast<std::int64_t>(min(lane / 8 + 8 * u, tokens - 1)) * groups * 32 +
+                       (whole ? 16 * (lane % 8) : 0);
+        const float* as_src = ascales + (whole ? static_cast<std::int64_t>(min(lane, tokens - 1)) * groups : 0);
+        const u32x4 *b_src[TJ], *s_src[TJ];
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const std::int64_t blk = min(block0 + j, blocks - 1);  // clamped blocks are never stored
+            b_src[j] = wcodes + blk * (2 * chunks) * 64 + lane;
+            s_src[j] = wscales + blk * (2 * chunks) * 4 + q;
+        }
+        u32x4 st_a[kA], codes[2][TJ], scales[2][TJ];
+        float4u st_as;
+        // Virtual chunk v: the last chunk of each pass first, then the others;
+        // past the end, chunk 0 of pass 0 (never consumed).
+        auto locate = [&](int v, int& pass, std::int64_t& c) __attribute__((always_inline)) {
+            const int w = v < total ? v - passes : 0;
+            pass = v < passes ? v : w >= inner && w > 0 ? 1 : 0;
+            c = v < passes ? inner : w - (w >= inner && w > 0 ? inner : 0);
+        };
+        auto load_b = [&](int v, int h) __attribute__((always_inline)) {
+            int pass;
+            std::int64_t c;
+            locate(v, pass, c);
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) {
+                codes[h][j] = __builtin_nontemporal_load(b_src[j] + (2 * c + h) * 64);
+                scales[h][j] = __builtin_nontemporal_load(s_src[j] + (2 * c + h) * 4);
+            }
+        };
+        auto load_a = [&](int v) __attribute__((always_inline)) {
+            int pass;
+            std::int64_t c;
+            locate(v, pass, c);
+#pragma unroll
+            for (int u = 0; u < kA; ++u)
+                st_a[u] = *reinterpret_cast<const u32x4*>(a_src[u] + pass * count * 32 + c * 128);
+            st_as = *reinterpret_cast<const float4u*>(as_src + pass * count + c * 4);
+        };
+        // The last chunk of a pass: groups past the last one carry scale 0 (their codes are clamped, finite).
+        auto load_edge = [&](int pass) __attribute__((always_inline)) {
+            const int real = groups - 4 * inner;  // 1 .. 4
+            const int unit = min(8 * inner + lane % 8, 2 * groups - 1);
+#pragma unroll
+            for (int u = 0; u < kA; ++u)
+                st_a[u] = *reinterpret_cast<const u32x4*>(
+                    acodes + pass * count * 32 +
+                    (static_cast<std::int64_t>(min(lane / 8 + 8 * u, tokens - 1)) * groups * 2 + unit) * 16);
+            const float* as = ascales + pass * count + static_cast<std::int64_t>(min(lane, tokens - 1)) * groups;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float v = as[min(4 * inner + g, groups - 1)];
+                st_as[g] = g < real ? v : 0.0f;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const std::uint32_t keep = (2 * h < real ? 0x0000ffffu : 0u) | (2 * h + 1 < real ? 0xffff0000u : 0u);
+                        scales[h][j][e] &= keep;
+                    }
+        };
+        std::uint32_t put[2];
+#pragma unroll
+        for (int odd = 0; odd < 2; ++odd) put[odd] = 16 * ((lane / 8) * 8 + ((lane % 8) ^ swizzle<8>(lane / 8 + 8 * odd)));
+        auto store = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int u = 0; u < kA; ++u) *reinterpret_cast<u32x4*>(lds + put[u & 1] + u * 1024) = st_a[u];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) *reinterpret_cast<float*>(lds + G::kAs + 4 * (64 * g + lane)) = st_as[g];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        };
+        std::uint32_t get[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) get[g] = 16 * (r * 8 + ((2 * g + (q >> 1)) ^ swizzle<8>(r))) + 8 * (q & 1);
+        auto source = [&](auto g) __attribute__((always_inline)) {
+            return A8TiledSource<TJ>{lds + get[g], lds + G::kAs + 4 * (64 * g + r), codes[g / 2], scales[g / 2], g % 2};
+        };
+        load_b(wave, 0);
+        load_b(wave, 1);
+        if (wave < passes) {
+            load_edge(wave);
+            store();
+        } else {
+            load_a(wave);
+            store();
+        }
+        load_a(wave + WK);
+        m.fill(source(Slot<0>{}));
+        for (int v = wave; v < total; v += WK) {
+            each_slot<4>([&](auto g) __attribute__((always_inline)) {
+                m.group(source(Slot<(g + 1) % 4>{}), [&](int t) __attribute__((always_inline)) {
+                    // The first half of the chunk is in use until group 1's
+                    // operands are taken, the second until group 3's.
+                    if (g == 1 && t == 0) load_b(v + WK, 0);
+                    if (g == 3 && t == 0) {
+                        load_b(v + WK, 1);
+                        store();  // every read of this chunk is issued
+                        load_a(v + 2 * WK);
+                    }
+                });
+            });
+        }
+    }
+
+    auto* o_lds = reinterpret_cast<float*>(a8p_lds);
+    constexpr int P = G::kPitch;
+    __syncthreads();
+    m.template put<0, TI, P>(o_lds + wave * TM * P, r, q);
+    __syncthreads();
+    store_partials<WK, TM, TN, P, G::kThreads>(o_lds, out, tokens, n, block0 * 16, [&](int row) { return row; });
+}
+
 struct A8Operands {
     const std::int8_t* acodes;
     const float* ascales;
@@ -557,6 +734,47 @@ void a8_fast_launch(const void* workspace, const std::int8_t* codes, const __hal
         case 7: launch_split<8, 2, 4>(o, stream); break;
         default: launch_split<8, 2, 2>(o, stream); break;
     }
+}
+
+template <int WK, int TI, int TJ>
+void launch_tiled_split(const std::int8_t* acodes, const float* ascales, const u32x4* codes, const u32x4* scales,
+                        __half* out, int tokens, int n, int padded, int groups, int passes, hipStream_t stream) {
+    using G = A8TiledGeom<WK, TI, TJ>;
+    const auto kernel = a8_tiled_split<WK, TI, TJ>;
+    static const bool raised = (raise_lds(kernel, G::kLds), true);
+    static_cast<void>(raised);
+    kernel<<<(n + G::kTN - 1) / G::kTN, G::kThreads, G::kLds, stream>>>(acodes, ascales, codes, scales, out, tokens, n,
+                                                                       padded, groups, passes);
+}
+
+// Operands are admitted by the caller (a8_tiled_launch); at most 32 tokens.
+void a8_tiled_split_launch(const void* workspace, const void* codes, const void* scales, void* out, int tokens, int n,
+                           int k, int padded, int passes, hipStream_t stream) {
+    const int groups = (k + 31) / 32;
+    const std::int64_t count = static_cast<std::int64_t>(tokens) * groups;
+    const auto* acodes = static_cast<const std::int8_t*>(workspace);
+    const auto* ascales = reinterpret_cast<const float*>(acodes + count * 32 * passes);
+    const auto* cp = static_cast<const u32x4*>(codes);
+    const auto* sp = static_cast<const u32x4*>(scales);
+    auto* op = static_cast<__half*>(out);
+    const int blocks = (n + 15) / 16;
+    auto launch = [&](auto waves, auto row_blocks) {
+        if (tokens > 16)
+            launch_tiled_split<waves, 2, row_blocks>(acodes, ascales, cp, sp, op, tokens, n, padded, groups, passes, stream);
+        else
+            launch_tiled_split<waves, 1, row_blocks>(acodes, ascales, cp, sp, op, tokens, n, padded, groups, passes, stream);
+    };
+    // Row blocks per workgroup so that up to 768 blocks make at most one
+    // workgroup of eight K waves per CU; beyond, four K waves and two
+    // workgroups per CU (at up to 16 tokens from 1024 blocks). MI355X, 32
+    // tokens, one pass, against the per-lane fragment form this replaces, us:
+    // 4096 x 4096 19.2 -> 8.5, 7168 x 5120 24.1 -> 15.2, 5120 x 17408 71 -> 35,
+    // 11702 x 15232 106 -> 43, 34816 x 5120 106 -> 45; the neighbouring shapes
+    // of the rule measured up to 1.5x slower there.
+    if (blocks <= 256) launch(Slot<8>{}, Slot<1>{});
+    else if (blocks <= 512 || (tokens <= 16 && blocks <= 1024)) launch(Slot<8>{}, Slot<2>{});
+    else if (blocks <= 768) launch(Slot<8>{}, Slot<3>{});
+    else launch(Slot<4>{}, Slot<3>{});
 }
 
 }  // namespace vt
