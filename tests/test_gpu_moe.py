@@ -233,3 +233,39 @@ def test_moe_graph_replays(backend, device, geometry, tokens):
         graph.replay()
         torch.cuda.synchronize(device)
         assert np.array_equal(bits(out), bits(eager)), replay
+
+
+# Few pairs (the form of decode steps). Rows of a pass are min(16, 67584 // (2 * (256-column chunks of K + 8))) and the
+# launch shapes go by the expected active row blocks, so: up to 2048 and 2560 blocks (gate/up, down), up to 9000, more;
+# K below one chunk, odd chunk counts and ragged last chunks; experts with more tokens than a pass holds (hidden 4104:
+# seven rows); one expert; 1024 experts (sixteen per scanning lane); the largest pair count.
+@pytest.mark.parametrize(
+    "geometry,tokens",
+    [
+        (MoEGeometry(136, 8, 2, 72), 3),
+        (MoEGeometry(2056, 8, 4, 264), 15),
+        (MoEGeometry(1288, 1, 1, 520), 16),
+        (MoEGeometry(4104, 40, 8, 8), 17),
+        (MoEGeometry(72, 128, 8, 600), 64),
+        (MoEGeometry(520, 128, 8, 344), 64),
+        (MoEGeometry(776, 48, 8, 1032), 48),
+        (MoEGeometry(64, 1024, 16, 8), 32),
+    ],
+)
+def test_moe_few_pairs(backend, device, geometry, tokens):
+    run_and_check(backend, device, geometry, tokens, seed=31 + tokens, duplicates=geometry.top_k >= 4)
+
+
+def test_moe_few_pairs_without_a_valid_id(backend, device):
+    geometry = MoEGeometry(128, 8, 2, 64)
+    print("case moe few pairs, no valid id", flush=True)
+    bank, _, _ = build(backend, device, geometry, 5)
+    x, ids, scores = routing(3, geometry, 6)
+    plan = bank.prepare(tokens=3)
+    workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=device)
+    out = torch.zeros(3, 128, dtype=torch.float16, device=device)
+    ids = torch.where(ids % 2 == 0, ids + 8, ids - 8)
+    plan.run(x.to(device), ids.to(device), scores.to(device), out=out, workspace=workspace)
+    views = plan.workspace_views(workspace)
+    assert int(views["status"][0]) == 6 and not bool(views["seg"].any()) and bool((views["pair_slot"] == -1).all())
+    assert bool(torch.isnan(out).all())

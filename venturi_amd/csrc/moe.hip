@@ -23,6 +23,7 @@
 #include "common.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace vt {
@@ -642,6 +643,273 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) 
     }
 }
 
+// ---------------------------------------------------------------------------
+// Few pairs: the grouped GEMM of decode steps (a handful of tokens per active
+// expert) over the same tiled planes, bound by the weight stream of the active
+// experts (8 tokens, 128 experts of 768 x 2048, top 8: 50 experts, 129 MB).
+//
+// q4_grouped at that size has few of its workgroups active, on the XCDs that
+// the routing happens to name, and pays a barrier per 256-column chunk. Here
+// * workgroup i takes part i % parts of the (i / parts)-th expert that has any
+//   pair, so the active experts' parts spread over every XCD and the
+//   workgroups without work are the last ones;
+// * a pass's activation rows (up to 16, whole K) are staged in LDS once; the
+//   waves then run without a barrier, WK of them sharing a row block's K (their
+//   sums meet in LDS, in wave order) and each streaming half chunks (1 KB per
+//   row block) of RB row blocks two ahead.
+// MI355X, 2048 x 768 x 128 experts, top 8, routed call, before -> after, us:
+// one token 43.6 -> 17.3, 4 tokens 52.6 -> 28, 8 tokens 55.5 -> 40, 16 tokens
+// 68 -> 57, 32 tokens 74.5 -> 67. Activations read per lane from L2 instead of
+// LDS needed 32 more registers and spilled.
+
+typedef std::uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kFewPairs = 512;      // pairs at most: one per thread routes them
+constexpr int kFewLds = 66 * 1024;  // activation rows of a pass: two workgroups share a CU
+
+template <int RB>
+struct FewItem {  // half of a chunk for a wave's row blocks: codes and group scales
+    u32x4 w[RB];
+    unsigned short s[RB];
+};
+
+template <int EPI, int WK, int RB, bool ROUTE>
+__global__ __launch_bounds__(512, 4) void q4_few(Q4Tiled p, int parts, int blocks, int rows) {
+    constexpr int W = 8, WR = W / WK;
+    extern __shared__ uint4 few_lds[];  // activation rows of a pass, then the waves' partial tiles
+    auto* xl = reinterpret_cast<_Float16*>(few_lds);
+    auto* partial = reinterpret_cast<float4v*>(few_lds);
+    __shared__ int count[ROUTE ? kMaxExperts : 1];
+    __shared__ int invalid;
+    __shared__ unsigned short elist[ROUTE ? kFewPairs : 1];
+    __shared__ unsigned short plist[ROUTE ? kFewPairs : 1];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, m = lane & 15;
+    const int wk = wave / WR, wr = wave % WR;
+    const int active = blockIdx.x / parts, part = blockIdx.x % parts;
+
+    // Pairs per expert, then the active-th expert that has any.
+    if constexpr (ROUTE) {
+        const std::int64_t e = p.ids[min(tid, p.pairs - 1)];
+        for (int i = tid; i < p.experts; i += 512) count[i] = 0;
+        if (tid == 0) invalid = 0;
+        __syncthreads();
+        if (tid < p.pairs) {
+            const bool ok = e >= 0 && e < p.experts;
+            elist[tid] = ok ? static_cast<unsigned short>(e) : 0xFFFFu;
+            atomicAdd(ok ? &count[e] : &invalid, 1);
+        }
+        __syncthreads();
+    }
+    const int run = (p.experts + 63) / 64;
+    const int lo = min(lane * run, p.experts), hi = min(lo + run, p.experts);
+    auto pairs_of = [&](int e) { return ROUTE ? count[e] : p.seg[e + 1] - p.seg[e]; };
+    int own = 0;  // pairs in the upper half, experts with any in the lower
+    for (int e = lo; e < hi; ++e) {
+        const int c = pairs_of(e);
+        own += (c << 16) + (c > 0);
+    }
+    int incl = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int other = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += other;
+    }
+    int rank = (incl - own) & 0xFFFF, first = (incl - own) >> 16;
+    int found = -1, found_first = 0, found_count = 0;
+    const bool tables = ROUTE && blockIdx.x == 0 && wave == 0;
+    for (int e = lo; e < hi; ++e) {
+        const int c = pairs_of(e);
+        if (c > 0 && rank++ == active) {
+            found = e;
+            found_first = first;
+            found_count = c;
+        }
+        first += c;
+        if (tables) p.seg_out[e + 1] = first;
+    }
+    if (tables) {
+        if (lane == 0) {
+            p.seg_out[0] = 0;
+            *p.status = invalid;
+        }
+        for (int i = lane; i < p.pairs; i += 64)
+            if (elist[i] == 0xFFFFu) p.pair_slot[i] = -1;
+    }
+    const std::uint64_t holder = __ballot(found >= 0);
+    if (holder == 0) return;  // fewer experts than this are active
+    const int source = __builtin_ctzll(holder);
+    const int expert = __builtin_amdgcn_readlane(found, source);
+    const int begin = __builtin_amdgcn_readlane(found_first, source);
+    const int total = __builtin_amdgcn_readlane(found_count, source);
+
+    if constexpr (ROUTE) {  // every wave ranks the pairs itself, all with the same result
+        int at = 0;
+        for (int base = 0; base < p.pairs; base += 64) {
+            const int i = base + lane;
+            const bool mine = i < p.pairs && elist[min(i, p.pairs - 1)] == expert;
+            const std::uint64_t hits = __ballot(mine);
+            if (mine) {
+                const int r = at + __popcll(hits & ((1ull << lane) - 1));
+                plist[r] = static_cast<unsigned short>(i);
+                if (part == 0 && wave == 0) {
+                    p.pair_slot[i] = begin + r;
+                    p.slot_token[begin + r] = i / p.top_k;
+                    p.slot_score[begin + r] = p.scores[i];
+                }
+            }
+            at += __popcll(hits);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+
+    const BiasedMasks masks = biased_masks();
+    const char* wbase = reinterpret_cast<const char*>(p.codes + expert * p.code_stride);
+    const char* sbase = reinterpret_cast<const char*>(p.scales + expert * p.scale_stride);
+    const int block0 = part * WR * RB;
+    std::int64_t unit[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        const int b = min(block0 + wr * RB + r, blocks - 1);
+        unit[r] = static_cast<std::int64_t>(b >> 3) * p.chunks * 8 + (b & 7);
+    }
+    const int items = 2 * p.chunks;
+    const int i0 = items * wk / WK, i1 = items * (wk + 1) / WK;
+
+    const int stride = p.chunks * kChunk + 8;
+    for (int pass = 0; pass < total; pass += rows) {
+        const int live = min(rows, total - pass);
+        float score[4];
+        if constexpr (EPI == kScore) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) score[i] = __half2float(p.score[begin + pass + min(4 * q + i, live - 1)]);
+        }
+        // Activations: half a wave per (row, chunk), four of them in flight.
+        constexpr int XU = 4;
+        const int units = live * p.chunks;
+        u32x4 xv[XU];
+        int xat[XU];
+        auto load_x = [&](int base) {
+#pragma unroll
+            for (int j = 0; j < XU; ++j) {
+                const int u = base + 16 * j + 2 * wave + (lane >> 5);
+                const int t = min(u, units - 1) / p.chunks, c = min(u, units - 1) - t * p.chunks;
+                const int row = ROUTE ? plist[pass + t] / p.top_k : begin + pass + t;
+                const int col = c * kChunk + 8 * (lane & 31);
+                xat[j] = u < units ? t * stride + col : -1;
+                xv[j] = *reinterpret_cast<const u32x4*>(p.x + static_cast<std::int64_t>(row) * p.x_stride + min(col, p.k - 8));
+                if (col >= p.k) xv[j] = u32x4{0, 0, 0, 0};
+            }
+        };
+        auto store_x = [&] {
+#pragma unroll
+            for (int j = 0; j < XU; ++j) {
+                u32x4 v;
+                v.x = __builtin_amdgcn_perm(xv[j].z, xv[j].x, 0x05040100u);
+                v.y = __builtin_amdgcn_perm(xv[j].z, xv[j].x, 0x07060302u);
+                v.z = __builtin_amdgcn_perm(xv[j].w, xv[j].y, 0x05040100u);
+                v.w = __builtin_amdgcn_perm(xv[j].w, xv[j].y, 0x07060302u);
+                if (xat[j] >= 0) *reinterpret_cast<u32x4*>(xl + xat[j]) = v;
+            }
+        };
+        auto load = [&](int i, FewItem<RB>& t) {
+            const int c = i >> 1, h = i & 1;
+            std::uint32_t at = 16 * lane, sat = 2 * lane;
+            asm volatile("" : "+v"(at), "+v"(sat));
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+                const std::int64_t u = unit[r] + static_cast<std::int64_t>(c) * 8;
+                t.w[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wbase + u * 2048 + 1024 * h + at));
+                t.s[r] = __builtin_nontemporal_load(reinterpret_cast<const unsigned short*>(sbase + u * 128 + sat));
+            }
+        };
+        float4v acc[RB];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) acc[r] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        const _Float16* xf0 = xl + min(m, live - 1) * stride + 64 * q;
+        auto compute = [&](int i, FewItem<RB>& t) {
+            const _Float16* xi = xf0 + (i >> 1) * kChunk + 32 * (i & 1);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const half8 xf = *reinterpret_cast<const half8*>(xi + 8 * s);
+#pragma unroll
+                for (int r = 0; r < RB; ++r) {
+                    std::uint32_t word = t.w[r][s], scale = t.s[r];
+                    asm volatile("" : "+v"(word), "+v"(scale));
+                    const half2v s2 = __builtin_bit_cast(half2v, scale * 0x10001u);
+                    acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf, dequant8_biased(word, s2, masks), acc[r], 0, 0, 0);
+                }
+            }
+        };
+        FewItem<RB> b0, b1;
+        load_x(0);
+        load(min(i0, items - 1), b0);
+        load(min(i0 + 1, items - 1), b1);
+        store_x();
+        for (int base = 16 * XU; base < units; base += 16 * XU) {
+            load_x(base);
+            store_x();
+        }
+        __syncthreads();
+        if (i0 < i1) {
+            int i = i0;
+            for (; i + 3 < i1; i += 2) {
+                compute(i, b0);
+                load(i + 2, b0);
+                compute(i + 1, b1);
+                load(i + 3, b1);
+            }
+            compute(i, b0);
+            if (i + 1 < i1) {
+                if (i + 2 < i1) load(i + 2, b0);
+                compute(i + 1, b1);
+                if (i + 2 < i1) compute(i + 2, b0);
+            }
+        }
+
+        auto store = [&](float4v y, int blk) {
+            if (blk >= blocks) return;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = 4 * q + i;
+                __half* o = p.out + static_cast<std::int64_t>(begin + pass + t) * p.out_stride;
+                if (EPI == kSwiGLU) {
+                    const float other = __shfl_xor(y[i], 8, 64);  // lane m^8 holds the paired up row
+                    const int col = (blk >> 3) * (kRows / 2) + 8 * (blk & 7) + m;
+                    if (m < 8 && t < live && col < p.half_rows) {
+                        const float g = __half2float(from_f32<__half>(y[i]));
+                        const float u = __half2float(from_f32<__half>(other));
+                        const float a = __half2float(from_f32<__half>(silu(g)));
+                        o[col] = from_f32<__half>(__fmul_rn(a, u));
+                    }
+                } else {
+                    const int col = 16 * blk + m;
+                    if (t < live && col < p.n)
+                        o[col] = from_f32<__half>(__fmul_rn(__half2float(from_f32<__half>(y[i])), score[i]));
+                }
+            }
+        };
+        if constexpr (WK == 1) {
+#pragma unroll
+            for (int r = 0; r < RB; ++r) store(acc[r], block0 + wr * RB + r);
+        } else {
+            __syncthreads();  // the activations have been read
+#pragma unroll
+            for (int r = 0; r < RB; ++r) partial[(wave * RB + r) * 64 + lane] = acc[r];
+            __syncthreads();
+            for (int b = wave; b < WR * RB; b += W) {
+                float4v y = partial[b * 64 + lane];  // K part 0: waves 0 .. WR - 1
+#pragma unroll
+                for (int w = 1; w < WK; ++w) y += partial[(w * WR * RB + b) * 64 + lane];
+                store(y, block0 + b);
+            }
+        }
+        __syncthreads();  // the next pass restages the LDS
+    }
+}
+
 // Routing: one workgroup of kRouteThreads. Pair i = token * top_k + position.
 // Pass 1 counts pairs per expert (LDS atomics give each pair a rank in its
 // expert); wave 0 turns the counts into segment offsets (each lane sums a run
@@ -831,6 +1099,60 @@ void launch_q4_grouped(const Q4Tiled& p, hipStream_t stream) {
     const int parts = (blocks + W * RB - 1) / (W * RB);
     const int wgs = (parts + TT - 1) / TT;
     q4_grouped<EPI, W, RB, NBMAX, ROUTE, TT><<<dim3(p.experts * wgs), W * 64, 0, stream>>>(p, parts, blocks);
+}
+
+// Activation rows that a pass of q4_few stages.
+int few_rows(const Q4Tiled& p) { return std::min(16, kFewLds / (2 * (p.chunks * kChunk + 8))); }
+
+template <int EPI, int WK, int RB, bool ROUTE>
+void launch_q4_few(const Q4Tiled& p, int active, hipStream_t stream) {
+    const int blocks = p.row_tiles * 8;
+    constexpr int kCover = 8 / WK * RB;
+    const int parts = (blocks + kCover - 1) / kCover;
+    const int rows = few_rows(p);
+    const int lds = std::max(rows * 2 * (p.chunks * kChunk + 8), WK > 1 ? 8 * RB * 1024 : 0);
+    if (lds > 48 * 1024) {
+        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(q4_few<EPI, WK, RB, ROUTE>),
+                                                             hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds);
+        check(raised);
+    }
+    q4_few<EPI, WK, RB, ROUTE><<<active * parts, 512, lds, stream>>>(p, parts, blocks, rows);
+}
+
+// Whether q4_few is the faster form: one pass per expert in nearly every case
+// (no more tokens than rows of a pass, or on average half of them per expert).
+// MI355X, us, q4_grouped against q4_few for gate/up: 4 tokens per expert 78 ->
+// 70 (2048 columns, 16 rows a pass), 8 per expert 131 -> 156 (4096 columns, 8
+// rows); down at 8 per expert 131 -> 123, at 16 per expert 154 -> 161.
+bool few_pairs(const Q4Tiled& p, int tokens, int pairs) {
+    const int rows = few_rows(p);
+    return pairs <= kFewPairs && rows > 0 && (tokens <= rows || 2 * pairs <= p.experts * rows);
+}
+
+// Row blocks of the experts that `pairs` uniformly routed pairs touch.
+double active_blocks(const Q4Tiled& p, int pairs) {
+    return p.experts * (1.0 - std::pow(1.0 - 1.0 / p.experts, pairs)) * p.row_tiles * 8;
+}
+
+// Shapes by the row blocks that the launch streams: K shared by several waves
+// and few row blocks per workgroup while there are too few blocks to give
+// every CU two workgroups, longer runs of K per wave beyond, where each
+// workgroup's start (routing, staging) counts. Gate/up (K 1024-4096), us, as
+// (WK, RB): 768 blocks (4,2) 27, (2,2) 29, (1,2) 34; 4500 blocks 71, 68, 72;
+// 10700 blocks 81, 70, 65. Down (K 256-1536): 1024 blocks (2,1) 35, (1,2) 36;
+// 512 blocks 38, 42; 3600 blocks 45, 42; 8000 blocks 80, 65.
+void gate_up_few(const Q4Tiled& p, int pairs, hipStream_t stream) {
+    const int active = std::min(pairs, p.experts);
+    const double blocks = active_blocks(p, pairs);
+    if (blocks <= 2048) launch_q4_few<kSwiGLU, 4, 2, true>(p, active, stream);
+    else if (blocks <= 9000) launch_q4_few<kSwiGLU, 2, 2, true>(p, active, stream);
+    else launch_q4_few<kSwiGLU, 1, 2, true>(p, active, stream);
+}
+
+void down_few(const Q4Tiled& p, int pairs, hipStream_t stream) {
+    const int active = std::min(pairs, p.experts);
+    if (active_blocks(p, pairs) <= 2560) launch_q4_few<kScore, 2, 1, false>(p, active, stream);
+    else launch_q4_few<kScore, 1, 2, false>(p, active, stream);
 }
 
 std::uint64_t align256(std::uint64_t v) { return (v + 255) / 256 * 256; }
@@ -1517,7 +1839,8 @@ void moe_q4_launch_cfg(const void* x, const std::int64_t* ids, const void* score
     gu.slot_score = slot_score;
     gu.pairs = pairs;
     gu.top_k = top_k;
-    if (route_inside) launch_q4_grouped<kSwiGLU, GW, GRB, NBMAX, true, 1>(gu, stream);
+    if (few_pairs(gu, tokens, pairs)) gate_up_few(gu, pairs, stream);
+    else if (route_inside) launch_q4_grouped<kSwiGLU, GW, GRB, NBMAX, true, 1>(gu, stream);
     else launch_q4_grouped<kSwiGLU, GW, GRB, NBMAX, false, 1>(gu, stream);
 
     Q4Tiled dn{};
@@ -1536,7 +1859,8 @@ void moe_q4_launch_cfg(const void* x, const std::int64_t* ids, const void* score
     dn.x_stride = inter;
     dn.out_stride = hidden;
     dn.experts = experts;
-    launch_q4_grouped<kScore, DW, DRB, NBMAX, false, 2>(dn, stream);
+    if (few_pairs(dn, tokens, pairs)) down_few(dn, pairs, stream);
+    else launch_q4_grouped<kScore, DW, DRB, NBMAX, false, 2>(dn, stream);
 
     combine_dispatch(top_k, ids, pair_slot, v, static_cast<__half*>(out), tokens, hidden, stream);
 }
