@@ -14,7 +14,7 @@ import torch
 
 from . import native
 from .backend import Backend, BackendCapabilities, OperatorSupport, UnsupportedOperationError
-from .operands import DTYPE_CODES, admit, disjoint, epsilon as admit_epsilon, extents, stream_of
+from .operands import DTYPE_CODES, admit, disjoint, epsilon as admit_epsilon, extents, on_device, stream_of
 from .weights import DenseWeight, Q4RowSplitWeight, Q8RowSplitWeight
 
 Q8_ROUTES = ("auto", "exact", "mfma", "dense")
@@ -165,7 +165,7 @@ class HipBackend(Backend):
         """Calls one C entry point on `device`'s current stream: tensors pass as data pointers,
         every other operand as it is; a -1 return raises the library's message."""
         arguments = [v.data_ptr() if isinstance(v, torch.Tensor) else v for v in operands]
-        with torch.cuda.device(device):
+        with on_device(device):
             self._check(getattr(self._native, entry)(*arguments, stream_of(device)))
 
     def synchronize(self, device):

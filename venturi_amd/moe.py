@@ -20,7 +20,7 @@ from dataclasses import dataclass
 
 import torch
 
-from .operands import admit, disjoint, stream_of
+from .operands import admit, disjoint, on_device, stream_of
 from .weights import Q4RowSplitWeight
 
 
@@ -207,7 +207,7 @@ class RoutedExpertsPlan:
             raise ValueError(f"workspace requires {self.workspace_bytes} bytes at 256-byte alignment")
         disjoint(out, (x, indices, scores, workspace) + b.storage_tensors)
         disjoint(workspace, (x, indices, scores) + b.storage_tensors)
-        with torch.cuda.device(b.device):
+        with on_device(b.device):
             b.backend._check(
                 b.backend._native.venturi_moe_q4_run(
                     x.data_ptr(), indices.data_ptr(), scores.data_ptr(),

@@ -11,7 +11,7 @@ from functools import cached_property
 
 import torch
 
-from .operands import DTYPE_CODES, admit, disjoint, extents, stream_of
+from .operands import DTYPE_CODES, admit, disjoint, extents, on_device, stream_of
 from .plugin import CodecEntry, RowCodecOperator
 from .weights import Q4RowSplitWeight, decode_k64_fp16, rtn_k64
 
@@ -230,7 +230,7 @@ class Q4LinearPlan:
             disjoint(workspace, (x, out) + self.storage_tensors)
         w, lib, stream = r.weight, r.backend._native, stream_of(r.device)
         args = (x.data_ptr(), w.codes.data_ptr(), w.scales.data_ptr(), out.data_ptr())
-        with torch.cuda.device(r.device):
+        with on_device(r.device):
             if kernel == "dense":
                 status = lib.venturi_row_dense_run(
                     *args[:2], None, *args[2:], self.tokens, w.out_features, w.in_features, w.padded_k, 4,

@@ -26,7 +26,7 @@ from dataclasses import dataclass
 import torch
 
 from .blocks import ResidentLinear
-from .operands import admit, disjoint, extents, stream_of
+from .operands import admit, disjoint, extents, on_device, stream_of
 from .vocabulary import ResidentQ8Vocabulary
 
 A8_ROUTES = ("auto", "exact", "mfma")
@@ -60,7 +60,7 @@ class PreparedQ8DP4A:
         disjoint(workspace, (x,) + r.storage_tensors)
         if workspace.data_ptr() % 16:
             raise ValueError("A8 workspace requires 16-byte alignment")
-        with torch.cuda.device(r.device):
+        with on_device(r.device):
             r.backend._check(
                 self._native.venturi_q8_dp4a_quantize(
                     x.data_ptr(), workspace.data_ptr(), self.workspace_bytes, self.tokens, r.hidden_size,
@@ -85,7 +85,7 @@ class PreparedQ8DP4A:
         else:
             entry = self._native.venturi_q8_dp4a_run if self.kernel == "exact" else self._native.venturi_q8_a8_gemm_run
             codes, scales = r.row_major_planes()
-        with torch.cuda.device(r.device):
+        with on_device(r.device):
             r.backend._check(
                 entry(
                     workspace.data_ptr(), self.workspace_bytes, codes.data_ptr(), scales.data_ptr(),
@@ -115,7 +115,7 @@ class PreparedQ8DP4A:
             self.quantize(x, workspace=workspace)
             return self.project(out=out, workspace=workspace)
         codes, scales = r.tiled_planes()
-        with torch.cuda.device(r.device):
+        with on_device(r.device):
             r.backend._check(
                 self._native.venturi_q8_a8_tiled_linear_run(
                     x.data_ptr(), workspace.data_ptr(), self.workspace_bytes, codes.data_ptr(), scales.data_ptr(),

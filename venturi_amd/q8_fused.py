@@ -20,7 +20,7 @@ from dataclasses import dataclass
 import torch
 
 from .blocks import ResidentLinear
-from .operands import admit, disjoint, stream_of
+from .operands import admit, disjoint, on_device, stream_of
 from .q8_dp4a import prepare_q8_dp4a
 
 _INT32_LIMIT = 2**31
@@ -85,7 +85,7 @@ class PreparedQ8Fused:
         table = self._descriptors(outputs)
         lead, a8 = self.residents[0], self.base
         backend = lead.backend
-        with torch.cuda.device(lead.device):
+        with on_device(lead.device):
             stream = stream_of(lead.device)
             if not packed:
                 backend._check(backend._native.venturi_q8_dp4a_quantize(

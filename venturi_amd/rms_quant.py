@@ -12,7 +12,7 @@ from dataclasses import dataclass
 import torch
 
 from .blocks import ResidentRMSNorm
-from .operands import admit, disjoint, extents, stream_of
+from .operands import admit, disjoint, extents, on_device, stream_of
 
 
 @dataclass(frozen=True)
@@ -34,7 +34,7 @@ class PreparedRMSQ8:
         if workspace.data_ptr() % 16:
             raise ValueError("A8 workspace requires 16-byte alignment")
         lib = n._backend._native
-        with torch.cuda.device(n.device):
+        with on_device(n.device):
             n._backend._check(
                 lib.venturi_rms_q8_quantize_passes(
                     x.data_ptr(), n._weight.data_ptr(), workspace.data_ptr(), self.workspace_bytes, self.tokens, k,

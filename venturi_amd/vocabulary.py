@@ -44,7 +44,7 @@ import threading
 import torch
 
 from .blocks import Q8_ROUTES
-from .operands import DTYPE_CODES, admit, disjoint, extents, stream_of
+from .operands import DTYPE_CODES, admit, disjoint, extents, on_device, stream_of
 
 EXACT_MAX_AUTO_TOKENS = 0
 MFMA_MAX_TOKENS = 32
@@ -306,7 +306,7 @@ class Q8Embedding:
         codes, scales = r.row_major_planes()
         admit(out, (self._indices.numel(), r.hidden_size), r.dtype, r.device, "out")
         disjoint(out, (codes, scales, self._indices))
-        with torch.cuda.device(r.device):
+        with on_device(r.device):
             r.backend._check(r.backend._native.venturi_q8_embedding_run(
                 codes.data_ptr(), scales.data_ptr(), self._indices.data_ptr(), out.data_ptr(), self._indices.numel(),
                 r.vocab_size, r.hidden_size, r.padded_k, DTYPE_CODES[r.dtype], stream_of(r.device)))
@@ -360,7 +360,7 @@ class Q8OutputHead:
                 raise ValueError("the dense Q8 route needs a 256-byte aligned workspace and 16-byte aligned x and out")
             disjoint(workspace, (x, out) + self.storage_tensors)
             codes, scales = r.row_major_planes()
-            with torch.cuda.device(r.device):
+            with on_device(r.device):
                 r.backend._check(lib.venturi_q8_dense_run(
                     x.data_ptr(), codes.data_ptr(), scales.data_ptr(), out.data_ptr(), self.tokens, r.vocab_size,
                     r.hidden_size, r.padded_k, DTYPE_CODES[r.dtype], workspace.data_ptr(), self.workspace_bytes,
@@ -373,7 +373,7 @@ class Q8OutputHead:
             entry = lib.venturi_q8_tiled_swiglu_run if kernel == "swiglu" else lib.venturi_q8_tiled_run
             planes = self.tiles
             tail = (0, 0) if self.slots is None else (self.slots.data_ptr(), self.slots.numel())
-        with torch.cuda.device(r.device):
+        with on_device(r.device):
             r.backend._check(entry(x.data_ptr(), planes[0].data_ptr(), planes[1].data_ptr(), out.data_ptr(),
                                    self.tokens, r.vocab_size, r.hidden_size, r.padded_k, DTYPE_CODES[r.dtype], *tail,
                                    stream_of(r.device)))
