@@ -260,3 +260,54 @@ def test_mfma_route_exact_group_dots(backend, device, k):
     assert (np.abs(dots) < 2048).all()
     np.testing.assert_array_equal(out.cpu().float().numpy(), dots.astype(np.float32))
     np.testing.assert_array_equal(bits(out), oracle.a8_linear(q, d, codes.numpy(), scales.numpy(), k))
+
+
+# A workgroup per row, staged in LDS (up to 61440 bytes) or read twice (longer or unaligned rows), and a wave per row
+# (up to 512 columns, or 1024 past 1024 rows; unaligned past 4096 rows); more rows than workgroups (65536).
+@pytest.mark.parametrize("dtype,tokens,k,shift", [
+    (torch.float16, 3, 520, 0), (torch.float16, 1025, 1024, 0), (torch.bfloat16, 2, 8200, 0),
+    (torch.float16, 2, 30720, 0), (torch.float16, 2, 30728, 0), (torch.float32, 3, 15360, 0),
+    (torch.float32, 3, 15368, 0), (torch.float16, 5, 4096, 1), (torch.float16, 4097, 2049, 0),
+    (torch.float16, 65539, 1032, 0)])
+def test_rms_forms(backend, device, dtype, tokens, k, shift):
+    print(f"case rms forms {dtype} tokens={tokens} k={k} shift={shift}", flush=True)
+    g = torch.Generator(device=device).manual_seed(k + tokens)
+    x = torch.randn(tokens * k + shift, generator=g, device=device).to(dtype)[shift:].view(tokens, k)
+    w = 1 + 0.03 * torch.randn(k, generator=g, device=device)
+    guard = torch.full((tokens * k + 16,), 47, dtype=dtype, device=device)
+    out = guard[8:-8].view(tokens, k)
+    backend.upload_rmsnorm(w, dtype=dtype, device=device, epsilon=1e-6).prepare(tokens=tokens).run(x, out=out)
+    assert bool((guard[:8] == 47).all()) and bool((guard[-8:] == 47).all())
+    rows = sorted({0, 1, tokens // 2, min(65536, tokens - 1), tokens - 1})
+    code = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}[dtype]
+    given = x[rows].cpu()
+    expected = oracle.rms(given.numpy() if code == 2 else bits(given), w.cpu().numpy(), 1e-6, dtype=code)
+    got = out[rows].cpu()
+    np.testing.assert_array_equal(got.numpy() if code == 2 else bits(got), expected)
+
+
+@pytest.mark.parametrize("tokens,k,shift", [(1, 2048, 0), (256, 2056, 0), (2, 30720, 0), (2, 30728, 0), (3, 4104, 1)])
+@pytest.mark.parametrize("passes", [1, 2])
+def test_rms_a8_few_rows(backend, device, tokens, k, shift, passes):
+    print(f"case rms-a8 few k={k} tokens={tokens} shift={shift} passes={passes}", flush=True)
+    g = torch.Generator().manual_seed(k + tokens)
+    x = torch.randn(tokens, k, generator=g).half()
+    x[tokens - 1, k - 3] = float("inf")
+    w = 1 + 0.03 * torch.randn(k, generator=g)
+    norm = backend.upload_rmsnorm(w, dtype=torch.float16, device=device, epsilon=1e-6)
+    plan = prepare_rms_q8(norm, tokens=tokens, residual_compensation=passes == 2)
+    workspace = torch.zeros(plan.workspace_bytes, dtype=torch.uint8, device=device)
+    inter = torch.empty(tokens, k, dtype=torch.float16, device=device)
+    moved = torch.empty(tokens * k + shift, dtype=torch.float16, device=device)[shift:].view(tokens, k).copy_(x)
+    plan.run(moved, workspace=workspace, intermediate=inter)
+    q, d, y = oracle.rms_a8(bits(x), w.numpy(), 1e-6, passes)
+    finite = slice(0, tokens - 1)
+    np.testing.assert_array_equal(bits(inter)[finite], y[finite])
+    separate = torch.zeros_like(workspace)
+    normed = torch.empty_like(inter)
+    norm.prepare(tokens=tokens).run(moved, out=normed)
+    np.testing.assert_array_equal(bits(normed), bits(inter))
+    backend._check(backend._native.venturi_q8_dp4a_quantize(
+        normed.data_ptr(), separate.data_ptr(), separate.numel(), tokens, k, passes,
+        torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(separate, workspace)

@@ -61,6 +61,24 @@ __global__ __launch_bounds__(256) void a8_quantize(const __half* __restrict__ x,
 // two-level tree; inv = 1/sqrt(sum/k + eps) with IEEE division and square
 // root. (The reference uses rsqrtf, an approximation its tests pin only by
 // tolerance; this library fixes the correctly rounded form.)
+//
+// A decode step's rows are few, so latency is all there is: one workgroup of
+// 256 threads per row, thread c running chain c, with the row read once in
+// 16-byte pieces into LDS (one memory round trip for up to 16384 columns, where
+// a wave per row took one per eight 256-column pieces and the second reading
+// one per column) and both phases reading it there. Rows of other alignments
+// or beyond kStagedRow bytes read global memory in both phases.
+// MI355X, fp16, against a wave per row, us: 8 x 5120 15.5 -> 4.0, 8 x 17408 47
+// -> 7.7, 2048 x 5120 31 -> 9.8, 2048 x 17408 111 -> 30.
+constexpr int kRowThreads = 256;
+constexpr int kStagedRow = 60 * 1024;
+
+// Rows that can be staged: whole 16-byte pieces, within the LDS bound.
+template <class T>
+bool row_staged(const void* x, int k) {
+    return k % 8 == 0 && aligned(x, 16) && static_cast<std::int64_t>(k) * sizeof(T) <= kStagedRow;
+}
+
 // Four consecutive 16-bit values as f32, one 8-byte load (p 8-byte aligned).
 template <class T>
 __device__ __forceinline__ void load4_f32(const T* p, float (&v)[4]) {
@@ -76,6 +94,90 @@ __device__ __forceinline__ void load4_f32(const T* p, float (&v)[4]) {
     }
 }
 
+// Inverse RMS of the row at src (every thread of the workgroup returns it);
+// STAGED leaves the row in `row` (LDS).
+template <class T, bool STAGED, int THREADS = kRowThreads>
+__device__ __forceinline__ float row_inverse_rms(const T* src, T* row, float* chains, int k, float epsilon) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    if constexpr (STAGED) {
+        constexpr int V = 16 / sizeof(T);
+        const int pieces = k / V;
+        for (int base = tid; base < pieces; base += 8 * THREADS) {
+            uint4 v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                v[j] = *reinterpret_cast<const uint4*>(src + V * min(base + j * THREADS, pieces - 1));
+#pragma unroll
+            for (int j = 0; j < 8; ++j)  // pieces past the last are not written
+                if (base + j * THREADS < pieces) *reinterpret_cast<uint4*>(row + V * (base + j * THREADS)) = v[j];
+        }
+        __syncthreads();
+    }
+    const T* from = STAGED ? row : src;
+    if (THREADS == kRowThreads || tid < kRowThreads) {
+        float chain = 0.0f;
+#pragma unroll 8
+        for (int col = tid; col < k; col += kRowThreads) {
+            const float v = to_f32(from[col]);
+            chain = fmaf(v, v, chain);
+        }
+        chains[tid] = chain;
+    }
+    __syncthreads();
+    const float4 c = *reinterpret_cast<const float4*>(chains + 4 * lane);
+    const float sum = __shfl(canonical_sum(c.x, c.y, c.z, c.w), 0, 64);  // every wave folds the chains itself
+    return __fdiv_rn(1.0f, sqrt_rn(__fdiv_rn(sum, static_cast<float>(k)) + epsilon));
+}
+
+// The normalised value is ((x * inv) * gamma) rounded once.
+template <class T, bool STAGED>
+__global__ __launch_bounds__(kRowThreads) void rms_norm(const T* __restrict__ x, const float* __restrict__ w,
+                                                        T* __restrict__ out, int tokens, int k, float epsilon) {
+    extern __shared__ uint4 rms_lds[];
+    __shared__ __attribute__((aligned(16))) float chains[kRowThreads];
+    auto* row = reinterpret_cast<T*>(rms_lds);
+    const int tid = threadIdx.x;
+    for (int token = blockIdx.x; token < tokens; token += gridDim.x) {
+        const T* src = x + static_cast<std::int64_t>(token) * k;
+        T* dst = out + static_cast<std::int64_t>(token) * k;
+        if constexpr (STAGED) {
+            // Gamma of the first two eight-column pieces arrives during the statistics.
+            const int pieces = k / 8;
+            float4 g[2][2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float* at = w + 8 * min(tid + j * kRowThreads, pieces - 1);
+                g[j][0] = *reinterpret_cast<const float4*>(at);
+                g[j][1] = *reinterpret_cast<const float4*>(at + 4);
+            }
+            const float inv = row_inverse_rms<T, true>(src, row, chains, k, epsilon);
+            auto piece = [&](int p, const float4& a, const float4& b) {
+                const float gv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+                T y[8];
+                const T* r = row + 8 * p;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = from_f32<T>((to_f32(r[i]) * inv) * gv[i]);
+                constexpr int U = sizeof(T) / 2;  // 16-byte units
+                uint4 o[U];
+                __builtin_memcpy(o, y, sizeof(o));
+#pragma unroll
+                for (int u = 0; u < U; ++u) reinterpret_cast<uint4*>(dst + 8 * p)[u] = o[u];
+            };
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                if (tid + j * kRowThreads < pieces) piece(tid + j * kRowThreads, g[j][0], g[j][1]);
+            for (int p = tid + 2 * kRowThreads; p < pieces; p += kRowThreads)
+                piece(p, *reinterpret_cast<const float4*>(w + 8 * p), *reinterpret_cast<const float4*>(w + 8 * p + 4));
+        } else {
+            const float inv = row_inverse_rms<T, false>(src, nullptr, chains, k, epsilon);
+#pragma unroll 4
+            for (int col = tid; col < k; col += kRowThreads) dst[col] = from_f32<T>((to_f32(src[col]) * inv) * w[col]);
+        }
+        __syncthreads();  // the next row reuses the LDS
+    }
+}
+
+// Short rows: a wave per row, four chains per lane.
 // Whether a row's four-value pieces can be read as 8-byte words: rows start
 // 8-byte aligned when k % 4 == 0 and the base is.
 template <class T>
@@ -84,7 +186,7 @@ __device__ __forceinline__ bool rows_vec4(const T* base, int k) {
 }
 
 template <class T>
-__device__ __forceinline__ float row_inverse_rms(const T* src, int k, float epsilon, int lane, bool vec) {
+__device__ __forceinline__ float wave_inverse_rms(const T* src, int k, float epsilon, int lane, bool vec) {
     float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     // Unrolled so that several pieces of the row are in flight at once; each
     // chain a[v] still runs over base in ascending order.
@@ -111,14 +213,14 @@ __device__ __forceinline__ float row_inverse_rms(const T* src, int k, float epsi
 
 // One wave per row; the normalised value is ((x * inv) * gamma) rounded once.
 template <class T>
-__global__ __launch_bounds__(256) void rms_norm(const T* __restrict__ x, const float* __restrict__ w,
+__global__ __launch_bounds__(256) void rms_norm_wave(const T* __restrict__ x, const float* __restrict__ w,
                                                 T* __restrict__ out, int tokens, int k, float epsilon) {
     const int lane = threadIdx.x & 63;
     const int token = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (token >= tokens) return;
     const T* src = x + static_cast<std::int64_t>(token) * k;
     T* dst = out + static_cast<std::int64_t>(token) * k;
-    const float inv = row_inverse_rms(src, k, epsilon, lane, rows_vec4(x, k));
+    const float inv = wave_inverse_rms(src, k, epsilon, lane, rows_vec4(x, k));
     for (int col = lane; col < k; col += 64) dst[col] = from_f32<T>((to_f32(src[col]) * inv) * w[col]);
 }
 
@@ -126,7 +228,7 @@ __global__ __launch_bounds__(256) void rms_norm(const T* __restrict__ x, const f
 // passes): the quantizer sees exactly the fp16-rounded normalised values.
 // One 4-wave workgroup per token: thread c runs the reference's chain c
 // (fmaf over columns c, c + 256, ...), wave 0 folds the 256 chains through the
-// same two-level tree as row_inverse_rms (so inv has the same bits), and the
+// same two-level tree as the norm's (so inv has the same bits), and the
 // four waves then quantize every fourth 256-column piece; 8 lanes x 4 values
 // form each group of 32.
 __global__ __launch_bounds__(256) void rms_a8(const __half* __restrict__ x, const float* __restrict__ w,
@@ -196,6 +298,51 @@ __global__ __launch_bounds__(256) void rms_a8(const __half* __restrict__ x, cons
         if (g < groups)
             quantize_group<4, 8>(r, bad, passes, codes + index * 32 + (col & 31), scales + index, count * 32,
                                  count, (lane & 7) == 0);
+    }
+}
+
+// The same for few rows (a decode step): 16 waves per row, so that the serial
+// part, a wave's pieces of 256 columns with their cross-lane maxima, is a
+// quarter as long; the row is staged in LDS and gamma read ahead of the
+// statistics. MI355X, 8 rows of 5120, two passes / one: 7.7 / 6.2 -> 5.0 /
+// 4.5 us; 17408 columns 20.9 / 16.1 -> 9.7 / 7.7.
+__global__ __launch_bounds__(1024) void rms_a8_few(const __half* __restrict__ x, const float* __restrict__ w,
+                                                   std::int8_t* codes, float* scales, __half* intermediate, int tokens,
+                                                   int k, int groups, int passes, float epsilon) {
+    extern __shared__ uint4 rms_lds[];
+    __shared__ __attribute__((aligned(16))) float chains[kRowThreads];
+    auto* row = reinterpret_cast<__half*>(rms_lds);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int token = blockIdx.x;
+    const std::int64_t count = static_cast<std::int64_t>(tokens) * groups;
+    // k % 8 == 0: a lane's four columns are all in or all out.
+    auto gamma = [&](int base) { return *reinterpret_cast<const float4*>(w + min(base + 4 * lane, k - 4)); };
+    float4 next = gamma(256 * wave);
+    const float inv = row_inverse_rms<__half, true, 1024>(x + static_cast<std::int64_t>(token) * k, row, chains, k, epsilon);
+    for (int base = 256 * wave; base < groups * 32; base += 4096) {
+        const int col = base + 4 * lane;
+        const int g = col >> 5;
+        const float wa[4] = {next.x, next.y, next.z, next.w};
+        next = gamma(base + 4096);
+        float xv[4], r[4];
+        load4_f32(row + min(col, k - 4), xv);
+        bool bad = false;
+        unsigned short yb[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const __half y = from_f32<__half>((xv[v] * inv) * wa[v]);
+            yb[v] = __half_as_ushort(y);
+            r[v] = col < k ? __half2float(y) : 0.0f;
+            bad |= !isfinite(r[v]);
+        }
+        if (intermediate && col < k)
+            *reinterpret_cast<uint2*>(intermediate + static_cast<std::int64_t>(token) * k + col) =
+                make_uint2(yb[0] | (static_cast<std::uint32_t>(yb[1]) << 16),
+                           yb[2] | (static_cast<std::uint32_t>(yb[3]) << 16));
+        const std::int64_t index = static_cast<std::int64_t>(token) * groups + min(g, groups - 1);
+        if (g < groups)  // the 8 lanes of a group share g
+            quantize_group<4, 8>(r, bad, passes, codes + index * 32 + (col & 31), scales + index, count * 32, count,
+                                 (lane & 7) == 0);
     }
 }
 
@@ -485,16 +632,28 @@ void rms_launch(const void* x, const float* w, void* out, int tokens, int k, int
                 hipStream_t stream) {
     require(x && w && out && tokens > 0 && k > 0, "invalid RMSNorm operand");
     require(epsilon > 0.0f && std::isfinite(epsilon), "invalid RMSNorm epsilon");
-    const dim3 grid((tokens + 3) / 4);
-    if (dtype == kF16)
-        rms_norm<<<grid, 256, 0, stream>>>(static_cast<const __half*>(x), w, static_cast<__half*>(out), tokens, k, epsilon);
-    else if (dtype == kBF16)
-        rms_norm<<<grid, 256, 0, stream>>>(static_cast<const __hip_bfloat16*>(x), w,
-                                           static_cast<__hip_bfloat16*>(out), tokens, k, epsilon);
-    else if (dtype == kF32)
-        rms_norm<<<grid, 256, 0, stream>>>(static_cast<const float*>(x), w, static_cast<float*>(out), tokens, k, epsilon);
-    else
-        throw Invalid("unsupported scalar type");
+    auto launch = [&](auto type) {
+        using T = decltype(type);
+        const auto* xp = static_cast<const T*>(x);
+        auto* op = static_cast<T*>(out);
+        // Short rows leave most of a workgroup idle; many rows fill the chip with
+        // a wave each (us, wave against workgroup per row: 256 x 512 3.4 / 3.0,
+        // 2048 x 512 3.9 / 4.4, 256 x 1024 4.8 / 3.0, 65536 x 1024 59 / 71, 65536 x
+        // 2048 184 / 108). Rows that cannot be staged are read twice from global
+        // memory: 8 x 5121 21 / 5.5, 2048 x 2048 8.5 / 6.2, 65536 x 1536 138 / 220.
+        const int grid = std::min(tokens, 65536);
+        const bool long_rows = k > 1024 || (k > 512 && tokens <= 1024);
+        if (long_rows && row_staged<T>(x, k) && aligned(w, 16) && aligned(out, 16))
+            rms_norm<T, true><<<grid, kRowThreads, k * sizeof(T), stream>>>(xp, w, op, tokens, k, epsilon);
+        else if (long_rows && tokens <= 4096)
+            rms_norm<T, false><<<grid, kRowThreads, 0, stream>>>(xp, w, op, tokens, k, epsilon);
+        else
+            rms_norm_wave<<<(tokens + 3) / 4, kRowThreads, 0, stream>>>(xp, w, op, tokens, k, epsilon);
+    };
+    if (dtype == kF16) launch(__half{});
+    else if (dtype == kBF16) launch(__hip_bfloat16{});
+    else if (dtype == kF32) launch(float{});
+    else throw Invalid("unsupported scalar type");
 }
 
 void rms_a8_launch(const void* x, const float* w, void* workspace, std::uint64_t available, int tokens, int k,
@@ -511,8 +670,14 @@ void rms_a8_launch(const void* x, const float* w, void* workspace, std::uint64_t
     const std::int64_t count = static_cast<std::int64_t>(tokens) * groups;
     auto* codes = static_cast<std::int8_t*>(workspace);
     auto* scales = reinterpret_cast<float*>(codes + count * 32 * passes);
-    rms_a8<<<tokens, 256, 0, stream>>>(static_cast<const __half*>(x), w, codes, scales,
-                                       static_cast<__half*>(intermediate), tokens, k, groups, passes, epsilon);
+    const auto* xp = static_cast<const __half*>(x);
+    auto* ip = static_cast<__half*>(intermediate);
+    // (Two passes, us, four waves against sixteen: 8 x 1024 3.2 / 3.5, 8 x 2048
+    // 4.3 / 3.7, 256 x 5120 8.3 / 5.7, 1024 x 5120 11.9 / 13.4.)
+    if (tokens <= 256 && k >= 2048 && row_staged<__half>(x, k) && aligned(w, 16) && aligned(intermediate, 8))
+        rms_a8_few<<<tokens, 1024, k * sizeof(__half), stream>>>(xp, w, codes, scales, ip, tokens, k, groups, passes, epsilon);
+    else
+        rms_a8<<<tokens, 256, 0, stream>>>(xp, w, codes, scales, ip, tokens, k, groups, passes, epsilon);
 }
 
 }  // namespace vt
