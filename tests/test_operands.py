@@ -24,6 +24,7 @@ def test_disjoint_is_the_byte_windows_intersection(a, b):
 @pytest.mark.parametrize("shape,dtype", [((2, 3), torch.float32), ((3, 2), torch.float16), ((6,), torch.float16)])
 def test_admit_refuses_other_shapes_and_types(shape, dtype):
     where = torch.device("cpu")
-    admit(torch.zeros(2, 3, dtype=torch.float16), (2, 3), torch.float16, where, "x")
+    for sizes in ((2, 3), [2, 3], torch.Size((2, 3))):
+        admit(torch.zeros(2, 3, dtype=torch.float16), sizes, torch.float16, where, "x")
     with pytest.raises(ValueError, match="x requires shape"):
         admit(torch.zeros(shape, dtype=dtype), (2, 3), torch.float16, where, "x")

@@ -36,7 +36,7 @@ def admit(tensor, shape, dtype, device, name):
     """Checks one operand against the plan's fixed (shape, dtype, device)."""
     if not isinstance(tensor, torch.Tensor):
         raise TypeError(f"{name} must be a tensor")
-    if tensor.shape != shape or tensor.dtype != dtype or tensor.device != device:
+    if tensor.shape != tuple(shape) or tensor.dtype != dtype or tensor.device != device:
         raise ValueError(f"{name} requires shape {shape}, dtype {dtype}, device {device}")
     if not tensor.is_contiguous():
         raise ValueError(f"{name} must be contiguous; no implicit copy")
