@@ -660,7 +660,9 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 // MI355X, 2048 x 768 x 128 experts, top 8, routed call, before -> after, us:
 // one token 43.6 -> 17.3, 4 tokens 52.6 -> 28, 8 tokens 55.5 -> 40, 16 tokens
 // 68 -> 57, 32 tokens 74.5 -> 67. Activations read per lane from L2 instead of
-// LDS needed 32 more registers and spilled.
+// LDS needed 32 more registers and spilled. Error against 64 bits with the fp16
+// boundaries kept, mean of 24 routings, q4_grouped and this: 8 tokens 1.03e-4,
+// 0.89e-4; one token, 64 experts of 1408 x 4096, 1.20e-4, 0.99e-4.
 
 typedef std::uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
