@@ -235,10 +235,10 @@ def test_moe_graph_replays(backend, device, geometry, tokens):
         assert np.array_equal(bits(out), bits(eager)), replay
 
 
-# Few pairs (the form of decode steps). Rows of a pass are min(16, 67584 // (2 * (256-column chunks of K + 8))) and the
-# launch shapes go by the expected active row blocks, so: up to 2048 and 2560 blocks (gate/up, down), up to 9000, more;
-# K below one chunk, odd chunk counts and ragged last chunks; experts with more tokens than a pass holds (hidden 4104:
-# seven rows); one expert; 1024 experts (sixteen per scanning lane); the largest pair count.
+# Few tokens: up to twice the rows of a pass (16, or as many as 67584 bytes of LDS hold), gate/up and down run the form of
+# decode steps, each as its own K allows, with four waves up to 40 KB of rows and eight beyond. K below one chunk, odd
+# chunk counts and ragged last chunks; experts with more pairs than two passes hold (repeated ids); one expert; 1024
+# experts (sixteen per scanning lane); calls past either form's token count.
 @pytest.mark.parametrize(
     "geometry,tokens",
     [
@@ -250,10 +250,15 @@ def test_moe_graph_replays(backend, device, geometry, tokens):
         (MoEGeometry(520, 128, 8, 344), 64),
         (MoEGeometry(776, 48, 8, 1032), 48),
         (MoEGeometry(64, 1024, 16, 8), 32),
+        (MoEGeometry(64, 1024, 16, 8), 33),  # one token past the form (the case above is its largest pair count)
+        (MoEGeometry(520, 2, 2, 344), 32),  # experts with pairs past two passes of 16 rows
+        (MoEGeometry(1544, 16, 4, 1800), 5),  # 14 and 16 half chunks: a whole round of six and a tail
+        (MoEGeometry(4104, 8, 4, 776), 14),  # two passes of seven rows
+        (MoEGeometry(776, 8, 4, 4104), 16),  # down past the form, gate/up in it
     ],
 )
 def test_moe_few_pairs(backend, device, geometry, tokens):
-    run_and_check(backend, device, geometry, tokens, seed=31 + tokens, duplicates=geometry.top_k >= 4)
+    run_and_check(backend, device, geometry, tokens, seed=31 + tokens, duplicates=geometry.top_k >= 4 or geometry.num_experts == 2)
 
 
 def test_moe_few_pairs_without_a_valid_id(backend, device):
@@ -269,3 +274,25 @@ def test_moe_few_pairs_without_a_valid_id(backend, device):
     views = plan.workspace_views(workspace)
     assert int(views["status"][0]) == 6 and not bool(views["seg"].any()) and bool((views["pair_slot"] == -1).all())
     assert bool(torch.isnan(out).all())
+
+
+@pytest.mark.parametrize("geometry", [MoEGeometry(2048, 16, 4, 768), MoEGeometry(520, 8, 2, 1032),
+                                      MoEGeometry(4104, 4, 2, 264), MoEGeometry(136, 40, 8, 72)])
+def test_moe_tokens_have_the_same_bits_in_every_batch(backend, device, geometry):
+    """Each call of the first tokens of a batch gives their rows of the whole batch's call (as the routed-expert loop,
+    whose sums run over K in one order, would)."""
+    print(f"case moe batches E={geometry.num_experts} H={geometry.hidden_size} I={geometry.intermediate_size}", flush=True)
+    bank, _, _ = build(backend, device, geometry, 8)
+    x, ids, scores = (t.to(device) for t in routing(70, geometry, 9))
+
+    def run(tokens):
+        plan = bank.prepare(tokens=tokens)
+        workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=device)
+        out = torch.empty((tokens, geometry.hidden_size), dtype=torch.float16, device=device)
+        plan.run(x[:tokens].contiguous(), ids[:tokens].contiguous(), scores[:tokens].contiguous(), out=out,
+                 workspace=workspace)
+        return bits(out)
+
+    whole = run(70)
+    for tokens in (1, 3, 8, 16, 19, 32, 33):
+        assert np.array_equal(run(tokens), whole[:tokens]), tokens

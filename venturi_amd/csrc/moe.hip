@@ -23,7 +23,6 @@
 #include "common.hpp"
 
 #include <algorithm>
-#include <cmath>
 #include <type_traits>
 
 namespace vt {
@@ -654,33 +653,31 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 //   pair, so the active experts' parts spread over every XCD and the
 //   workgroups without work are the last ones;
 // * a pass's activation rows (up to 16, whole K) are staged in LDS once; the
-//   waves then run without a barrier, WK of them sharing a row block's K (their
-//   sums meet in LDS, in wave order) and each streaming half chunks (1 KB per
-//   row block) of RB row blocks two ahead.
-// MI355X, 2048 x 768 x 128 experts, top 8, routed call, before -> after, us:
-// one token 43.6 -> 17.3, 4 tokens 52.6 -> 28, 8 tokens 55.5 -> 40, 16 tokens
-// 68 -> 57, 32 tokens 74.5 -> 67. Activations read per lane from L2 instead of
-// LDS needed 32 more registers and spilled. Error against 64 bits with the fp16
-// boundaries kept, mean of 24 routings, q4_grouped and this: 8 tokens 1.03e-4,
-// 0.89e-4; one token, 64 experts of 1408 x 4096, 1.20e-4, 0.99e-4.
+//   waves of a workgroup then run without a barrier, each streaming the half
+//   chunks (1 KB) of one row block, six of them in flight.
+// A row block's K stays in one wave, in q4_grouped's order: a token's outputs
+// have the same bits in every batch, whichever form a call of its size takes.
+// (K split over waves, summed in LDS, gave other bits than larger batches: rel
+// 1.2e-4 after the contract's fp16 roundings.)
+// MI355X, 128 experts of 768 x 2048, top 8, routed call, q4_grouped -> this, us
+// (eight routings in turn): one token 39 -> 18, 4 tokens 52 -> 27, 8 tokens 55 ->
+// 40, 16 tokens 67 -> 59; 64 experts of 1408 x 4096, top 4: 55 -> 21, 82 -> 37,
+// 97 -> 57, 109 -> 86.
+// Two waves, two row blocks per wave and 2, 4 or 8 half chunks in flight
+// measured 1-20% slower on average over six geometries at 1-16 tokens.
 
 typedef std::uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kFewPairs = 512;      // pairs at most: one per thread routes them
+constexpr int kFewRows = 16;        // one MFMA's activation rows
+constexpr int kFewPairs = 512;      // pairs at most: the routing lists
 constexpr int kFewLds = 66 * 1024;  // activation rows of a pass: two workgroups share a CU
+constexpr int kFewItems = 6;        // half chunks of a row block in flight
 
-template <int RB>
-struct FewItem {  // half of a chunk for a wave's row blocks: codes and group scales
-    u32x4 w[RB];
-    unsigned short s[RB];
-};
-
-template <int EPI, int WK, int RB, bool ROUTE>
-__global__ __launch_bounds__(512, 4) void q4_few(Q4Tiled p, int parts, int blocks, int rows) {
-    constexpr int W = 8, WR = W / WK;
-    extern __shared__ uint4 few_lds[];  // activation rows of a pass, then the waves' partial tiles
+template <int EPI, int W, bool ROUTE>
+__global__ __launch_bounds__(W * 64, 4) void q4_few(Q4Tiled p, int parts, int blocks, int rows) {
+    constexpr int T = W * 64, D = kFewItems;
+    extern __shared__ uint4 few_lds[];  // activation rows of a pass
     auto* xl = reinterpret_cast<_Float16*>(few_lds);
-    auto* partial = reinterpret_cast<float4v*>(few_lds);
     __shared__ int count[ROUTE ? kMaxExperts : 1];
     __shared__ int invalid;
     __shared__ unsigned short elist[ROUTE ? kFewPairs : 1];
@@ -689,18 +686,17 @@ __global__ __launch_bounds__(512, 4) void q4_few(Q4Tiled p, int parts, int block
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = lane >> 4, m = lane & 15;
-    const int wk = wave / WR, wr = wave % WR;
     const int active = blockIdx.x / parts, part = blockIdx.x % parts;
 
     // Pairs per expert, then the active-th expert that has any.
     if constexpr (ROUTE) {
-        const std::int64_t e = p.ids[min(tid, p.pairs - 1)];
-        for (int i = tid; i < p.experts; i += 512) count[i] = 0;
+        for (int i = tid; i < p.experts; i += T) count[i] = 0;
         if (tid == 0) invalid = 0;
         __syncthreads();
-        if (tid < p.pairs) {
+        for (int i = tid; i < p.pairs; i += T) {
+            const std::int64_t e = p.ids[i];
             const bool ok = e >= 0 && e < p.experts;
-            elist[tid] = ok ? static_cast<unsigned short>(e) : 0xFFFFu;
+            elist[i] = ok ? static_cast<unsigned short>(e) : 0xFFFFu;
             atomicAdd(ok ? &count[e] : &invalid, 1);
         }
         __syncthreads();
@@ -770,16 +766,9 @@ __global__ __launch_bounds__(512, 4) void q4_few(Q4Tiled p, int parts, int block
     const BiasedMasks masks = biased_masks();
     const char* wbase = reinterpret_cast<const char*>(p.codes + expert * p.code_stride);
     const char* sbase = reinterpret_cast<const char*>(p.scales + expert * p.scale_stride);
-    const int block0 = part * WR * RB;
-    std::int64_t unit[RB];
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-        const int b = min(block0 + wr * RB + r, blocks - 1);
-        unit[r] = static_cast<std::int64_t>(b >> 3) * p.chunks * 8 + (b & 7);
-    }
+    const int block = part * W + wave, from = min(block, blocks - 1);
+    const std::int64_t unit = static_cast<std::int64_t>(from >> 3) * p.chunks * 8 + (from & 7);
     const int items = 2 * p.chunks;
-    const int i0 = items * wk / WK, i1 = items * (wk + 1) / WK;
-
     const int stride = p.chunks * kChunk + 8;
     for (int pass = 0; pass < total; pass += rows) {
         const int live = min(rows, total - pass);
@@ -796,7 +785,7 @@ __global__ __launch_bounds__(512, 4) void q4_few(Q4Tiled p, int parts, int block
         auto load_x = [&](int base) {
 #pragma unroll
             for (int j = 0; j < XU; ++j) {
-                const int u = base + 16 * j + 2 * wave + (lane >> 5);
+                const int u = base + 2 * W * j + 2 * wave + (lane >> 5);
                 const int t = min(u, units - 1) / p.chunks, c = min(u, units - 1) - t * p.chunks;
                 const int row = ROUTE ? plist[pass + t] / p.top_k : begin + pass + t;
                 const int col = c * kChunk + 8 * (lane & 31);
@@ -816,96 +805,76 @@ __global__ __launch_bounds__(512, 4) void q4_few(Q4Tiled p, int parts, int block
                 if (xat[j] >= 0) *reinterpret_cast<u32x4*>(xl + xat[j]) = v;
             }
         };
-        auto load = [&](int i, FewItem<RB>& t) {
-            const int c = i >> 1, h = i & 1;
+        struct Item {  // half of a chunk: 16 code bytes and the group scale
+            u32x4 w;
+            unsigned short s;
+        };
+        auto load = [&](int i, Item& t) {
+            const std::int64_t u = unit + static_cast<std::int64_t>(i >> 1) * 8;
             std::uint32_t at = 16 * lane, sat = 2 * lane;
             asm volatile("" : "+v"(at), "+v"(sat));
-#pragma unroll
-            for (int r = 0; r < RB; ++r) {
-                const std::int64_t u = unit[r] + static_cast<std::int64_t>(c) * 8;
-                t.w[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wbase + u * 2048 + 1024 * h + at));
-                t.s[r] = __builtin_nontemporal_load(reinterpret_cast<const unsigned short*>(sbase + u * 128 + sat));
-            }
+            t.w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wbase + u * 2048 + 1024 * (i & 1) + at));
+            t.s = __builtin_nontemporal_load(reinterpret_cast<const unsigned short*>(sbase + u * 128 + sat));
         };
-        float4v acc[RB];
-#pragma unroll
-        for (int r = 0; r < RB; ++r) acc[r] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
         const _Float16* xf0 = xl + min(m, live - 1) * stride + 64 * q;
-        auto compute = [&](int i, FewItem<RB>& t) {
+        auto compute = [&](int i, const Item& t) {
             const _Float16* xi = xf0 + (i >> 1) * kChunk + 32 * (i & 1);
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const half8 xf = *reinterpret_cast<const half8*>(xi + 8 * s);
-#pragma unroll
-                for (int r = 0; r < RB; ++r) {
-                    std::uint32_t word = t.w[r][s], scale = t.s[r];
-                    asm volatile("" : "+v"(word), "+v"(scale));
-                    const half2v s2 = __builtin_bit_cast(half2v, scale * 0x10001u);
-                    acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf, dequant8_biased(word, s2, masks), acc[r], 0, 0, 0);
-                }
+                std::uint32_t word = t.w[s], scale = t.s;
+                asm volatile("" : "+v"(word), "+v"(scale));
+                const half2v s2 = __builtin_bit_cast(half2v, scale * 0x10001u);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf, dequant8_biased(word, s2, masks), acc, 0, 0, 0);
             }
         };
-        FewItem<RB> b0, b1;
+        Item b[D];
         load_x(0);
-        load(min(i0, items - 1), b0);
-        load(min(i0 + 1, items - 1), b1);
+#pragma unroll
+        for (int j = 0; j < D; ++j) load(min(j, items - 1), b[j]);
         store_x();
-        for (int base = 16 * XU; base < units; base += 16 * XU) {
+        for (int base = 2 * W * XU; base < units; base += 2 * W * XU) {
             load_x(base);
             store_x();
         }
         __syncthreads();
-        if (i0 < i1) {
-            int i = i0;
-            for (; i + 3 < i1; i += 2) {
-                compute(i, b0);
-                load(i + 2, b0);
-                compute(i + 1, b1);
-                load(i + 3, b1);
-            }
-            compute(i, b0);
-            if (i + 1 < i1) {
-                if (i + 2 < i1) load(i + 2, b0);
-                compute(i + 1, b1);
-                if (i + 2 < i1) compute(i + 2, b0);
+        int i = 0;
+        for (; i + 2 * D <= items; i += D) {
+#pragma unroll
+            for (int j = 0; j < D; ++j) {
+                compute(i + j, b[j]);
+                load(i + j + D, b[j]);
             }
         }
+#pragma unroll
+        for (int j = 0; j < D; ++j) {  // the last D .. 2 D - 1 items
+            if (i + j < items) compute(i + j, b[j]);
+            if (i + j + D < items) load(i + j + D, b[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < D; ++j)
+            if (i + j + D < items) compute(i + j + D, b[j]);
 
-        auto store = [&](float4v y, int blk) {
-            if (blk >= blocks) return;
+        if (block < blocks) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int t = 4 * q + i;
                 __half* o = p.out + static_cast<std::int64_t>(begin + pass + t) * p.out_stride;
                 if (EPI == kSwiGLU) {
-                    const float other = __shfl_xor(y[i], 8, 64);  // lane m^8 holds the paired up row
-                    const int col = (blk >> 3) * (kRows / 2) + 8 * (blk & 7) + m;
+                    const float other = __shfl_xor(acc[i], 8, 64);  // lane m^8 holds the paired up row
+                    const int col = (block >> 3) * (kRows / 2) + 8 * (block & 7) + m;
                     if (m < 8 && t < live && col < p.half_rows) {
-                        const float g = __half2float(from_f32<__half>(y[i]));
+                        const float g = __half2float(from_f32<__half>(acc[i]));
                         const float u = __half2float(from_f32<__half>(other));
                         const float a = __half2float(from_f32<__half>(silu(g)));
                         o[col] = from_f32<__half>(__fmul_rn(a, u));
                     }
                 } else {
-                    const int col = 16 * blk + m;
+                    const int col = 16 * block + m;
                     if (t < live && col < p.n)
-                        o[col] = from_f32<__half>(__fmul_rn(__half2float(from_f32<__half>(y[i])), score[i]));
+                        o[col] = from_f32<__half>(__fmul_rn(__half2float(from_f32<__half>(acc[i])), score[i]));
                 }
-            }
-        };
-        if constexpr (WK == 1) {
-#pragma unroll
-            for (int r = 0; r < RB; ++r) store(acc[r], block0 + wr * RB + r);
-        } else {
-            __syncthreads();  // the activations have been read
-#pragma unroll
-            for (int r = 0; r < RB; ++r) partial[(wave * RB + r) * 64 + lane] = acc[r];
-            __syncthreads();
-            for (int b = wave; b < WR * RB; b += W) {
-                float4v y = partial[b * 64 + lane];  // K part 0: waves 0 .. WR - 1
-#pragma unroll
-                for (int w = 1; w < WK; ++w) y += partial[(w * WR * RB + b) * 64 + lane];
-                store(y, block0 + b);
             }
         }
         __syncthreads();  // the next pass restages the LDS
@@ -1104,21 +1073,8 @@ void launch_q4_grouped(const Q4Tiled& p, hipStream_t stream) {
 }
 
 // Activation rows that a pass of q4_few stages.
-int few_rows(const Q4Tiled& p) { return std::min(16, kFewLds / (2 * (p.chunks * kChunk + 8))); }
-
-template <int EPI, int WK, int RB, bool ROUTE>
-void launch_q4_few(const Q4Tiled& p, int active, hipStream_t stream) {
-    const int blocks = p.row_tiles * 8;
-    constexpr int kCover = 8 / WK * RB;
-    const int parts = (blocks + kCover - 1) / kCover;
-    const int rows = few_rows(p);
-    const int lds = std::max(rows * 2 * (p.chunks * kChunk + 8), WK > 1 ? 8 * RB * 1024 : 0);
-    if (lds > 48 * 1024) {
-        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(q4_few<EPI, WK, RB, ROUTE>),
-                                                             hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds);
-        check(raised);
-    }
-    q4_few<EPI, WK, RB, ROUTE><<<active * parts, 512, lds, stream>>>(p, parts, blocks, rows);
+int few_rows(const Q4Tiled& p, int tokens) {
+    return std::min(std::min(tokens, kFewRows), kFewLds / (2 * (p.chunks * kChunk + 8)));
 }
 
 // Whether q4_few is the faster form: one pass per expert in nearly every case
@@ -1127,34 +1083,29 @@ void launch_q4_few(const Q4Tiled& p, int active, hipStream_t stream) {
 // 70 (2048 columns, 16 rows a pass), 8 per expert 131 -> 156 (4096 columns, 8
 // rows); down at 8 per expert 131 -> 123, at 16 per expert 154 -> 161.
 bool few_pairs(const Q4Tiled& p, int tokens, int pairs) {
-    const int rows = few_rows(p);
+    const int rows = few_rows(p, kFewRows);
     return pairs <= kFewPairs && rows > 0 && (tokens <= rows || 2 * pairs <= p.experts * rows);
 }
 
-// Row blocks of the experts that `pairs` uniformly routed pairs touch.
-double active_blocks(const Q4Tiled& p, int pairs) {
-    return p.experts * (1.0 - std::pow(1.0 - 1.0 / p.experts, pairs)) * p.row_tiles * 8;
+template <int EPI, int W, bool ROUTE>
+void launch_q4_few(const Q4Tiled& p, int tokens, int pairs, int lds, hipStream_t stream) {
+    const int blocks = p.row_tiles * 8, parts = (blocks + W - 1) / W;
+    if (lds > 48 * 1024) {
+        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(q4_few<EPI, W, ROUTE>),
+                                                             hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds);
+        check(raised);
+    }
+    q4_few<EPI, W, ROUTE><<<std::min(pairs, p.experts) * parts, W * 64, lds, stream>>>(p, parts, blocks, few_rows(p, tokens));
 }
 
-// Shapes by the row blocks that the launch streams: K shared by several waves
-// and few row blocks per workgroup while there are too few blocks to give
-// every CU two workgroups, longer runs of K per wave beyond, where each
-// workgroup's start (routing, staging) counts. Gate/up (K 1024-4096), us, as
-// (WK, RB): 768 blocks (4,2) 27, (2,2) 29, (1,2) 34; 4500 blocks 71, 68, 72;
-// 10700 blocks 81, 70, 65. Down (K 256-1536): 1024 blocks (2,1) 35, (1,2) 36;
-// 512 blocks 38, 42; 3600 blocks 45, 42; 8000 blocks 80, 65.
-void gate_up_few(const Q4Tiled& p, int pairs, hipStream_t stream) {
-    const int active = std::min(pairs, p.experts);
-    const double blocks = active_blocks(p, pairs);
-    if (blocks <= 2048) launch_q4_few<kSwiGLU, 4, 2, true>(p, active, stream);
-    else if (blocks <= 9000) launch_q4_few<kSwiGLU, 2, 2, true>(p, active, stream);
-    else launch_q4_few<kSwiGLU, 1, 2, true>(p, active, stream);
-}
-
-void down_few(const Q4Tiled& p, int pairs, hipStream_t stream) {
-    const int active = std::min(pairs, p.experts);
-    if (active_blocks(p, pairs) <= 2560) launch_q4_few<kScore, 2, 1, false>(p, active, stream);
-    else launch_q4_few<kScore, 1, 2, false>(p, active, stream);
+// Four waves where the activations leave a CU at least four workgroups, eight
+// where they leave fewer (gate/up of 768 x 2048, four / eight waves, us saved
+// against q4_grouped: 8 tokens 10 / 8, 12 tokens 6 / 10, 16 tokens 6 / 13).
+template <int EPI, bool ROUTE>
+void few_dispatch(const Q4Tiled& p, int tokens, int pairs, hipStream_t stream) {
+    const int lds = few_rows(p, tokens) * 2 * (p.chunks * kChunk + 8);
+    if (lds <= 40 * 1024) launch_q4_few<EPI, 4, ROUTE>(p, tokens, pairs, lds, stream);
+    else launch_q4_few<EPI, 8, ROUTE>(p, tokens, pairs, lds, stream);
 }
 
 std::uint64_t align256(std::uint64_t v) { return (v + 255) / 256 * 256; }
@@ -1841,7 +1792,7 @@ void moe_q4_launch_cfg(const void* x, const std::int64_t* ids, const void* score
     gu.slot_score = slot_score;
     gu.pairs = pairs;
     gu.top_k = top_k;
-    if (few_pairs(gu, tokens, pairs)) gate_up_few(gu, pairs, stream);
+    if (few_pairs(gu, tokens, pairs)) few_dispatch<kSwiGLU, true>(gu, tokens, pairs, stream);
     else if (route_inside) launch_q4_grouped<kSwiGLU, GW, GRB, NBMAX, true, 1>(gu, stream);
     else launch_q4_grouped<kSwiGLU, GW, GRB, NBMAX, false, 1>(gu, stream);
 
@@ -1861,7 +1812,7 @@ void moe_q4_launch_cfg(const void* x, const std::int64_t* ids, const void* score
     dn.x_stride = inter;
     dn.out_stride = hidden;
     dn.experts = experts;
-    if (few_pairs(dn, tokens, pairs)) down_few(dn, pairs, stream);
+    if (few_pairs(dn, tokens, pairs)) few_dispatch<kScore, false>(dn, tokens, pairs, stream);
     else launch_q4_grouped<kScore, DW, DRB, NBMAX, false, 2>(dn, stream);
 
     combine_dispatch(top_k, ids, pair_slot, v, static_cast<__half*>(out), tokens, hidden, stream);
