@@ -1,0 +1,48 @@
+"""Kernel and launch shape of calls, recorded without a GPU (launches.py)."""
+
+import pytest
+
+from launches import LdsLimit, Launch, a8_gemm, a8_tiled, moe, padded, pointers, q4_gemm, q8_prefill, record
+
+DEFAULT_LDS = 64 * 1024
+
+
+def q8(entry, tokens, n, k, dtype, slots=False):
+    x, codes, scales, out, workspace = pointers(5)
+    return entry, [x, codes, scales, out, tokens, n, k, padded(k), dtype, *((workspace, 1 << 30) if slots else ()), None]
+
+
+# Calls whose kernels need more LDS than a launch may have by default: the prefill GEMMs' forms, the decode forms that
+# stage long activations, the canonical-order route and the few-token MoE.
+CALLS = {
+    "q8 prefill, cooperative": q8_prefill(2048, 34816, 5120),
+    "q8 prefill, split": q8_prefill(200, 4096, 5120),
+    "q8 prefill, long rows": q8_prefill(64, 128, (1 << 22) + 8),
+    "a8 prefill, cooperative": a8_gemm(2048, 34816, 5120, 1),
+    "a8 prefill, split": a8_gemm(200, 4096, 5120, 2),
+    "a8 decode, staged": a8_tiled(16, 4096, 5120, 2),
+    "q4 prefill, cooperative": q4_gemm(512, 7168, 5120),
+    "q4 prefill, split": q4_gemm(64, 7168, 5120),
+    "q4 prefill, wide": q4_gemm(2048, 34816, 5120),
+    "q8 decode": q8("venturi_q8_tiled_run", 1, 4096, 40960, 0, slots=True),
+    "q8 exact": q8("venturi_q8_head_run", 2, 7168, 17408, 0),
+    "q8 exact, slab": q8("venturi_q8_head_run", 64, 7168, 17408, 1),
+    "moe, few tokens": moe(16, 2048, 128, 8, 768),
+}
+
+
+@pytest.mark.parametrize("name", CALLS)
+def test_lds_limit_is_raised_on_every_device(name):
+    """A process that drives two devices: the attribute belongs to a device, so each kernel's limit is raised on the
+    one that it is launched on, before the launch."""
+    entry, args = CALLS[name]
+    limits, large = {}, 0
+    for events in record([(device, entry, args) for device in (0, 1, 0, 70)]):
+        for e in events:
+            if isinstance(e, LdsLimit):
+                limits[e.kernel, e.device] = e.bytes
+            elif e.shared > DEFAULT_LDS:
+                large += 1
+                assert limits.get((e.kernel, e.device), 0) >= e.shared, e
+        assert any(isinstance(e, Launch) for e in events)
+    assert large, "the call no longer needs the limit raised"

@@ -591,9 +591,8 @@ void dispatch_a8_lds(const A8Shape& sh, const __half* x, const std::int8_t* acod
         using T = decltype(tag);
         auto* kernel = a8_tiled_lds<T::waves, T::rb, P, T::nbuf, STAGE, T::ks>;
         if (lds > 64 * 1024) {
-            static const hipError_t raised = hipFuncSetAttribute(
-                reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            check(raised);
+            static LdsLimit limit;
+            limit.raise(kernel, 160 * 1024);
         }
         kernel<<<(blocks + T::rb - 1) / T::rb * T::ks, T::waves * 64, lds, stream>>>(
             x, acodes, ascales, wcodes, wscales, codes, scales, out, slots, tokens, n, k, groups, chunks, blocks);

@@ -503,7 +503,7 @@ struct A8TiledGeom {
     static constexpr int kPitch = kTN + 4;
     static constexpr int kOut = WK * kTM * kPitch * 4;
     static constexpr int kLds = WK * kWave > kOut ? WK * kWave : kOut;
-    static_assert(kTM <= 64 && kLds <= 160 * 1024, "tiled split tile exceeds LDS");
+    static_assert(kTM <= 64 && kLds <= 64 * 1024, "tiled split tile exceeds the default LDS limit");
 };
 
 template <int TJ>
@@ -679,8 +679,8 @@ void launch_coop(const A8Operands& o, hipStream_t stream) {
     using G = A8Geom<WT, WN, WK, TI, TJ>;
     const auto kernel = a8_prefill<WT, WN, WK, TI, TJ, Off>;
     const TileOrder order = tile_order(o.tokens, G::kTM, o.n, G::kTN);
-    static const bool raised = (raise_lds(kernel, G::kLds), true);
-    static_cast<void>(raised);
+    static LdsLimit limit;
+    limit.raise(kernel, G::kLds);
     kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(o.acodes, o.ascales, o.codes, o.scales, o.out, o.tokens,
                                                                o.n, o.padded, o.groups, o.passes, order);
 }
@@ -690,8 +690,8 @@ void launch_split(const A8Operands& o, hipStream_t stream) {
     using G = A8SplitGeom<WK, TI, TJ>;
     const auto kernel = a8_prefill_split<WK, TI, TJ>;
     const TileOrder order = tile_order(o.tokens, G::kTM, o.n, G::kTN);
-    static const bool raised = (raise_lds(kernel, G::kLds), true);
-    static_cast<void>(raised);
+    static LdsLimit limit;
+    limit.raise(kernel, G::kLds);
     kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(o.acodes, o.ascales, o.codes, o.scales, o.out, o.tokens,
                                                                o.n, o.padded, o.groups, o.passes, order);
 }
@@ -740,11 +740,8 @@ template <int WK, int TI, int TJ>
 void launch_tiled_split(const std::int8_t* acodes, const float* ascales, const u32x4* codes, const u32x4* scales,
                         __half* out, int tokens, int n, int padded, int groups, int passes, hipStream_t stream) {
     using G = A8TiledGeom<WK, TI, TJ>;
-    const auto kernel = a8_tiled_split<WK, TI, TJ>;
-    static const bool raised = (raise_lds(kernel, G::kLds), true);
-    static_cast<void>(raised);
-    kernel<<<(n + G::kTN - 1) / G::kTN, G::kThreads, G::kLds, stream>>>(acodes, ascales, codes, scales, out, tokens, n,
-                                                                       padded, groups, passes);
+    a8_tiled_split<WK, TI, TJ><<<(n + G::kTN - 1) / G::kTN, G::kThreads, G::kLds, stream>>>(
+        acodes, ascales, codes, scales, out, tokens, n, padded, groups, passes);
 }
 
 // Operands are admitted by the caller (a8_tiled_launch); at most 32 tokens.

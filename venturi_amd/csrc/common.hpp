@@ -12,6 +12,7 @@
 #include <hip/hip_bf16.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
@@ -187,6 +188,29 @@ __device__ __forceinline__ float warp32_sum(float v) {
     v += row_shl<1>(v);
     return v;
 }
+
+// A kernel's raised dynamic-LDS limit (a launch may have 64 KB by default). The
+// attribute belongs to a device, so it is set once on each device that the
+// kernel is launched on; devices past the 64 of the mask set it every time.
+// Declared static beside the launch; one per kernel.
+class LdsLimit {
+   public:
+    void raise(const void* kernel, int bytes) {
+        int device = 0;
+        check(hipGetDevice(&device));
+        const std::uint64_t bit = device < 64 ? std::uint64_t{1} << device : 0;
+        if (raised_.load(std::memory_order_acquire) & bit) return;
+        check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+        raised_.fetch_or(bit, std::memory_order_release);
+    }
+    template <class... Args>
+    void raise(void (*kernel)(Args...), int bytes) {
+        raise(reinterpret_cast<const void*>(kernel), bytes);
+    }
+
+   private:
+    std::atomic<std::uint64_t> raised_{0};
+};
 
 // Compute units of the current device (read once).
 inline int device_cus() {

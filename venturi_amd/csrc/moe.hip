@@ -1091,9 +1091,8 @@ template <int EPI, int W, bool ROUTE>
 void launch_q4_few(const Q4Tiled& p, int tokens, int pairs, int lds, hipStream_t stream) {
     const int blocks = p.row_tiles * 8, parts = (blocks + W - 1) / W;
     if (lds > 48 * 1024) {
-        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(q4_few<EPI, W, ROUTE>),
-                                                             hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds);
-        check(raised);
+        static LdsLimit limit;
+        limit.raise(q4_few<EPI, W, ROUTE>, kFewLds);
     }
     q4_few<EPI, W, ROUTE><<<std::min(pairs, p.experts) * parts, W * 64, lds, stream>>>(p, parts, blocks, few_rows(p, tokens));
 }
@@ -1306,10 +1305,8 @@ void launch_row_prefill(const __half* x, const std::uint8_t* codes, const std::u
     const dim3 grid((n + G::kTN - 1) / G::kTN, (tokens + G::kTM - 1) / G::kTM);
     require(grid.y <= 65535, "token tiles exceed the launch grid");
     if constexpr (G::kLds > 64 * 1024) {
-        static const hipError_t raised = hipFuncSetAttribute(
-            reinterpret_cast<const void*>(row_prefill<HB, WM, WN, TI, TJ, PF, GS>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(G::kLds));
-        check(raised);
+        static LdsLimit limit;
+        limit.raise(row_prefill<HB, WM, WN, TI, TJ, PF, GS>, static_cast<int>(G::kLds));
     }
     row_prefill<HB, WM, WN, TI, TJ, PF, GS><<<grid, G::kThreads, G::kLds, stream>>>(x, codes, high, scales, out,
                                                                                    tokens, n, k, padded);

@@ -107,12 +107,6 @@ __device__ __forceinline__ std::uint64_t lane_offset(std::uint64_t& off) { retur
 // 256 rows of fp16) below 2^32.
 constexpr int kNarrowK = 1 << 22;
 
-// Raises a kernel's dynamic LDS limit once per instantiation.
-template <class Kernel>
-inline void raise_lds(Kernel kernel, int bytes) {
-    check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-}
-
 __device__ __forceinline__ std::uint32_t pack_half2(float a, float b) {
     return static_cast<std::uint32_t>(__half_as_ushort(from_f32<__half>(a))) |
            static_cast<std::uint32_t>(__half_as_ushort(from_f32<__half>(b))) << 16;

@@ -558,17 +558,8 @@ void launch_tile(const void* x, const std::int8_t* codes, const __half* scales, 
         reinterpret_cast<const void*>(q8_exact<T, TT, RR, U, false, true>),
     };
     if (lds > 64 * 1024) {
-        // Raise the dynamic-LDS limit of every variant once per process.
-        static const hipError_t raised = [&kernels] {
-            hipError_t status = hipSuccess;
-            for (const void* f : kernels) {
-                const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                         static_cast<int>(kMaxLds));
-                if (status == hipSuccess) status = e;
-            }
-            return status;
-        }();
-        check(raised);
+        static LdsLimit limits[4];
+        for (int i = 0; i < 4; ++i) limits[i].raise(kernels[i], static_cast<int>(kMaxLds));
     }
     const T* xp = static_cast<const T*>(x);
     T* op = static_cast<T*>(out);
@@ -600,10 +591,12 @@ void launch_slab(const void* x, const std::int8_t* codes, const __half* scales, 
         GENERAL ? reinterpret_cast<const void*>(q8_exact_slab<T, TT, RR, S, W, B, true, GENERAL>) : nullptr,
         GENERAL ? reinterpret_cast<const void*>(q8_exact_slab<T, TT, RR, S, W, B, !GENERAL, GENERAL>) : nullptr,
     };
+    if (G::kLds > 64 * 1024) {
+        static LdsLimit limits[4];
+        for (int i = 0; i < 4; ++i)
+            if (kernels[i]) limits[i].raise(kernels[i], static_cast<int>(G::kLds));
+    }
     static const int capacity = [&kernels] {
-        if (G::kLds > 64 * 1024)
-            for (const void* f : kernels)
-                if (f) check(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(G::kLds)));
         int device = 0, cus = 0, per = 0;
         check(hipGetDevice(&device));
         check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));

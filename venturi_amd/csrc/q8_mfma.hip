@@ -590,10 +590,8 @@ void launch_tiled_lds(const __half* x, const uint4* codes, const std::uint32_t* 
     const std::size_t lds = std::max(lds_x_bytes(tokens, kper), static_cast<std::size_t>(W) * RB * 1024);
     require(lds <= 160 * 1024, "staged activations exceed LDS");
     require(KS == 1 || slots, "a split projection needs its slot buffer");
-    static const hipError_t raised =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(q8_tiled_lds<W, RB, STEPS, TMAX, KS, SWIGLU>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    check(raised);
+    static LdsLimit limit;
+    limit.raise(q8_tiled_lds<W, RB, STEPS, TMAX, KS, SWIGLU>, 160 * 1024);
     q8_tiled_lds<W, RB, STEPS, TMAX, KS, SWIGLU><<<(blocks + RB - 1) / RB * KS, W * 64, lds, stream>>>(
         x, codes, scales, out, slots, tokens, n, k, chunks, blocks);
 }

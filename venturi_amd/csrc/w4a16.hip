@@ -462,8 +462,8 @@ void launch_coop(const Q4Operands& o, hipStream_t stream) {
     using G = Q4Geom<WT, WN, WK, TI, TJ>;
     const auto kernel = q4_prefill<WT, WN, WK, TI, TJ>;
     const TileOrder order = tile_order(o.tokens, G::kTM, o.n, G::kTN);
-    static const bool raised = (raise_lds(kernel, G::kLds), true);
-    static_cast<void>(raised);
+    static LdsLimit limit;
+    limit.raise(kernel, G::kLds);
     kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(o.x, o.codes, o.scales, o.out, o.tokens, o.n, o.k,
                                                                o.padded, order);
 }
@@ -473,8 +473,8 @@ void launch_split(const Q4Operands& o, hipStream_t stream) {
     using G = Q4SplitGeom<WK, TI, TJ>;
     const auto kernel = q4_prefill_split<WK, TI, TJ>;
     const TileOrder order = tile_order(o.tokens, G::kTM, o.n, G::kTN);
-    static const bool raised = (raise_lds(kernel, G::kLds), true);
-    static_cast<void>(raised);
+    static LdsLimit limit;
+    limit.raise(kernel, G::kLds);
     kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(o.x, o.codes, o.scales, o.out, o.tokens, o.n, o.k,
                                                                o.padded, order);
 }

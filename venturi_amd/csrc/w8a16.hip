@@ -309,8 +309,8 @@ void launch_prefill(const __half* x, const std::int8_t* codes, const __half* sca
     using G = PrefillGeom<WT, WN, WK, TI, TJ>;
     const auto kernel = q8_prefill<WT, WN, WK, TI, TJ, PF, Off>;
     const TileOrder order = tile_order(tokens, G::kTM, n, G::kTN);
-    static const bool raised = (raise_lds(kernel, G::kLds), true);
-    static_cast<void>(raised);
+    static LdsLimit limit;
+    limit.raise(kernel, G::kLds);
     kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(x, codes, scales, out, tokens, n, k, padded,
                                                                (k + 31) / 32, order);
 }
@@ -522,8 +522,8 @@ void launch_split(const __half* x, const std::int8_t* codes, const __half* scale
     using G = SplitGeom<WK, TI, TJ>;
     const auto kernel = q8_prefill_split<WK, TI, TJ>;
     const TileOrder order = tile_order(tokens, G::kTM, n, G::kTN);
-    static const bool raised = (raise_lds(kernel, G::kLds), true);
-    static_cast<void>(raised);
+    static LdsLimit limit;
+    limit.raise(kernel, G::kLds);
     kernel<<<8 * order.per_xcd, G::kThreads, G::kLds, stream>>>(x, codes, scales, out, tokens, n, k, padded,
                                                                (k + 31) / 32, order);
 }
