@@ -46,3 +46,20 @@ def test_lds_limit_is_raised_on_every_device(name):
                 assert limits.get((e.kernel, e.device), 0) >= e.shared, e
         assert any(isinstance(e, Launch) for e in events)
     assert large, "the call no longer needs the limit raised"
+
+
+def rows_of_a_pass(k):
+    """Activation rows that the few-token MoE form stages: 67584 bytes of rows of whole 256-column chunks and 8 halves."""
+    return min(16, 67584 // (2 * ((padded(k) + 255) // 256 * 256 + 8)))
+
+
+@pytest.mark.parametrize("hidden,experts,top_k,inter", [(2048, 128, 8, 768), (4096, 64, 4, 1408), (2880, 32, 4, 2880),
+                                                        (1024, 32, 16, 512), (776, 8, 1, 4104), (8, 1024, 2, 8)])
+def test_moe_few_token_form_takes_at_most_two_passes(hidden, experts, top_k, inter):
+    """However the routing shares experts among the tokens, no expert takes more than two passes of the form's rows;
+    past that, gate/up and down each run the grouped form."""
+    gate_up, down = 2 * rows_of_a_pass(hidden), 2 * rows_of_a_pass(inter)
+    tokens = sorted({1, 8, 16, gate_up, gate_up + 1, down, down + 1, 33, 64})
+    for t, events in zip(tokens, record([(0, *moe(t, hidden, experts, top_k, inter)) for t in tokens])):
+        forms = [e.kernel.split("<")[0] for e in events if isinstance(e, Launch)]
+        assert forms[:2] == ["q4_few" if t <= gate_up else "q4_grouped", "q4_few" if t <= down else "q4_grouped"], (t, forms)

@@ -643,9 +643,9 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 }
 
 // ---------------------------------------------------------------------------
-// Few pairs: the grouped GEMM of decode steps (a handful of tokens per active
-// expert) over the same tiled planes, bound by the weight stream of the active
-// experts (8 tokens, 128 experts of 768 x 2048, top 8: 50 experts, 129 MB).
+// Few tokens: the grouped GEMM of decode steps (up to 32 tokens) over the same
+// tiled planes, bound by the weight stream of the active experts (8 tokens, 128
+// experts of 768 x 2048, top 8: 50 experts, 129 MB).
 //
 // q4_grouped at that size has few of its workgroups active, on the XCDs that
 // the routing happens to name, and pays a barrier per 256-column chunk. Here
@@ -669,7 +669,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 typedef std::uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kFewRows = 16;        // one MFMA's activation rows
-constexpr int kFewPairs = 512;      // pairs at most: the routing lists
+constexpr int kFewPairs = 512;      // two passes of them times the largest top_k
 constexpr int kFewLds = 66 * 1024;  // activation rows of a pass: two workgroups share a CU
 constexpr int kFewItems = 6;        // half chunks of a row block in flight
 
@@ -1077,15 +1077,13 @@ int few_rows(const Q4Tiled& p, int tokens) {
     return std::min(std::min(tokens, kFewRows), kFewLds / (2 * (p.chunks * kChunk + 8)));
 }
 
-// Whether q4_few is the faster form: one pass per expert in nearly every case
-// (no more tokens than rows of a pass, or on average half of them per expert).
-// MI355X, us, q4_grouped against q4_few for gate/up: 4 tokens per expert 78 ->
-// 70 (2048 columns, 16 rows a pass), 8 per expert 131 -> 156 (4096 columns, 8
-// rows); down at 8 per expert 131 -> 123, at 16 per expert 154 -> 161.
-bool few_pairs(const Q4Tiled& p, int tokens, int pairs) {
-    const int rows = few_rows(p, kFewRows);
-    return pairs <= kFewPairs && rows > 0 && (tokens <= rows || 2 * pairs <= p.experts * rows);
-}
+// Whether the call takes q4_few: an expert's tokens fit two passes, wherever the
+// routing sends them (which the host cannot see). Beyond, the wider passes of
+// q4_grouped are the faster ones where tokens share experts: all tokens on the
+// same 4 of 64 experts of 1408 x 4096 (eight rows a pass), us, q4_grouped
+// against this for gate/up: 16 tokens 62 / 54, 24 tokens 73 / 73, 32 tokens 69 /
+// 82, 48 tokens 79 / 110; tokens spread evenly gain up to 20 us at all of these.
+bool few_tokens(const Q4Tiled& p, int tokens) { return tokens <= 2 * few_rows(p, tokens); }
 
 template <int EPI, int W, bool ROUTE>
 void launch_q4_few(const Q4Tiled& p, int tokens, int pairs, int lds, hipStream_t stream) {
@@ -1789,7 +1787,7 @@ void moe_q4_launch_cfg(const void* x, const std::int64_t* ids, const void* score
     gu.slot_score = slot_score;
     gu.pairs = pairs;
     gu.top_k = top_k;
-    if (few_pairs(gu, tokens, pairs)) few_dispatch<kSwiGLU, true>(gu, tokens, pairs, stream);
+    if (few_tokens(gu, tokens)) few_dispatch<kSwiGLU, true>(gu, tokens, pairs, stream);
     else if (route_inside) launch_q4_grouped<kSwiGLU, GW, GRB, NBMAX, true, 1>(gu, stream);
     else launch_q4_grouped<kSwiGLU, GW, GRB, NBMAX, false, 1>(gu, stream);
 
@@ -1809,7 +1807,7 @@ void moe_q4_launch_cfg(const void* x, const std::int64_t* ids, const void* score
     dn.x_stride = inter;
     dn.out_stride = hidden;
     dn.experts = experts;
-    if (few_pairs(dn, tokens, pairs)) few_dispatch<kScore, false>(dn, tokens, pairs, stream);
+    if (few_tokens(dn, tokens)) few_dispatch<kScore, false>(dn, tokens, pairs, stream);
     else launch_q4_grouped<kScore, DW, DRB, NBMAX, false, 2>(dn, stream);
 
     combine_dispatch(top_k, ids, pair_slot, v, static_cast<__half*>(out), tokens, hidden, stream);
