@@ -62,6 +62,14 @@ const char* recorder_take() {
     return taken.c_str();
 }
 
+// The names of all registered kernels, one per line.
+const char* recorder_kernels() {
+    static std::string text;
+    text.clear();
+    for (const auto& [host, name] : names()) text += name_of(host) + "\n";
+    return text.c_str();
+}
+
 void** __hipRegisterFatBinary(const void*) {
     static void* modules = nullptr;
     return &modules;

@@ -25,7 +25,7 @@ POINTER = 1 << 30  # a device address that every alignment check accepts; never 
 CHILD = """
 import ctypes as C, json, sys
 recorder = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
-recorder.recorder_take.restype = C.c_char_p
+recorder.recorder_take.restype = recorder.recorder_kernels.restype = C.c_char_p
 library = C.CDLL(sys.argv[2])
 library.venturi_blocks_error.restype = C.c_char_p
 types = {"P": C.c_void_p, "i": C.c_int, "Q": C.c_uint64, "f": C.c_float}
@@ -36,7 +36,7 @@ for device, entry, signature, args in json.load(sys.stdin):
     recorder.recorder_device(device)
     status = function(*args)
     results.append((status, library.venturi_blocks_error().decode(), recorder.recorder_take().decode()))
-json.dump(results, sys.stdout)
+json.dump([results, recorder.recorder_kernels().decode()], sys.stdout)
 """
 
 
@@ -60,9 +60,10 @@ class LdsLimit:
 def _recorder():
     if shutil.which("g++") is None or not native.DEFAULT_LIBRARY.exists():
         pytest.skip("needs g++ and the built library")
-    target = Path(tempfile.mkdtemp(prefix="venturi-recorder-")) / "recorder.so"
+    folder = tempfile.TemporaryDirectory(prefix="venturi-recorder-")  # kept by the cache, removed at exit
+    target = Path(folder.name) / "recorder.so"
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(SOURCE), "-o", str(target)], check=True)
-    return target
+    return folder, target
 
 
 def _event(line):
@@ -70,16 +71,25 @@ def _event(line):
     return (Launch if kind == "launch" else LdsLimit)(kernel, *map(int, numbers))
 
 
+def _run(calls):
+    coded = [(device, entry, "".join(CODES[t] for t in native.SIGNATURES[entry][0]), args) for device, entry, args in calls]
+    done = subprocess.run([sys.executable, "-c", CHILD, str(_recorder()[1]), str(native.DEFAULT_LIBRARY)],
+                          input=json.dumps(coded), capture_output=True, text=True, check=True, timeout=120)
+    return json.loads(done.stdout)
+
+
 def record(calls):
     """The events of each call (device, entry point, arguments), in order, in one process."""
-    coded = [(device, entry, "".join(CODES[t] for t in native.SIGNATURES[entry][0]), args) for device, entry, args in calls]
-    done = subprocess.run([sys.executable, "-c", CHILD, str(_recorder()), str(native.DEFAULT_LIBRARY)],
-                          input=json.dumps(coded), capture_output=True, text=True, check=True, timeout=120)
     events = []
-    for (status, message, text), call in zip(json.loads(done.stdout), calls):
+    for (status, message, text), call in zip(_run(calls)[0], calls):
         assert status == 0, (call, message)
         events.append([_event(line) for line in text.splitlines()])
     return events
+
+
+def built(name):
+    """Every instantiation of a kernel template in the library."""
+    return {kernel for kernel in _run([])[1].splitlines() if kernel.split("<")[0] == name}
 
 
 def kernels(calls):

@@ -38,10 +38,13 @@ def activations(tokens, k, device, seed):
     return torch.randn(tokens, k, generator=torch.Generator().manual_seed(seed)).half().to(device)
 
 
-# (tokens, rows, columns): 256 x 128, 128 x 128, 64 x 128, 80 x 64, 64 x 64, 48 x 64, 32 x 64 and 32 x 32 tiles.
+# (tokens, rows, columns): 256 x 128, 128 x 128 and 64 x 128 tiles (the latter two with and without a K split), 80 x 64,
+# 64 x 64, 48 x 64, 32 x 64 and 32 x 32 tiles; test_launches.py checks that every tiling is reached.
 Q8_SHAPES = [(257, 14003, 136), (513, 7001, 136), (1025, 7001, 136), (300, 10001, 264), (97, 14003, 136),
              (33, 20001, 520), (129, 7001, 1032), (81, 14003, 1000), (160, 4100, 1032), (113, 7001, 1032),
-             (79, 14003, 136), (300, 4100, 136), (33, 14003, 136), (65, 10001, 200), (33, 257, 136), (97, 31, 3976)]
+             (79, 14003, 136), (300, 4100, 136), (33, 14003, 136), (65, 10001, 200), (33, 257, 136), (97, 31, 3976),
+             (700, 7001, 520), (2047, 2049, 520), (257, 10001, 520), (300, 20001, 264), (1025, 14003, 72), (129, 7001, 2056),
+             (33, 10001, 264)]
 
 
 @pytest.mark.parametrize("tokens,n,k", Q8_SHAPES)
@@ -60,8 +63,11 @@ def test_q8_tilings(backend, device, tokens, n, k):
     assert torch.equal(aligned, out)
 
 
-@pytest.mark.parametrize("tokens,n,k,shift", [(40, 70, 8, 0), (70, 33, 40, 0), (33, 64, 120, 0), (40, 300, 1000, 1),
-                                              (130, 64, 4096, 1), (33, 3, (1 << 22) + 8, 0)])
+Q8_OUTSIDE_SPLIT = [(40, 70, 8, 0), (70, 33, 40, 0), (33, 64, 120, 0), (40, 300, 1000, 1), (130, 64, 4096, 1),
+                    (33, 3, (1 << 22) + 8, 0)]
+
+
+@pytest.mark.parametrize("tokens,n,k,shift", Q8_OUTSIDE_SPLIT)
 def test_q8_operands_outside_the_split_form(backend, device, tokens, n, k, shift):
     # Fewer than 128 columns, scales aligned to 2 bytes only, rows past the 32-bit lane offsets.
     print(f"case q8 prefill fallback tokens={tokens} n={n} k={k} shift={shift}", flush=True)
@@ -76,6 +82,36 @@ def test_q8_operands_outside_the_split_form(backend, device, tokens, n, k, shift
                                          padded, 0, torch.cuda.current_stream(device).cuda_stream))
     assert guard[0] == 47 and guard[-1] == 47
     assert_bound(out, x.double(), values(codes, scales, k))
+
+
+def integers(shape, low, high, device, seed):
+    gen = torch.Generator().manual_seed(seed)
+    return torch.randint(low, high + 1, shape, dtype=torch.int8, generator=gen).to(device)
+
+
+def powers(shape, device, seed):
+    """Group scales 1/2, 1 and 2."""
+    return torch.exp2(integers(shape, -1, 1, device, seed).float())
+
+
+def assert_exact(got, x, w):
+    """Sums of small integers times powers of two: every association gives the same fp16 value."""
+    exact = x @ w.T
+    assert bool((exact.half().double() == exact).all())
+    assert torch.equal(got.double(), exact)
+
+
+@pytest.mark.parametrize("tokens,n,k", Q8_SHAPES)
+def test_q8_tilings_place_every_product(backend, device, tokens, n, k):
+    print(f"case q8 prefill exact sums tokens={tokens} n={n} k={k}", flush=True)
+    p = (k + 127) // 128 * 128
+    codes, scales = integers((n, p), -1, 1, device, n + k), powers((n, p // 32), device, n).half()
+    x = integers((tokens, k), -1, 1, device, tokens)
+    plan = backend.upload_linear(Q8RowSplitWeight(codes, scales, k), dtype=torch.float16, device=device).prepare(
+        tokens=tokens, route="mfma")
+    out = torch.empty(tokens, n, dtype=torch.float16, device=device)
+    plan.run(x.half(), out=out)
+    assert_exact(out, x.double(), values(codes, scales, k))
 
 
 def represented(workspace, tokens, k, passes):

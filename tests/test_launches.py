@@ -2,7 +2,9 @@
 
 import pytest
 
-from launches import LdsLimit, Launch, a8_gemm, a8_tiled, moe, padded, pointers, q4_gemm, q8_prefill, record
+from launches import (LdsLimit, Launch, a8_gemm, a8_tiled, built, kernels, moe, padded, pointers, q4_gemm, q8_prefill,
+                      record)
+import test_gpu_prefill_tilings as tilings
 
 DEFAULT_LDS = 64 * 1024
 
@@ -63,3 +65,21 @@ def test_moe_few_token_form_takes_at_most_two_passes(hidden, experts, top_k, int
     for t, events in zip(tokens, record([(0, *moe(t, hidden, experts, top_k, inter)) for t in tokens])):
         forms = [e.kernel.split("<")[0] for e in events if isinstance(e, Launch)]
         assert forms[:2] == ["q4_few" if t <= gate_up else "q4_grouped", "q4_few" if t <= down else "q4_grouped"], (t, forms)
+
+
+def reached(calls):
+    return {kernel for launched in kernels([(0, *call) for call in calls]) for kernel in launched}
+
+
+def test_q8_prefill_tests_reach_every_tiling():
+    calls = [q8_prefill(*shape) for shape in tilings.Q8_SHAPES]
+    calls += [q8_prefill(t, n, k, scales_offset=2 * shift) for t, n, k, shift in tilings.Q8_OUTSIDE_SPLIT]
+    assert built("q8_prefill") | built("q8_prefill_split") == reached(calls)
+
+
+def test_q8_prefill_of_short_rows_shares_the_cus():
+    """Where K is a few hundred columns and the grid fills the chip, the prologue and the output are the time: such calls
+    take a tiling without a K split, of which two or four workgroups share a CU."""
+    shapes = [(100, 34816, 136), (128, 34816, 256), (1024, 16384, 136), (8192, 16384, 256), (2048, 34816, 64)]
+    for shape, launched in zip(shapes, kernels([(0, *q8_prefill(*shape)) for shape in shapes])):
+        assert launched[0].startswith(("q8_prefill<1, 4, 1, 8, 2,", "q8_prefill<1, 4, 1, 4, 2,")), (shape, launched)

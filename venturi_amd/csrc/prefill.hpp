@@ -49,8 +49,8 @@ __device__ __forceinline__ int tile_of(const TileOrder& o) {
 
 // A tiling's measured time model, in microseconds: every round of workgroups
 // costs `round` (prologue, sum over the K waves, output) plus, per 1024
-// columns, `solo` when it leaves at most one workgroup on a CU and `full` when
-// a CU holds `per_cu`; `base` once.
+// columns, `solo` when it leaves at most one workgroup on a CU, `full` when a
+// CU holds `per_cu`, and in proportion between; `base` once.
 struct PrefillTiling {
     int tm, tn, per_cu;
     double base, round, solo, full;
@@ -60,9 +60,9 @@ inline double tiling_time(const PrefillTiling& t, int tokens, int n, double k) {
     const std::int64_t tiles = static_cast<std::int64_t>((tokens + t.tm - 1) / t.tm) * ((n + t.tn - 1) / t.tn);
     const std::int64_t slots = static_cast<std::int64_t>(device_cus()) * t.per_cu;
     const std::int64_t whole = tiles / slots, rest = tiles % slots;
-    const bool solo = rest > 0 && rest <= device_cus();
-    const double columns = static_cast<double>(whole + (rest > 0 && !solo)) * t.full + (solo ? t.solo : 0.0);
-    return t.base + static_cast<double>(whole + (rest > 0)) * t.round + k / 1024.0 * columns;
+    const std::int64_t level = (rest + device_cus() - 1) / device_cus();  // workgroups on a CU in the last round
+    const double last = level == 0 ? 0.0 : level == 1 ? t.solo : t.solo + (t.full - t.solo) * static_cast<double>(level - 1) / (t.per_cu - 1);
+    return t.base + static_cast<double>(whole + (rest > 0)) * t.round + k / 1024.0 * (static_cast<double>(whole) * t.full + last);
 }
 
 template <int N>

@@ -70,10 +70,11 @@ struct PrefillGeom {
     // A buffer holds whole rounds of the threads' stores, so no store is guarded.
     static constexpr int kABytes = kAPer * kThreads * 16, kBBytes = kBPer * kThreads * 16, kSBytes = kSPer * kThreads * 4;
     static constexpr int kStageBytes = kABytes + kBBytes + kSBytes;
-    // Output: the WK partial sums of OI token tiles of every wave at a time, fp32 rows of kTN + 4.
+    // Output: the WK partial sums of OI token tiles of every wave at a time, fp32 rows of kTN + 4. Where one wave runs
+    // the whole K, up to 36 KB of them at once: four workgroups still share a CU.
     static constexpr int kPitch = kTN + 4;
     static constexpr int out_bytes(int oi) { return WK * WT * oi * 16 * kPitch * 4; }
-    static constexpr int kOI = out_bytes(TI) <= 2 * kStageBytes   ? TI
+    static constexpr int kOI = out_bytes(TI) <= 2 * kStageBytes || (WK == 1 && out_bytes(TI) <= 36 * 1024) ? TI
                                : TI % 2 == 0 && out_bytes(TI / 2) <= 2 * kStageBytes ? TI / 2
                                : TI % 4 == 0 && out_bytes(TI / 4) <= 2 * kStageBytes ? TI / 4
                                                                                       : 1;
@@ -126,8 +127,9 @@ __global__ __launch_bounds__(WT * WN * WK * 64, 2) void q8_prefill(const __half*
     // stage 0 then starts at the last column base, stage s > 0 at s - 1.
     constexpr int KC = 32 * KG;
     const int whole = k / KC, first = whole < stages ? whole : 0, shift = whole < stages ? 1 : 0;
-    uint4 st_a[PF][G::kAPer], st_b[PF][G::kBPer];  // PF stages in flight
-    unsigned short st_s[PF][G::kSPer];
+    constexpr int kSlots = PF < 2 ? 2 : PF;  // PF stages in flight, two in the prologue
+    uint4 st_a[kSlots][G::kAPer], st_b[kSlots][G::kBPer];
+    unsigned short st_s[kSlots][G::kSPer];
     // Loads stage columns [c0, c0 + KC), all of them real ones.
     auto load = [&](int base, auto slot) __attribute__((always_inline)) {
 #pragma unroll
@@ -221,10 +223,11 @@ __global__ __launch_bounds__(WT * WN * WK * 64, 2) void q8_prefill(const __half*
     // (each activation fragment as soon as its register is free), stage s + 2
     // is written to LDS and stage s + 3 is requested from memory.
     const int last = max(whole - 1, 0);  // the last whole stage's column base
+    // The first two stages are requested together: for short rows the prologue
+    // is most of the time.
     load_edge(first, Slot<0>{});
-    store(0, Slot<0>{});
     if (whole == 0) {
-        // The partial stage is the only one: the loop's requests (never
+        // The partial stage is the only one: the other requests (never
         // consumed) stay on column 0 of their rows.
 #pragma unroll
         for (int u = 0; u < G::kAPer; ++u) a_off[u] -= 16u * ((tid + u * T) % AU);
@@ -233,10 +236,9 @@ __global__ __launch_bounds__(WT * WN * WK * 64, 2) void q8_prefill(const __half*
 #pragma unroll
         for (int u = 0; u < G::kSPer; ++u) s_off[u] -= 2u * ((tid + u * T) % KG);
     }
-    if (stages > 1) {
-        load(1 - shift, Slot<0>{});
-        store(1, Slot<0>{});
-    }
+    load(min(1 - shift, last), Slot<1>{});
+    store(0, Slot<0>{});
+    store(1, Slot<1>{});
     each_slot<PF>([&](auto p) __attribute__((always_inline)) { load(min(2 + p - shift, last), p); });
     __syncthreads();
 #pragma unroll
@@ -603,26 +605,33 @@ void q8_prefill_launch(const void* x, const std::int8_t* codes, const __half* sc
         launch_prefill<1, 2, 4, 4, 4, 1, std::uint64_t>(xp, codes, scales, op, tokens, n, k, padded, stream);
         return;
     }
-    // The tiling with the least predicted time; the constants are a fit to 115
-    // shapes (33-2048 tokens, 1024-34816 rows, 1024-25600 columns; each
-    // candidate timed on each shape on MI355X): the choice is within 8% of the
-    // fastest candidate on every one of them and 0.4% on average.
-    constexpr PrefillTiling kTilings[8] = {
-        {256, 128, 1, 0.0, 6.67, 18.50, 18.50}, {128, 128, 1, 0.0, 6.84, 9.59, 9.59}, {64, 128, 1, 0.3, 4.87, 5.93, 5.93},
-        {80, 64, 2, 0.0, 6.93, 3.75, 9.03},     {64, 64, 2, 2.2, 3.33, 3.42, 7.26},   {48, 64, 2, 2.6, 2.48, 2.80, 6.13},
-        {32, 64, 2, 2.9, 1.04, 2.51, 5.16},     {32, 32, 1, 2.3, 0.45, 1.88, 1.88}};
+    // The tiling with the least predicted time; the constants are a fit to 770
+    // shapes (33-8192 tokens, 256-151936 rows, 64-25600 columns; each candidate
+    // timed on each shape on MI355X): the choice is within 11% of the fastest
+    // candidate on every one of them and 0.2% on average. The two without a K
+    // split share a CU (two and four workgroups) and win where K is short, so
+    // that prologue and output count (16384 rows x 256 columns, 8192 tokens:
+    // 256 x 128 tiles 198 us, these 147; 100 tokens x 34816 rows x 136: the
+    // fastest of the others 13.6, these 8.0).
+    constexpr PrefillTiling kTilings[10] = {
+        {256, 128, 1, 0.6, 7.09, 19.16, 19.16}, {128, 128, 1, 0.1, 6.02, 10.00, 10.00}, {64, 128, 1, 0.1, 4.77, 5.80, 5.80},
+        {128, 128, 2, 1.5, 2.33, 15.02, 27.81}, {64, 128, 4, 0.6, 1.77, 10.98, 40.16},  {80, 64, 1, 1.6, 4.23, 3.94, 3.94},
+        {64, 64, 2, 2.0, 2.67, 3.91, 6.87},     {48, 64, 2, 2.4, 1.84, 2.28, 7.21},     {32, 64, 2, 2.7, 0.91, 1.59, 5.30},
+        {32, 32, 1, 2.1, 1.64, 1.32, 1.32}};
     int best = fastest_tiling(kTilings, tokens, n, k);
     // The split form reads a chunk's four scales as one 8-byte word and needs
     // one whole chunk.
-    if (best >= 3 && (k < 128 || !aligned(scales, 8))) best = 2;
+    if (best >= 5 && (k < 128 || !aligned(scales, 8))) best = k < 128 ? 4 : 2;
     switch (best) {
         case 0: launch_prefill<2, 2, 2, 8, 4, 1>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
         case 1: launch_prefill<1, 2, 4, 8, 4, 1>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
         case 2: launch_prefill<1, 2, 4, 4, 4, 2>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
-        case 3: launch_split<4, 5, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
-        case 4: launch_split<4, 4, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
-        case 5: launch_split<4, 3, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
-        case 6: launch_split<4, 2, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 3: launch_prefill<1, 4, 1, 8, 2, 1>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 4: launch_prefill<1, 4, 1, 4, 2, 1>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 5: launch_split<4, 5, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 6: launch_split<4, 4, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 7: launch_split<4, 3, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
+        case 8: launch_split<4, 2, 4>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
         default: launch_split<8, 2, 2>(xp, codes, scales, op, tokens, n, k, padded, stream); break;
     }
 }
