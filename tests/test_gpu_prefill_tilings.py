@@ -123,12 +123,17 @@ def represented(workspace, tokens, k, passes):
     return (codes * scales).sum(0).view(tokens, groups * 32)[:, :k]
 
 
-# 256 x 128, 128 x 128, 64 x 128, 64 x 64 (eight and four K waves), 48 x 64 (four and eight), 32 x 64 and 32 x 32
-# tiles; whole and partial stages and chunks (K % 128), K below one chunk, one and two passes.
+# 256 x 128, 128 x 128 and 64 x 128 (with and without a K split), 32 x 128, 64 x 64 (eight and four K waves), 48 x 64 (four
+# and eight), 32 x 64 and 32 x 32 tiles (test_launches.py checks that every tiling is reached); whole and partial stages
+# and chunks (K % 128), K below one chunk, one and two passes, two passes that each have a partial and whole stages.
 A8_SHAPES = [(257, 14003, 136, 1), (513, 7001, 128, 2), (129, 14003, 136, 1), (257, 7001, 300, 1), (65, 10001, 136, 1),
              (33, 14003, 256, 1), (97, 7001, 520, 1), (160, 4100, 520, 2), (97, 14003, 4104, 1), (200, 7001, 2056, 2),
              (65, 10001, 1032, 1), (79, 10001, 519, 2), (33, 14003, 136, 2), (97, 4100, 520, 1), (33, 4100, 1032, 1),
-             (47, 4100, 520, 2), (65, 257, 136, 1), (33, 257, 129, 2), (81, 31, 3971, 1), (65, 70, 31, 2), (40, 33, 127, 1)]
+             (47, 4100, 520, 2), (65, 257, 136, 1), (33, 257, 129, 2), (81, 31, 3971, 1), (65, 70, 31, 2), (40, 33, 127, 1),
+             (700, 7001, 520, 1), (700, 7001, 264, 2), (257, 7001, 264, 1), (257, 7001, 136, 2), (200, 7001, 264, 1),
+             (200, 7001, 136, 2), (700, 10001, 136, 1), (700, 7001, 136, 2), (129, 7001, 72, 1), (513, 7001, 130, 2),
+             (97, 4100, 136, 1), (160, 4100, 2056, 2), (47, 4100, 1032, 2), (97, 4100, 2056, 1),
+             (33, 3, (1 << 22) + 8, 1)]  # the last: rows past the 32-bit lane offsets
 
 
 @pytest.mark.parametrize("tokens,n,k,passes", A8_SHAPES)
@@ -151,7 +156,26 @@ def test_a8_tilings(backend, device, tokens, n, k, passes):
     assert torch.equal(aligned[keep], out[keep])
 
 
-@pytest.mark.parametrize("tokens,n,k,passes", [(130, 300, 1000, 1), (70, 64, 4096, 2)])
+@pytest.mark.parametrize("tokens,n,k,passes", A8_SHAPES[:-1])  # (sums of four million products exceed fp16's integers)
+def test_a8_tilings_place_every_product(backend, device, tokens, n, k, passes):
+    print(f"case a8 prefill exact sums tokens={tokens} n={n} k={k} passes={passes}", flush=True)
+    p, groups = (k + 127) // 128 * 128, (k + 31) // 32
+    codes, scales = integers((n, p), -1, 1, device, n + k), powers((n, p // 32), device, n).half()
+    acts = integers((passes, tokens, groups * 32), -1, 1, device, tokens)
+    acts[:, :, k:] = 0
+    ascales = powers((passes, tokens, groups), device, tokens + 1)
+    workspace = torch.cat((acts.flatten().view(torch.uint8), ascales.flatten().view(torch.uint8)))
+    lib, stream = backend._native, torch.cuda.current_stream(device).cuda_stream
+    out = torch.empty(tokens, n, dtype=torch.float16, device=device)
+    lib.check(lib.venturi_q8_a8_gemm_run(workspace.data_ptr(), workspace.numel(), codes.data_ptr(), scales.data_ptr(),
+                                         out.data_ptr(), tokens, n, k, p, passes, stream))
+    assert_exact(out, represented(workspace, tokens, k, passes), values(codes, scales, k))
+
+
+A8_TWO_BYTE_SCALES = [(130, 300, 1000, 1), (70, 64, 4096, 2), (70, 64, 4104, 2)]
+
+
+@pytest.mark.parametrize("tokens,n,k,passes", A8_TWO_BYTE_SCALES)
 def test_a8_scales_aligned_to_two_bytes(backend, device, tokens, n, k, passes):
     print(f"case a8 prefill fallback tokens={tokens} n={n} k={k}", flush=True)
     codes, scales = (t.to(device) for t in random_q8(n, k, 5 + n + tokens))

@@ -83,3 +83,28 @@ def test_q8_prefill_of_short_rows_shares_the_cus():
     shapes = [(100, 34816, 136), (128, 34816, 256), (1024, 16384, 136), (8192, 16384, 256), (2048, 34816, 64)]
     for shape, launched in zip(shapes, kernels([(0, *q8_prefill(*shape)) for shape in shapes])):
         assert launched[0].startswith(("q8_prefill<1, 4, 1, 8, 2,", "q8_prefill<1, 4, 1, 4, 2,")), (shape, launched)
+
+
+def test_a8_prefill_tests_reach_every_tiling():
+    calls = [a8_gemm(*shape) for shape in tilings.A8_SHAPES]
+    calls += [a8_gemm(*shape, scales_offset=2) for shape in tilings.A8_TWO_BYTE_SCALES]
+    assert built("a8_prefill") | built("a8_prefill_split") == reached(calls)
+
+
+def test_a8_prefill_tests_reach_two_passes_with_partial_and_whole_stages():
+    """Both passes' partial stages come first, then the whole ones of each: on every cooperative tiling that can have a
+    partial stage (K split over two or four waves, one 32-column group per wave and stage)."""
+    want = {name for name in built("a8_prefill") if int(name.split(",")[2]) > 1 and "unsigned int" in name}
+    seen = set()
+    for shape, launched in zip(tilings.A8_SHAPES, kernels([(0, *a8_gemm(*shape)) for shape in tilings.A8_SHAPES])):
+        if shape[3] == 2 and launched[0] in want:
+            groups, waves = (shape[2] + 31) // 32, int(launched[0].split(",")[2])
+            if groups > waves and groups % waves:
+                seen.add(launched[0])
+    assert seen == want
+
+
+def test_a8_prefill_of_short_rows_shares_the_cus():
+    shapes = [(100, 34816, 136, 1), (128, 34816, 256, 1), (1024, 16384, 136, 1), (8192, 16384, 256, 1), (2048, 34816, 64, 1)]
+    for shape, launched in zip(shapes, kernels([(0, *a8_gemm(*shape)) for shape in shapes])):
+        assert launched[0].startswith(("a8_prefill<1, 4, 1, 8, 2,", "a8_prefill<1, 4, 1, 4, 2,")), (shape, launched)

@@ -210,10 +210,13 @@ __global__ __launch_bounds__(WT * WN * WK * 64, 2) void a8_prefill(const std::in
     // stages of pass 0 and of pass 1.
     const int whole = groups / KG, edges = whole * KG < groups ? passes : 0;
     const int stages = edges + passes * whole;
-    u32x4 st_a[G::kAPer], st_b[G::kBPer];
-    float st_as[G::kAsPer];
-    unsigned short st_ws[G::kWsPer];
-    auto load = [&](int stage) __attribute__((always_inline)) {
+    struct Stage {
+        u32x4 a[G::kAPer], b[G::kBPer];
+        float as[G::kAsPer];
+        unsigned short ws[G::kWsPer];
+    };
+    Stage st;
+    auto load = [&](int stage, Stage& st) __attribute__((always_inline)) {
         const int w = min(max(stage - edges, 0), max(passes * whole - 1, 0));
         const int pass = w >= whole && w > 0 ? 1 : 0;
         const std::int64_t base = w - pass * whole;
@@ -222,28 +225,28 @@ __global__ __launch_bounds__(WT * WN * WK * 64, 2) void a8_prefill(const std::in
         const char* bp = b_base + base * (32 * KG);
         const char* wp = ws_base + base * (2 * KG);
 #pragma unroll
-        for (int u = 0; u < G::kAPer; ++u) st_a[u] = *reinterpret_cast<const u32x4*>(ap + lane_offset(a_off[u]));
+        for (int u = 0; u < G::kAPer; ++u) st.a[u] = *reinterpret_cast<const u32x4*>(ap + lane_offset(a_off[u]));
 #pragma unroll
-        for (int u = 0; u < G::kBPer; ++u) st_b[u] = *reinterpret_cast<const u32x4*>(bp + lane_offset(b_off[u]));
+        for (int u = 0; u < G::kBPer; ++u) st.b[u] = *reinterpret_cast<const u32x4*>(bp + lane_offset(b_off[u]));
 #pragma unroll
-        for (int u = 0; u < G::kAsPer; ++u) st_as[u] = *reinterpret_cast<const float*>(sp + lane_offset(as_off[u]));
+        for (int u = 0; u < G::kAsPer; ++u) st.as[u] = *reinterpret_cast<const float*>(sp + lane_offset(as_off[u]));
 #pragma unroll
         for (int u = 0; u < G::kWsPer; ++u)
-            st_ws[u] = *reinterpret_cast<const unsigned short*>(wp + lane_offset(ws_off[u]));
+            st.ws[u] = *reinterpret_cast<const unsigned short*>(wp + lane_offset(ws_off[u]));
     };
     // The partial stage of a pass: groups past the last one carry scale 0 (their codes are clamped, finite).
-    auto load_edge = [&](int pass) __attribute__((always_inline)) {
+    auto load_edge = [&](int pass, Stage& st) __attribute__((always_inline)) {
         const int g0 = whole * KG;
 #pragma unroll
         for (int u = 0; u < G::kAPer; ++u) {
             const int unit = (tid + u * T) % U;
-            st_a[u] = *reinterpret_cast<const u32x4*>(
+            st.a[u] = *reinterpret_cast<const u32x4*>(
                 a_base + pass * count * 32 + a_off[u] + 16 * static_cast<std::int64_t>(min(2 * g0, 2 * groups - 1 - unit)));
         }
 #pragma unroll
         for (int u = 0; u < G::kBPer; ++u) {
             const int unit = (tid + u * T) % U;
-            st_b[u] = *reinterpret_cast<const u32x4*>(
+            st.b[u] = *reinterpret_cast<const u32x4*>(
                 b_base + b_off[u] + 16 * static_cast<std::int64_t>(min(2 * g0, 2 * groups - 1 - unit)));
         }
 #pragma unroll
@@ -251,27 +254,27 @@ __global__ __launch_bounds__(WT * WN * WK * 64, 2) void a8_prefill(const std::in
             const int g = (tid + u * T) % KG;
             const float v = *reinterpret_cast<const float*>(as_base + pass * count * 4 + as_off[u] +
                                                             4 * static_cast<std::int64_t>(min(g0, groups - 1 - g)));
-            st_as[u] = g0 + g < groups ? v : 0.0f;
+            st.as[u] = g0 + g < groups ? v : 0.0f;
         }
 #pragma unroll
         for (int u = 0; u < G::kWsPer; ++u) {
             const int g = (tid + u * T) % KG;
             const unsigned short v = *reinterpret_cast<const unsigned short*>(
                 ws_base + ws_off[u] + 2 * static_cast<std::int64_t>(min(g0, groups - 1 - g)));
-            st_ws[u] = g0 + g < groups ? v : 0;
+            st.ws[u] = g0 + g < groups ? v : 0;
         }
     };
-    auto store = [&](int buf) __attribute__((always_inline)) {
+    auto store = [&](int buf, const Stage& st) __attribute__((always_inline)) {
         unsigned char* base = lds + buf * G::kStage;
 #pragma unroll
-        for (int u = 0; u < G::kAPer; ++u) *reinterpret_cast<u32x4*>(base + a_put[u]) = st_a[u];
+        for (int u = 0; u < G::kAPer; ++u) *reinterpret_cast<u32x4*>(base + a_put[u]) = st.a[u];
 #pragma unroll
-        for (int u = 0; u < G::kBPer; ++u) *reinterpret_cast<u32x4*>(base + b_put[u]) = st_b[u];
+        for (int u = 0; u < G::kBPer; ++u) *reinterpret_cast<u32x4*>(base + b_put[u]) = st.b[u];
 #pragma unroll
-        for (int u = 0; u < G::kAsPer; ++u) *reinterpret_cast<float*>(base + as_put[u]) = st_as[u];
+        for (int u = 0; u < G::kAsPer; ++u) *reinterpret_cast<float*>(base + as_put[u]) = st.as[u];
 #pragma unroll
         for (int u = 0; u < G::kWsPer; ++u)
-            *reinterpret_cast<float*>(base + ws_put[u]) = __half2float(__ushort_as_half(st_ws[u]));
+            *reinterpret_cast<float*>(base + ws_put[u]) = __half2float(__ushort_as_half(st.ws[u]));
     };
     const std::uint32_t a_get = 16 * ((wt * TI * 16 + r) * U + ((2 * wk + (q >> 1)) ^ swizzle<U>(r))) + 8 * (q & 1);
     const std::uint32_t b_get =
@@ -285,19 +288,14 @@ __global__ __launch_bounds__(WT * WN * WK * 64, 2) void a8_prefill(const std::in
 
     A8Tile<TI, TJ> m;
     m.clear();
-    if (edges > 0) {
-        load_edge(0);
-        store(0);
-    } else {
-        load(0);
-        store(0);
-    }
-    if (edges > 1) {
-        load_edge(1);
-        store(1);
-    } else if (stages > 1) {
-        load(1);
-        store(1);
+    {  // the first two stages are requested together: for short rows the prologue is most of the time
+        Stage first;
+        if (edges > 0) load_edge(0, first);
+        else load(0, first);
+        if (edges > 1) load_edge(1, st);
+        else if (stages > 1) load(1, st);
+        store(0, first);
+        if (stages > 1) store(1, st);
     }
     if (whole == 0) {  // no whole stage: the loop's requests (never consumed) stay on group 0 of their rows
 #pragma unroll
@@ -309,15 +307,15 @@ __global__ __launch_bounds__(WT * WN * WK * 64, 2) void a8_prefill(const std::in
 #pragma unroll
         for (int u = 0; u < G::kWsPer; ++u) ws_off[u] -= 2 * ((tid + u * T) % KG);
     }
-    load(2);
+    load(2, st);
     __syncthreads();
     m.fill(source(0));
     __syncthreads();
     constexpr int kStoreAt = TI * TJ / 4, kLoadAt = TI * TJ / 4 + 2;
     for (int sg = 0; sg < stages; ++sg) {
         m.group(source((sg + 1) & 1), [&](int t) __attribute__((always_inline)) {
-            if (t == kStoreAt) store(sg & 1);
-            if (t == kLoadAt) load(sg + 3);
+            if (t == kStoreAt) store(sg & 1, st);
+            if (t == kLoadAt) load(sg + 3, st);
         });
         __syncthreads();
     }
@@ -711,27 +709,35 @@ void a8_fast_launch(const void* workspace, const std::int8_t* codes, const __hal
         return;
     }
     // The tiling with the least predicted time (the passes run one after the
-    // other over K); the constants are a fit to 105 shapes (33-2048 tokens,
-    // 1024-34816 rows, 1024-25600 columns, one and two passes; each candidate
-    // timed on each shape on MI355X): the choice is within 9% of the fastest
-    // candidate on every one of them and 0.5% on average.
-    constexpr PrefillTiling kTilings[9] = {
-        {256, 128, 1, 0.0, 6.12, 21.59, 21.59}, {128, 128, 1, 0.0, 7.25, 10.83, 10.83}, {64, 128, 1, 0.9, 4.39, 7.05, 7.05},
-        {64, 64, 1, 0.8, 5.99, 3.22, 3.22},     {64, 64, 2, 3.1, 4.02, 3.66, 6.34},     {48, 64, 2, 3.5, 2.78, 3.14, 5.40},
-        {48, 64, 1, 1.2, 4.84, 2.70, 2.70},     {32, 64, 1, 1.5, 3.74, 2.23, 2.23},     {32, 32, 1, 2.9, 0.72, 1.71, 1.71}};
+    // other over K); the constants are a fit to 770 shapes (33-8192
+    // tokens, 256-151936 rows, 64-25600 columns; each candidate timed on each
+    // shape on MI355X): the choice is within 11% of the fastest candidate on
+    // every one of them and 0.2% on average. The three without a K split share
+    // a CU (two or four workgroups) and win where K is short, so that prologue
+    // and output count (16384 rows x 256 columns, 8192 tokens: 256 x 128 tiles
+    // 228 us, these 184; 100 tokens x 34816 rows x 136: the fastest of the
+    // others 16.2, these 9.0).
+    constexpr PrefillTiling kTilings[12] = {
+        {256, 128, 1, 1.1, 6.25, 24.46, 24.46}, {128, 128, 1, 0.0, 5.10, 12.71, 12.71}, {64, 128, 1, 0.7, 3.98, 7.14, 7.14},
+        {128, 128, 2, 2.4, 2.96, 17.78, 30.71}, {64, 128, 4, 0.8, 1.64, 16.16, 54.83},  {32, 128, 4, 0.2, 0.00, 30.22, 68.00},
+        {64, 64, 1, 1.7, 4.73, 3.48, 3.48},     {64, 64, 2, 1.8, 3.36, 4.10, 6.94},     {48, 64, 2, 1.9, 2.83, 3.60, 6.05},
+        {48, 64, 1, 0.9, 4.41, 3.13, 3.13},     {32, 64, 1, 1.0, 2.96, 3.00, 3.00},     {32, 32, 1, 1.8, 0.88, 2.03, 2.03}};
     int best = fastest_tiling(kTilings, tokens, n, static_cast<double>(k) * passes);
     // The split form reads a chunk's four weight scales as one 8-byte word and
     // needs one whole chunk.
-    if (best >= 3 && (k < 128 || !aligned(scales, 8))) best = 2;
+    if (best >= 6 && (k < 128 || !aligned(scales, 8))) best = k < 128 ? 4 : 2;
     switch (best) {
         case 0: launch_coop<2, 2, 2, 8, 4>(o, stream); break;
         case 1: launch_coop<1, 2, 4, 8, 4>(o, stream); break;
         case 2: launch_coop<1, 2, 4, 4, 4>(o, stream); break;
-        case 3: launch_split<8, 4, 4>(o, stream); break;
-        case 4: launch_split<4, 4, 4>(o, stream); break;
-        case 5: launch_split<4, 3, 4>(o, stream); break;
-        case 6: launch_split<8, 3, 4>(o, stream); break;
-        case 7: launch_split<8, 2, 4>(o, stream); break;
+        case 3: launch_coop<1, 4, 1, 8, 2>(o, stream); break;
+        case 4: launch_coop<1, 4, 1, 4, 2>(o, stream); break;
+        case 5: launch_coop<1, 4, 1, 2, 2>(o, stream); break;
+        case 6: launch_split<8, 4, 4>(o, stream); break;
+        case 7: launch_split<4, 4, 4>(o, stream); break;
+        case 8: launch_split<4, 3, 4>(o, stream); break;
+        case 9: launch_split<8, 3, 4>(o, stream); break;
+        case 10: launch_split<8, 2, 4>(o, stream); break;
         default: launch_split<8, 2, 2>(o, stream); break;
     }
 }
