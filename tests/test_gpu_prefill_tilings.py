@@ -192,11 +192,14 @@ def test_a8_scales_aligned_to_two_bytes(backend, device, tokens, n, k, passes):
     assert_bound(out, represented(workspace, tokens, k, passes), values(codes, scales, k))
 
 
-# 128 x 128, 64 x 128, 64 x 64 (eight and four K waves), 48 x 64 (four and eight), 32 x 64 and 32 x 32 tiles, the wide
-# tiles of the large grids, K below one chunk, and the first token count of the route.
+# 128 x 128 (with and without a K split), 64 x 128, 64 x 64 (eight and four K waves), 48 x 64 (four and eight), 32 x 64 and
+# 32 x 32 tiles, the wide tiles of the large grids (test_launches.py checks that every tiling is reached), K below one
+# chunk, and the first token count of the route.
 Q4_SHAPES = [(300, 10001, 264), (129, 7001, 520), (97, 7001, 1032), (113, 14003, 2056), (65, 14003, 520),
              (97, 4100, 1032), (47, 4100, 1032), (65, 257, 136), (32, 33, 3976), (33, 70, 40), (40, 300, 120),
-             (1025, 14003, 264), (513, 14003, 136), (1025, 10001, 136), (700, 7001, 2056), (65, 10001, 136), (200, 2049, 1000), (513, 1000, 2056)]
+             (1025, 14003, 264), (513, 14003, 136), (1025, 10001, 136), (700, 7001, 2056), (65, 10001, 136), (200, 2049, 1000), (513, 1000, 2056),
+             (65, 20001, 136), (200, 10001, 2056), (513, 7001, 4104), (2047, 4100, 136), (513, 14003, 2056),
+             (2047, 7001, 136), (33, 3, (1 << 22) + 8)]  # the last: rows past the 32-bit lane offsets
 
 
 @pytest.mark.parametrize("tokens,n,k", Q4_SHAPES)
@@ -220,6 +223,20 @@ def test_q4_tilings(backend, device, tokens, n, k):
     aligned = torch.empty(tokens, n, dtype=torch.float16, device=device)
     plan.run(x, out=aligned)  # 16-byte stores where n allows them: the same bits
     assert torch.equal(aligned, out)
+
+
+@pytest.mark.parametrize("tokens,n,k", Q4_SHAPES[:-1])  # (sums of four million products exceed fp16's integers)
+def test_q4_tilings_place_every_product(backend, device, tokens, n, k):
+    print(f"case q4 prefill exact sums tokens={tokens} n={n} k={k}", flush=True)
+    p = (k + 127) // 128 * 128
+    signed, scales = integers((n, p), -1, 1, device, n + k), powers((n, p // 64), device, n).half()
+    nibbles = signed.view(torch.uint8) & 15
+    x = integers((tokens, k), -1, 1, device, tokens)
+    plan = backend.upload_linear(Q4RowSplitWeight(nibbles[:, 0::2] | (nibbles[:, 1::2] << 4), scales, k),
+                                 dtype=torch.float16, device=device).prepare(tokens=tokens, route="mfma")
+    out = torch.empty(tokens, n, dtype=torch.float16, device=device)
+    plan.run(x.half(), out=out)
+    assert_exact(out, x.double(), values(signed, scales, k))
 
 
 # The split form over the tiled planes: one, two and three row blocks per workgroup, four K waves past 768 blocks;

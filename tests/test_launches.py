@@ -108,3 +108,18 @@ def test_a8_prefill_of_short_rows_shares_the_cus():
     shapes = [(100, 34816, 136, 1), (128, 34816, 256, 1), (1024, 16384, 136, 1), (8192, 16384, 256, 1), (2048, 34816, 64, 1)]
     for shape, launched in zip(shapes, kernels([(0, *a8_gemm(*shape)) for shape in shapes])):
         assert launched[0].startswith(("a8_prefill<1, 4, 1, 8, 2,", "a8_prefill<1, 4, 1, 4, 2,")), (shape, launched)
+
+
+def test_q4_prefill_tests_reach_every_tiling():
+    names = built("q4_prefill") | built("q4_prefill_split") | {k for k in built("row_prefill") if k.startswith("row_prefill<0,")}
+    assert names == reached([q4_gemm(*shape) for shape in tilings.Q4_SHAPES])
+
+
+def test_q4_prefill_of_short_rows_and_of_rows_past_the_lane_offsets_takes_the_tiles_that_win_there():
+    """Short rows on a full grid, and, below 256 tokens, rows past the 32-bit lane offsets: 128 x 128 tiles with the whole
+    K in one wave, two workgroups to a CU. Those rows in longer prompts: the 256-token tiles."""
+    short = [(100, 34816, 1024), (128, 151936, 1024), (200, 65536, 512), (100, 250000, 136), (33, 151936, 64),
+             (100, 64, (1 << 22) + 8)]
+    for shape, launched in zip(short, kernels([(0, *q4_gemm(*shape)) for shape in short])):
+        assert launched == ["row_prefill<0, 4, 2, 2, 4, 2, 1>"], (shape, launched)
+    assert kernels([(0, *q4_gemm(256, 64, (1 << 22) + 8))])[0][0].startswith("row_prefill<0, 4, 2, 4, ")

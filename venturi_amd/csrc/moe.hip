@@ -27,9 +27,9 @@
 
 namespace vt {
 
-// w4a16.hip: false where the wide tiles of row_prefill are the faster ones.
-bool q4_prefill_launch(const __half* x, const std::uint8_t* codes, const __half* scales, __half* out, int tokens, int n,
-                       int k, int padded, hipStream_t stream);
+// w4a16.hip: 0, or the tile of row_prefill that is the faster form for this shape (-1: none is known to be).
+int q4_prefill_launch(const __half* x, const std::uint8_t* codes, const __half* scales, __half* out, int tokens, int n,
+                      int k, int padded, hipStream_t stream);
 
 namespace {
 
@@ -1662,24 +1662,18 @@ void row_decode_dispatch(const __half* x, const std::uint8_t* codes, const std::
 // GEMM reads each weight once per 16 or 32 tokens).
 constexpr int kRowPrefillMinTokens = 32;
 
-// Prefill tiles. Q4 runs the kernels of w4a16.hip except where these are the
-// faster ones. Q5 and Q6, below 256 tokens: 128 tokens x 128 rows (8 waves of
-// 32 x 64). Otherwise: 256 tokens x 32*TJ rows, 8 waves of 64 x 16*TJ (one
+// Prefill tiles. Q4 asks w4a16.hip, which runs the projection itself or names
+// the tile here that its time model finds the fastest. Q5 and Q6 (and Q4 rows
+// past that model), below 256 tokens: 128 tokens x 128 rows (8 waves of 32 x 64).
+// Otherwise: 256 tokens x 32*TJ rows, 8 waves of 64 x 16*TJ (one
 // workgroup per CU by LDS), TJ in {5, 6, 7} picked for the fewest tile rounds
 // over the CUs weighted by the wider tiles' higher rate (fewer LDS bytes per
 // MFMA): at M = 2048 on MI355X, 5120 rows take TJ = 5 (256 tiles, one round),
 // 7168 and 34816 rows TJ = 7 (config-2 W4A16 at M = 2048: QKV / o_proj /
 // gate+up / down 214 / 196 / 908 / 532 -> 155-162 / 144-151 / 729-774 /
 // 386-409 us against 128 x 128 tiles; same bytes).
-template <int HB>
-void row_prefill_dispatch(const __half* x, const std::uint8_t* codes, const std::uint8_t* high, const __half* scales,
-                          __half* out, int tokens, int n, int k, int padded, hipStream_t stream) {
-    if constexpr (HB == 0) {
-        if (q4_prefill_launch(x, codes, scales, out, tokens, n, k, padded, stream)) return;
-    } else if (tokens < 256) {
-        launch_row_prefill<HB, 4, 2, 2, 4, 2>(x, codes, high, scales, out, tokens, n, k, padded, stream);
-        return;
-    }
+int row_prefill_tile(int tokens, int n) {
+    if (tokens < 256) return 4;
     const int cus = device_cus();
     const std::int64_t token_tiles = (tokens + 255) / 256;
     int best = 5;
@@ -1693,9 +1687,22 @@ void row_prefill_dispatch(const __half* x, const std::uint8_t* codes, const std:
             best_cost = cost;
         }
     }
-    if (best == 5) launch_row_prefill<HB, 4, 2, 4, 5, 2>(x, codes, high, scales, out, tokens, n, k, padded, stream);
-    else if (best == 6) launch_row_prefill<HB, 4, 2, 4, 6, 2>(x, codes, high, scales, out, tokens, n, k, padded, stream);
-    else launch_row_prefill<HB, 4, 2, 4, 7, 1>(x, codes, high, scales, out, tokens, n, k, padded, stream);
+    return best;
+}
+
+template <int HB>
+void row_prefill_dispatch(const __half* x, const std::uint8_t* codes, const std::uint8_t* high, const __half* scales,
+                          __half* out, int tokens, int n, int k, int padded, hipStream_t stream) {
+    int tile = -1;
+    if constexpr (HB == 0) tile = q4_prefill_launch(x, codes, scales, out, tokens, n, k, padded, stream);
+    if (tile < 0) tile = row_prefill_tile(tokens, n);
+    switch (tile) {
+        case 0: break;
+        case 4: launch_row_prefill<HB, 4, 2, 2, 4, 2>(x, codes, high, scales, out, tokens, n, k, padded, stream); break;
+        case 5: launch_row_prefill<HB, 4, 2, 4, 5, 2>(x, codes, high, scales, out, tokens, n, k, padded, stream); break;
+        case 6: launch_row_prefill<HB, 4, 2, 4, 6, 2>(x, codes, high, scales, out, tokens, n, k, padded, stream); break;
+        default: launch_row_prefill<HB, 4, 2, 4, 7, 1>(x, codes, high, scales, out, tokens, n, k, padded, stream); break;
+    }
 }
 
 void row_gemm_launch(const void* x, const void* codes, const void* high, const void* scales, void* out, int tokens,

@@ -481,28 +481,33 @@ void launch_split(const Q4Operands& o, hipStream_t stream) {
 
 }  // namespace
 
-// Runs the projection unless the 256-token tiles of row_prefill are the faster
-// ones for this shape (false: nothing was launched). Operands are admitted by
-// the caller.
-bool q4_prefill_launch(const __half* x, const std::uint8_t* codes, const __half* scales, __half* out, int tokens, int n,
-                       int k, int padded, hipStream_t stream) {
-    if (k > kNarrowK) return false;  // rows too long for 32-bit lane offsets
+// Runs the projection and returns 0, or launches nothing and returns the tile of
+// row_prefill that is the fastest for this shape (4: 128 tokens x 128 rows; 5, 6
+// and 7: 256 tokens x 32 times that many rows). Operands are admitted by the
+// caller; rows of more than kNarrowK columns, past the 32-bit lane offsets, are
+// left to row_prefill's own rule (-1).
+int q4_prefill_launch(const __half* x, const std::uint8_t* codes, const __half* scales, __half* out, int tokens, int n,
+                      int k, int padded, hipStream_t stream) {
+    if (k > kNarrowK) return -1;
     const Q4Operands o{x, codes, scales, out, tokens, n, k, padded};
-    // The tiling with the least predicted time; the last three are row_prefill's
-    // 256 x 160 / 192 / 224 tiles, which read fewer LDS bytes per MFMA and win
-    // where whole rounds of them fill the chip (2048 tokens x 34816 rows: 736 us
-    // against 885). The constants are a fit to 105 shapes (32-2600 tokens,
-    // 1024-34816 rows, 1024-25600 columns; each candidate timed on each shape on
-    // MI355X): the choice is within 18% of the fastest candidate on every one of
-    // them and 0.9% on average.
-    constexpr PrefillTiling kTilings[11] = {
-        {128, 128, 1, 0.0, 6.69, 7.98, 7.98},   {64, 128, 1, 1.0, 4.13, 5.82, 5.82},   {64, 64, 1, 1.1, 4.61, 2.90, 2.90},
-        {64, 64, 2, 2.9, 3.02, 3.12, 5.97},     {48, 64, 2, 4.0, 1.29, 2.71, 5.09},    {48, 64, 1, 1.4, 3.62, 2.44, 2.44},
-        {32, 64, 1, 3.3, 1.31, 1.98, 1.98},     {32, 32, 1, 2.6, 0.65, 1.49, 1.49},    {256, 160, 1, 0.0, 6.08, 19.97, 19.97},
-        {256, 192, 1, 0.0, 6.69, 21.83, 21.83}, {256, 224, 1, 0.0, 6.97, 23.96, 23.96}};
-    int best = fastest_tiling(kTilings, tokens, n, k);
-    if (best >= 8) return false;
-    if (best >= 2 && k < 128) best = 1;  // the split form needs one whole chunk
+    // The tiling with the least predicted time; the last four are row_prefill's,
+    // whose 256-token tiles read fewer LDS bytes per MFMA and win where whole
+    // rounds of them fill the chip (2048 tokens x 34816 rows: 736 us against
+    // 885), and whose 128 x 128 tile, two workgroups to a CU, wins where K is
+    // short (128 tokens x 34816 rows x 1024: 26 us in the others, 21). The
+    // constants are a fit to 770 shapes (33-8192 tokens, 256-151936 rows,
+    // 64-25600 columns; each candidate timed on each shape on MI355X): the choice
+    // is within 12% of the fastest candidate on every one of them and 0.3% on
+    // average.
+    constexpr PrefillTiling kTilings[12] = {
+        {128, 128, 1, 0.0, 6.71, 7.70, 7.70},   {64, 128, 1, 0.8, 4.25, 6.10, 6.10},    {64, 64, 1, 1.4, 2.85, 3.36, 3.36},
+        {64, 64, 2, 2.1, 3.01, 3.40, 6.13},     {48, 64, 2, 2.7, 1.38, 2.59, 5.08},     {48, 64, 1, 0.7, 3.53, 2.43, 2.43},
+        {32, 64, 1, 3.0, 0.92, 2.20, 2.20},     {32, 32, 1, 1.3, 1.08, 1.76, 1.76},     {128, 128, 2, 1.3, 2.95, 9.09, 17.27},
+        {256, 160, 1, 0.0, 7.58, 19.63, 19.63}, {256, 192, 1, 1.6, 8.60, 21.28, 21.28}, {256, 224, 1, 0.7, 7.86, 23.88, 23.88}};
+    // (Past row_prefill's launch grid of 65535 token tiles, the forms here take every shape.)
+    int best = tokens <= 65535 * 128 ? fastest_tiling(kTilings, tokens, n, k) : 0;
+    if (best >= 2 && k < 128) best = 8;  // the split form needs one whole chunk
+    if (best >= 8) return best - 4;
     switch (best) {
         case 0: launch_coop<1, 2, 4, 8, 4>(o, stream); break;
         case 1: launch_coop<1, 2, 4, 4, 4>(o, stream); break;
@@ -513,7 +518,7 @@ bool q4_prefill_launch(const __half* x, const std::uint8_t* codes, const __half*
         case 6: launch_split<8, 2, 4>(o, stream); break;
         default: launch_split<8, 2, 2>(o, stream); break;
     }
-    return true;
+    return 0;
 }
 
 }  // namespace vt
