@@ -81,12 +81,17 @@ def epsilon(value):
 # host side sets the rate of a chain of such calls. Reading the raw stream and
 # the current device takes 0.1 us each where a Stream object takes 1.8 us and
 # entering torch.cuda.device 1.2 us; one span per operand makes disjoint() over
-# five tensors 0.9 us instead of 2.9 us. Per run(): 12.5 -> 7.5 us.
+# five tensors 0.9 us instead of 2.9 us. Per run(): 12.5 -> 7.5 us. Both readings
+# are torch-internal names; a torch without them gets the public calls.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def stream_of(device):
     """The raw hipStream_t of the device's current torch stream."""
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 _CURRENT = nullcontext()
@@ -94,4 +99,4 @@ _CURRENT = nullcontext()
 
 def on_device(device):
     """``torch.cuda.device(device)`` where the calling thread's current device is another one."""
-    return _CURRENT if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+    return _CURRENT if _current_device() == device.index else torch.cuda.device(device)
