@@ -239,11 +239,13 @@ def test_q4_tilings_place_every_product(backend, device, tokens, n, k):
     assert_exact(out, x.double(), values(signed, scales, k))
 
 
-# The split form over the tiled planes: one, two and three row blocks per workgroup, four K waves past 768 blocks;
-# K below one chunk, partial chunks, odd group counts; up to 16 tokens where the activations exceed the decode LDS.
+# The split form over the tiled planes: one, two and three row blocks per workgroup, four K waves past 768 blocks (past
+# 1024 at up to 16 tokens); K below one chunk, partial chunks, odd group counts; up to 16 tokens where the activations
+# exceed the decode LDS, and there the register form at 513-768 row blocks (test_launches.py checks what is reached).
 A8_TILED_SHAPES = [(17, 4096, 1000, 1), (32, 70, 31, 2), (31, 33, 97, 1), (20, 500, 4000, 2), (24, 5120, 519, 1),
                    (32, 7167, 2056, 2), (17, 11702, 391, 2), (32, 12300, 136, 1), (25, 20001, 264, 2),
-                   (16, 300, 16392, 2), (12, 5000, 17408, 2), (16, 13000, 5120, 2), (9, 17000, 12296, 1)]
+                   (16, 300, 16392, 2), (12, 5000, 17408, 2), (16, 13000, 5120, 2), (9, 17000, 12296, 1),
+                   (16, 17000, 5128, 2), (13, 16999, 12296, 2), (12, 300, 30000, 2), (12, 9001, 15240, 2), (16, 9001, 30001, 1)]
 
 
 @pytest.mark.parametrize("tokens,n,k,passes", A8_TILED_SHAPES)

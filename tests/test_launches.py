@@ -123,3 +123,35 @@ def test_q4_prefill_of_short_rows_and_of_rows_past_the_lane_offsets_takes_the_ti
     for shape, launched in zip(short, kernels([(0, *q4_gemm(*shape)) for shape in short])):
         assert launched == ["row_prefill<0, 4, 2, 2, 4, 2, 1>"], (shape, launched)
     assert kernels([(0, *q4_gemm(256, 64, (1 << 22) + 8))])[0][0].startswith("row_prefill<0, 4, 2, 4, ")
+
+
+def a8_tiled_linear(tokens, n, k, passes):
+    x, workspace, codes, scales, out, slots = pointers(6)
+    return "venturi_q8_a8_tiled_linear_run", [x, workspace, 1 << 35, codes, scales, out, tokens, n, k, padded(k), passes,
+                                              slots, 1 << 30, None]
+
+
+def test_a8_tiled_tests_reach_every_form_without_an_lds_copy():
+    assert built("a8_tiled_split") | built("a8_tiled_decode") <= reached([a8_tiled(*shape) for shape in tilings.A8_TILED_SHAPES])
+
+
+def test_a8_projection_keeps_the_one_launch_order():
+    """Quantizing and projecting in one launch or in two gives the same bytes where the workgroup shape is the same:
+    wherever the one-launch form serves run(), project() takes the staged form, in its shape unless it splits K (long rows
+    of 257-384 row blocks)."""
+    shapes = [(t, n, k, p) for t in (1, 3, 8, 9, 16) for n in (16, 4096, 4097, 8176, 8192, 8208, 12288, 12300, 17000, 34816)
+              for k in (8, 128, 1000, 2048, 4096, 6144, 9000, 14336, 17408, 30000) for p in (1, 2)]
+    one = record([(0, *a8_tiled_linear(*shape)) for shape in shapes])
+    two = record([(0, *a8_tiled(*shape)) for shape in shapes])
+    served = 0
+    for shape, run, project in zip(shapes, one, two):
+        run, project = ([e for e in events if isinstance(e, Launch)] for events in (run, project))
+        assert len(project) == 1
+        if len(run) == 1:  # no separate quantizer
+            served += 1
+            fused, staged = (e.kernel.split("<")[1].replace(" ", "").split(",") for e in (run[0], project[0]))
+            assert run[0].kernel.startswith("a8_tiled_lds<") and project[0].kernel.startswith("a8_tiled_lds<"), shape
+            if not staged[5].startswith("2"):  # workgroups that share a row block's K
+                assert fused[:4] == staged[:4], shape
+                assert (run[0].blocks, run[0].threads) == (project[0].blocks, project[0].threads), shape
+    assert served > 100

@@ -22,26 +22,27 @@
 // [2 groups]), and its activation scales are the two of its own token. B
 // fragments are 8 bytes of the token's group codes at [group][8q ..].
 //
-// Three forms share that arithmetic (17-32 tokens, and fewer whose activations
-// exceed the LDS of these forms, run the split form of the prefill GEMM over
-// the tiled planes, a8_fast.hip):
+// Three forms share that arithmetic, for up to 16 tokens (17-32 tokens, and
+// fewer whose activations exceed the LDS of the staged form, run the split form
+// of the prefill GEMM over the tiled planes, a8_fast.hip, except where the first
+// form below is the faster one):
 // * a8_tiled_decode reads a filled A8 workspace ([pass][token][group][32]
 //   codes, then fp32 scales [pass][token][group]) from global memory, each
-//   lane its own B fragments (up to 16 tokens);
+//   lane its own B fragments (513-768 row blocks whose activations exceed the
+//   LDS of the staged form);
 // * a8_tiled_lds<STAGE = true> copies a filled workspace into LDS once per
-//   workgroup (up to 16 tokens where the copy fits one round of loads and the
-//   LDS keeps the shape's workgroups resident), and its waves read their B
-//   fragments from LDS: the per-lane 8- and 4-byte fragment loads of the
-//   first form, repeated by every workgroup, become one coalesced copy;
-// * a8_tiled_lds<STAGE = false> (a8_tiled_fused; up to 16 tokens, k % 8 == 0,
-//   its activations within 64 KB of LDS) quantizes the fp16 activations
+//   workgroup (where the copy fits one round of loads and the LDS keeps the
+//   shape's workgroups resident), and its waves read their B fragments from
+//   LDS: the per-lane 8- and 4-byte fragment loads of the first form, repeated
+//   by every workgroup, become one coalesced copy;
+// * a8_tiled_lds<STAGE = false> (a8_tiled_fused; k % 8 == 0, its activations within 64 KB of LDS) quantizes the fp16 activations
 //   itself: each workgroup issues its first two weight batches, quantizes
 //   every token's groups into LDS with the quantizer's arithmetic (workgroup 0
 //   also writes them to the workspace, so the workspace ends as the quantizer
 //   leaves it), and reads its B fragments from LDS. One launch replaces the
 //   quantizer's and the projection's.
-// The group sums and their order depend only on the workgroup shape, which
-// all three take from one table: at one shape they give the same bytes.
+// The group sums and their order depend only on the workgroup shape: at one
+// shape, the three give the same bytes.
 //
 // Launch: W waves over RB row blocks per workgroup, the chunks split evenly
 // over the waves, two batches of one chunk in flight per wave (the loads are
@@ -529,7 +530,7 @@ __global__ __launch_bounds__(W * 64) void a8_tiled_lds(const __half* x, const st
     }
 }
 
-// Workgroup shape of both kernels (unsplit K): W waves over RB row blocks,
+// Workgroup shape of the LDS forms (unsplit K): W waves over RB row blocks,
 // NBUF batches in flight per wave: 16 waves over one row block up to 256
 // blocks, over two up to 511 (grids of at most 256 workgroups, one per CU),
 // else 8 waves over three.
@@ -562,15 +563,12 @@ void visit_one_block_shape(const A8Shape& sh, F&& f) {
     visit_shape<ShapeTag<16, 1, 2>, ShapeTag<16, 2, 2>, ShapeTag<8, 3, 2>>(sh, f);
 }
 
+// The register form serves only grids of 8-wave workgroups over three row blocks.
 template <int P>
-void dispatch_a8_tiled(const std::int8_t* acodes, const float* ascales, const uint4* codes, const uint4* scales,
-                       __half* out, int tokens, int n, int groups, int chunks, int blocks, hipStream_t stream) {
-    auto launch = [&](auto tag) {
-        using T = decltype(tag);
-        a8_tiled_decode<T::waves, T::rb, P, T::nbuf><<<(blocks + T::rb - 1) / T::rb, T::waves * 64, 0, stream>>>(
-            acodes, ascales, codes, scales, out, tokens, n, groups, chunks, blocks);
-    };
-    visit_one_block_shape(a8_shape(blocks), launch);
+void launch_a8_tiled(const std::int8_t* acodes, const float* ascales, const uint4* codes, const uint4* scales,
+                     __half* out, int tokens, int n, int groups, int chunks, int blocks, hipStream_t stream) {
+    a8_tiled_decode<8, 3, P, 2><<<(blocks + 2) / 3, 8 * 64, 0, stream>>>(acodes, ascales, codes, scales, out, tokens, n,
+                                                                        groups, chunks, blocks);
 }
 
 // LDS bytes of a8_tiled_lds: the activation rows of the workgroup's groups
@@ -634,8 +632,8 @@ void validate_a8_tiled(const void* workspace, std::uint64_t available, const voi
 // one workgroup's share of the CU splits K over two workgroups of 16 waves and
 // three row blocks, which exchange their halves through slots, where that grid
 // runs in at most two rounds of one workgroup per CU, or where rows of at
-// least 128 chunks in 257-384 blocks would leave CUs idle), else the register
-// form.
+// least 128 chunks in 257-384 blocks would leave CUs idle), else one of the
+// forms without an LDS copy of the activations.
 struct A8TiledPlan {
     bool staged;
     A8Shape shape;
@@ -704,19 +702,18 @@ void a8_tiled_launch(const void* workspace, std::uint64_t available, const void*
         return;
     }
     // Past 16 tokens, and where one token block's activations exceed the LDS of
-    // the forms above, the split form of the prefill GEMM reads the tiled
+    // the staged form, the split form of the prefill GEMM reads the tiled
     // planes. (Between 513 and 768 row blocks the register form stays the
-    // faster one at 9-16 tokens: 15232 columns x 732 blocks at 12 tokens, two
+    // faster one at up to 16 tokens: 15232 columns x 732 blocks at 12 tokens, two
     // passes, 59 against 65 us; 1088 blocks against it 72 -> 67, 320 blocks 63
-    // -> 49. Where the one-launch form could also serve the call, both steps
-    // keep its order of sums.)
-    const bool one_launch = a8_lds_bytes(tokens, groups, passes, a8_shape(blocks)) <= kA8FusedLdsMax;
-    if (tokens > 16 || (!one_launch && (blocks <= 512 || blocks > 768)))
+    // -> 49. Whatever the one-launch form can serve, within 64 KB of LDS, is
+    // staged above, with its order of sums.)
+    if (tokens > 16 || blocks <= 512 || blocks > 768)
         a8_tiled_split_launch(workspace, codes, scales, out, tokens, n, k, padded, passes, stream);
     else if (passes == 1)
-        dispatch_a8_tiled<1>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
+        launch_a8_tiled<1>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
     else
-        dispatch_a8_tiled<2>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
+        launch_a8_tiled<2>(acodes, ascales, cp, sp, op, tokens, n, groups, chunks, blocks, stream);
 }
 
 void a8_tiled_linear_launch(const void* x, void* workspace, std::uint64_t available, const void* codes,

@@ -488,8 +488,8 @@ __global__ __launch_bounds__(WK * 64, 2) void a8_prefill_split(const std::int8_t
 
 // The split form over the tiled Q8 planes (the decode route's copy: codes
 // [row block][64-column chunk][lane 16q + m][two groups' 8 bytes], scales
-// [row block][chunk][row][2]), for 17-32 tokens and for fewer whose
-// activations exceed the decode kernels' LDS. A lane's 16 code bytes are its
+// [row block][chunk][row][2]), for 17-32 tokens, and for fewer whose
+// activations exceed the decode kernels' LDS outside 513-768 row blocks. A lane's 16 code bytes are its
 // fragments of a chunk's two groups and its 16 scale bytes the four rows'
 // pairs, so weights go straight to registers in 1 KB wave loads; activations
 // travel through the wave's LDS region as in the row-major form.
@@ -761,23 +761,29 @@ void a8_tiled_split_launch(const void* workspace, const void* codes, const void*
     const auto* sp = static_cast<const u32x4*>(scales);
     auto* op = static_cast<__half*>(out);
     const int blocks = (n + 15) / 16;
-    auto launch = [&](auto waves, auto row_blocks) {
-        if (tokens > 16)
-            launch_tiled_split<waves, 2, row_blocks>(acodes, ascales, cp, sp, op, tokens, n, padded, groups, passes, stream);
-        else
-            launch_tiled_split<waves, 1, row_blocks>(acodes, ascales, cp, sp, op, tokens, n, padded, groups, passes, stream);
+    auto launch = [&](auto waves, auto token_blocks, auto row_blocks) {
+        launch_tiled_split<waves, token_blocks, row_blocks>(acodes, ascales, cp, sp, op, tokens, n, padded, groups, passes,
+                                                            stream);
     };
     // Row blocks per workgroup so that up to 768 blocks make at most one
     // workgroup of eight K waves per CU; beyond, four K waves and two
-    // workgroups per CU (at up to 16 tokens from 1024 blocks). MI355X, 32
+    // workgroups per CU (at up to 16 tokens past 1024 blocks). MI355X, 32
     // tokens, one pass, against the per-lane fragment form this replaces, us:
     // 4096 x 4096 19.2 -> 8.5, 7168 x 5120 24.1 -> 15.2, 5120 x 17408 71 -> 35,
     // 11702 x 15232 106 -> 43, 34816 x 5120 106 -> 45; the neighbouring shapes
     // of the rule measured up to 1.5x slower there.
-    if (blocks <= 256) launch(Slot<8>{}, Slot<1>{});
-    else if (blocks <= 512 || (tokens <= 16 && blocks <= 1024)) launch(Slot<8>{}, Slot<2>{});
-    else if (blocks <= 768) launch(Slot<8>{}, Slot<3>{});
-    else launch(Slot<4>{}, Slot<3>{});
+    if (tokens > 16) {
+        if (blocks <= 256) launch(Slot<8>{}, Slot<2>{}, Slot<1>{});
+        else if (blocks <= 512) launch(Slot<8>{}, Slot<2>{}, Slot<2>{});
+        else if (blocks <= 768) launch(Slot<8>{}, Slot<2>{}, Slot<3>{});
+        else launch(Slot<4>{}, Slot<2>{}, Slot<3>{});
+    } else if (blocks <= 256) {
+        launch(Slot<8>{}, Slot<1>{}, Slot<1>{});
+    } else if (blocks <= 1024) {  // 513-768 blocks stay with the decode kernels
+        launch(Slot<8>{}, Slot<1>{}, Slot<2>{});
+    } else {
+        launch(Slot<4>{}, Slot<1>{}, Slot<3>{});
+    }
 }
 
 }  // namespace vt
