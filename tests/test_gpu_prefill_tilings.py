@@ -44,7 +44,7 @@ Q8_SHAPES = [(257, 14003, 136), (513, 7001, 136), (1025, 7001, 136), (300, 10001
              (33, 20001, 520), (129, 7001, 1032), (81, 14003, 1000), (160, 4100, 1032), (113, 7001, 1032),
              (79, 14003, 136), (300, 4100, 136), (33, 14003, 136), (65, 10001, 200), (33, 257, 136), (97, 31, 3976),
              (700, 7001, 520), (2047, 2049, 520), (257, 10001, 520), (300, 20001, 264), (1025, 14003, 72), (129, 7001, 2056),
-             (33, 10001, 264)]
+             (33, 10001, 264), (33, 4100, 136), (47, 4100, 264)]
 
 
 @pytest.mark.parametrize("tokens,n,k", Q8_SHAPES)
