@@ -553,7 +553,7 @@ def prefill_a8(backend, device, steps, warmup, cpu_seconds):
     workspace; o_proj (K 6144) and down (K 17408) quantize seeded N(0, 1)
     activations with the plain A8 quantizer. Each stage runs `steps` times back
     to back between one pair of events; TOPS = 2*M*N*K / average time. The
-    GEMMs run on the plan's auto route (matrix cores, natural group order);
+    GEMMs run on the plan's auto route (matrix cores, free fp32 order);
     the reference-order route is timed beside it and its outputs are the
     parity reference.
     """

@@ -59,9 +59,9 @@ int venturi_q8_dp4a_run(const void* workspace, uint64_t available, const int8_t*
                         void* out, int tokens, int n, int k, int padded, int passes, void* stream);
 
 /* Extension (no counterpart in the reference): the same W8A8 projection on
- * int-exact fp16 matrix cores, with the 32-column group dots exact (as the
- * reference's int32 accumulators) and the scaled group terms summed in
- * natural order, so outputs match the reference to fp32 association. Same
+ * int8 matrix cores, with the 32-column group dots exact (the reference's int32
+ * accumulators) and the scaled group terms summed in a free fp32 order that the
+ * shape fixes, so outputs match the reference to fp32 association. Same
  * arguments and workspace as venturi_q8_dp4a_run. */
 int venturi_q8_a8_gemm_run(const void* workspace, uint64_t available, const int8_t* codes, const void* scales,
                            void* out, int tokens, int n, int k, int padded, int passes, void* stream);
@@ -70,8 +70,9 @@ int venturi_q8_a8_gemm_run(const void* workspace, uint64_t available, const int8
  * 1..32 tokens on int8 matrix cores (v_mfma_i32_16x16x32_i8: one exact int32
  * group dot per 32-column group) over the tiled Q8 planes that
  * venturi_q8_tiled_run reads (codes [block][chunk][lane][16 B], scales
- * [block][chunk][row][2]); the scaled group terms summed in natural order, so
- * outputs match the reference to fp32 association. Same workspace as
+ * [block][chunk][row][2]); the scaled group terms summed in a free fp32 order
+ * that the shape fixes, so outputs match the reference to fp32 association.
+ * Same workspace as
  * venturi_q8_dp4a_run; workspace and planes 16-byte aligned. Shapes whose
  * launch splits K over two workgroups take `slots`: at least
  * venturi_q8_a8_tiled_workspace_bytes bytes, 8-byte aligned, armed once with

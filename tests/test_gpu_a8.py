@@ -182,7 +182,7 @@ def check_a8_tolerance(got_bits, q, d, wcodes, wscales, k, expected_bits):
     """The mfma route against FP64 over the exact group dots and against the reference order.
 
     FP64: y = sum_p sum_g dot_pg * fp32(ws_g * as_pg), the reference's per-group
-    terms; the fp32 natural-order sum may differ from it by at most
+    terms; the fp32 sum, in whatever order, may differ from it by at most
     G * 2^-24 * sum|terms| plus the final fp16 rounding (half an ulp).
     Reference order: every output within max(2e-3, 1 fp16 ulp) and rel-L2 <= 1e-3
     (the stated tolerance for fp16 outputs).

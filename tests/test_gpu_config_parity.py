@@ -178,7 +178,7 @@ def test_rms_a8_config3_input(backend, device, passes):
     np.testing.assert_array_equal(bits(inter), y)
     np.testing.assert_array_equal(workspace.cpu().numpy(), oracle.a8_workspace(q, d))
     # The config-3 QKV projection on this workspace (auto route: matrix cores,
-    # natural group order) on sampled rows against the reference-order oracle.
+    # free fp32 order) on sampled rows against the reference-order oracle.
     packed = _packed(backend, device, QKV, k, 33)
     resident = backend.upload_linear(packed, dtype=torch.float16, device=device)
     gemm = prepare_q8_dp4a(resident, tokens=m, residual_compensation=passes == 2)

@@ -710,9 +710,9 @@ VT_EXPORT int venturi_q8_dp4a_run(const void* workspace, std::uint64_t available
 }
 
 // Extension: the same W8A8 projection on matrix cores with the groups summed
-// in natural order (exact int32 group dots, fp32 association differs from the
-// reference's lane-slot tree); same arguments and workspace as
-// venturi_q8_dp4a_run.
+// in a free fp32 order that shape and tiling fix (exact int32 group dots, fp32
+// association differs from the reference's lane-slot tree); same arguments and
+// workspace as venturi_q8_dp4a_run.
 VT_EXPORT int venturi_q8_a8_gemm_run(const void* workspace, std::uint64_t available, const std::int8_t* codes,
                                      const __half* scales, void* out, int tokens, int n, int k, int padded,
                                      int passes, void* stream) {

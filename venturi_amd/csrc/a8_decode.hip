@@ -9,9 +9,10 @@
 // (q8_dp4a.cuh:47-58): one v_mfma_i32_16x16x32_i8 per group and 16 x 16
 // tile, accumulating from zero, so the integer accumulator is the
 // reference's. The group terms use the reference's products and FMA but are
-// summed in natural group order into one fp32 per output (the reference
-// combines 32 lane slots through a shuffle tree), so outputs agree with the
-// reference to fp32 association, as the matrix-core A8 prefill GEMM.
+// summed per wave, in the order of its groups, and over the waves in wave order
+// (the reference combines 32 lane slots through a shuffle tree), so outputs
+// agree with the reference to fp32 association, as the matrix-core A8 prefill
+// GEMM.
 //
 // The MFMA computes the transposed tile: A is 16 weight rows x 32 codes, B is
 // 32 activation codes x 16 tokens, so lane (q, r) of D holds rows 4q .. 4q+3
@@ -753,7 +754,8 @@ void a8_tiled_linear_launch(const void* x, void* workspace, std::uint64_t availa
 // Extension: the W8A8 projection of venturi_q8_dp4a_run at 1..32 tokens on
 // int8 matrix cores over the tiled Q8 planes (the layout of
 // venturi_q8_tiled_run); same A8 workspace; outputs equal the reference's up
-// to fp32 association (exact int32 group dots, groups summed in natural order).
+// to fp32 association (exact int32 group dots, scaled terms summed in a free
+// fp32 order that the shape fixes).
 // Shapes whose launch splits K take an exchange-slot buffer of
 // venturi_q8_a8_tiled_workspace_bytes bytes, armed once with
 // venturi_q8_tiled_workspace_init and left idle by every run.

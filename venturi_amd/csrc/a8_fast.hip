@@ -12,24 +12,33 @@
 // because 1.5 * 2^23 * ws is exact (an 11-bit significand times 3); then
 // y = fma(t, as, y). Two VALU instructions per output and group, as the
 // reference's product and FMA (q8_dp4a.cuh:59-70), with one fp32 rounding
-// besides the sum's as there. Groups are summed in natural order per wave and
-// the waves that split K afterwards, so outputs agree with the reference to
-// fp32 association, not bit for bit. The second pass of the residual profile
-// is a second run over the same weight columns. (A row with a non-finite
-// weight scale, which the format excludes, gives NaN.)
+// besides the sum's as there. A wave sums its groups in the order it visits
+// them (the passes' last, perhaps partial, stages or chunks first, then the
+// others of each pass from column 0 up) and the sums of the waves that split K
+// are added in wave order. The order depends on shape and tiling only: outputs
+// are deterministic and agree with the reference to fp32 association, not bit
+// for bit. The second pass of the residual profile is a second run over the
+// same weight columns. (A row with a non-finite weight scale, which the format
+// excludes, gives NaN.)
 //
-// What binds it is VALU issue: eight instructions (32 cycles) per 16 x 16 tile
-// and group against one MFMA of 16 cycles. So the two forms (cooperative and
-// split, prefill.hpp) keep everything else off the VALU: codes go from memory
-// through LDS into the MFMA unconverted, an operand is replaced by the next
-// group's as soon as its last use is issued, and a tile's MFMA is issued four
-// tiles before its VALU work. Measured on MI355X against the form this
+// Per 16 x 16 tile and group there are eight VALU instructions beside one MFMA
+// of 16 cycles. So the two forms (cooperative and split, prefill.hpp) keep
+// everything else off the VALU: codes go from memory through LDS into the MFMA
+// unconverted, an operand is replaced by the next group's as soon as its last
+// use is issued, and a tile's MFMA is issued four tiles before its VALU work.
+// What binds it then is closest to the VALU, but not that alone. Counters,
+// [34816 x 5120] at 2048 tokens: 10.1 VALU instructions per MFMA, VALU busy at
+// most 69% of the time (4 cycles per instruction; an FMA measured 2.7 in a
+// dense loop, which gives 46%), matrix cores 27%, LDS 20%, waves waiting 26% of
+// theirs, two waves per SIMD. Measured on MI355X against the form this
 // replaces (codes converted to fp16 once per workgroup, one 8-wave workgroup
 // per 128- or 256-token tile, a barrier per group), us:
 //   tokens x [7168 x 5120]: 64: 114 -> 18, 200: 119 -> 38, 512: 129 -> 66;
 //   [5120 x 17408]: 64: 395 -> 54, 512: 422 -> 175;
-//   [34816 x 5120], 2048 tokens: 1794 -> 1135 (643 TOP/s; the VALU work alone
-//     would take about 700 us).
+//   [34816 x 5120], 2048 tokens: 1794 -> 1135 (643 TOP/s).
+// At 100-128 tokens over 34816 rows of 64-512 columns, and at 1024 tokens over
+// very many rows of up to 136, it is 1.12-1.20 times the time of the replaced
+// form: prologue and output, not the K loop, are the time there.
 #include "prefill.hpp"
 
 #include <algorithm>

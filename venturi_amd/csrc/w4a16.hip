@@ -10,11 +10,14 @@
 // prefill.hpp; the activation fragments are replaced in place and the next
 // slice's weights are dequantized beside the MFMAs of the current one.
 //
-// What binds it at these token counts: LDS (320 bytes read per MFMA at 128 x 64
-// wave tiles) and the dequantization per wave; the 256-token tiles of
-// row_prefill, whose workgroup dequantizes a weight once, stay the faster form
-// from about 1000 tokens on. Measured on MI355X against row_prefill at every
-// token count (grids of 128- and 256-token tiles, K serial), us:
+// What binds it at these token counts: no unit alone. Counters, [5120 x 25600]
+// at 128 tokens: 7.2 VALU instructions per MFMA (the dequantization per wave),
+// VALU busy at most 41% of the time, matrix cores 23%, LDS 34% (320 bytes read
+// per MFMA at 128 x 64 wave tiles; waves wait for it 14% of theirs), any wait
+// 34%; one 64-column step of activations is in flight per wave. The 256-token
+// tiles of row_prefill, whose workgroup dequantizes a weight once, stay the
+// faster form from about 1000 tokens on. Measured on MI355X against row_prefill
+// at every token count (grids of 128- and 256-token tiles, K serial), us:
 //   tokens x [7168 x 5120]: 64: 56 -> 15.4, 200: 56 -> 32, 512: 107 -> 49;
 //   [5120 x 25600]: 128: 269 -> 64, 512: 537 -> 208.
 #include "prefill.hpp"

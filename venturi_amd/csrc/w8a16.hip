@@ -5,33 +5,44 @@
 //
 // Each 32-column group's D is one v_mfma_f32_16x16x32_f16 on the fp16
 // activations and the int8 codes converted to fp16 exactly (every x * code
-// product is exact in fp32); the group scale is one fp32 FMA per (t, n, g),
-// each wave's groups summed in natural order and the waves that split K
-// afterwards, so outputs agree with the canonical order (blocks.cu:306-321) to
-// fp32 association, like the decode route.
+// product is exact in fp32); the group scale is one fp32 FMA per (t, n, g).
+// A wave sums its groups in the order it visits them (cooperative: the partial
+// stage first, then the others from column 0 up; split: its chunks from the
+// last one down, a chunk's groups upwards), and the sums of the waves that
+// split K are added in wave order. The order depends on shape and tiling only,
+// so outputs are deterministic and agree with the canonical order
+// (blocks.cu:306-321) to fp32 association, like the decode route.
 //
 // Two forms (prefill.hpp), chosen per shape by a measured time model:
 // * cooperative (q8_prefill): WT x WN x WK waves compute (WT*TI*16) tokens x
 //   (WN*TJ*16) rows; a stage is WK groups, staged in two LDS buffers
 //   (activations as fp16, codes biased to unsigned), one group per K wave, one
-//   barrier per stage. For grids that fill the chip.
+//   barrier per stage. For grids that fill the chip; with short rows its
+//   tilings of four waves that do not split K (64 x 128 and 128 x 128), which
+//   need no sum and leave room for two to four workgroups per CU.
 // * split (q8_prefill_split): each of WK waves computes the whole TI*16 x TJ*16
 //   tile over its own 128-column chunks through its own LDS region; no barrier
 //   before the sum. For the small grids of short prompts, where it fills the
 //   CUs with K instead of tiles.
 //
-// What binds them is instruction issue: per 16 x 16 tile and group one MFMA
-// (16 cycles of the matrix cores) and four scaling FMAs (16 cycles of the
-// VALU), plus a tile row's share of the code conversion. So both forms issue a
-// tile's MFMA four tiles before its FMAs, replace each activation fragment by
-// the next group's as soon as its last MFMA is issued, and pin that order with
-// scheduling barriers; LDS, memory and matrix work then overlap within a wave.
+// What binds them: no unit alone. Per 16 x 16 tile and group there are one MFMA
+// and four scaling FMAs, plus a tile row's share of the code conversion, so
+// both forms issue a tile's MFMA four tiles before its FMAs, replace each
+// activation fragment by the next group's as soon as its last MFMA is issued,
+// and pin that order with scheduling barriers. Counters, [34816 x 5120] at 2048
+// tokens / [7168 x 5120] at 200: matrix cores busy 33 / 19% of the time, VALU
+// at most 56 / 38% (4 cycles per instruction; an FMA measured 2.7 in a dense
+// loop), LDS active 31 / 30%, waves waiting 35 / 32% of theirs. The shares add
+// up to about the whole: with the two waves per SIMD that the registers leave
+// room for, matrix, VALU and LDS work still run largely one after another.
 // Measured on MI355X against one workgroup of 8 waves with a barrier per group
 // (the form this replaces), us:
 //   tokens x [7168 x 5120]:  64: 74.6 -> 17.0, 200: 76.5 -> 33.3, 512: 77.3 -> 55,
 //     1024: 137 -> 101; [5120 x 17408]: 64: 255 -> 43, 512: 267 -> 178;
-//   [34816 x 5120], 2048 tokens: 1210 -> 1030 (710 TFLOP/s; the wave's VALU and
-//     MFMA issue alone would take about 640).
+//   [34816 x 5120], 2048 tokens: 1210 -> 1030 (710 TFLOP/s).
+// Up to about 256 columns over 16384 or more rows, and at 100-128 tokens over
+// 34816 rows of 64-512, it is up to 1.14 (at 64 columns 1.24) times the time of
+// the replaced form: prologue and output, not the K loop, are the time there.
 #include "prefill.hpp"
 
 #include <algorithm>

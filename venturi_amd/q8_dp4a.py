@@ -9,16 +9,18 @@ fp16 activations into a caller-owned workspace (``workspace_bytes`` bytes,
 * ``exact``: groups combined in fp32 in the reference's lane-slot and
   shuffle-tree order (SIMT below 64 tokens, matrix cores above), so the fp16
   outputs are byte-identical to the reference's;
-* ``mfma``: matrix cores with the scaled group terms summed in natural order
-  (one accumulator per output), equal to the reference up to fp32
+* ``mfma``: matrix cores with the scaled group terms summed in a free fp32
+  order (fixed by the shape), equal to the reference up to fp32
   association: up to 32 tokens the int8 decode kernel over the resident's
   tiled planes (``venturi_q8_a8_tiled_run``, the layout of the A16 decode
   route, built once per resident; ``run`` quantizes and projects in one
   launch through ``venturi_q8_a8_tiled_linear_run`` where the activations
-  fit), above that the prefill GEMM's large tiles;
+  fit), above that the prefill GEMM;
 * ``auto``: ``mfma`` up to 32 tokens and from 64 (decode and prefill),
-  ``exact`` between (the SIMT kernel streams the weights there, and the
-  prefill GEMM's 256-token tiles would mostly hold padding).
+  ``exact`` between. The SIMT kernel streams the weights once per four tokens
+  there and the prefill GEMM would be the faster one (64 tokens of
+  [7168 x 5120] take it 18 us); the route of these counts is kept as plans
+  have reported it and as their bytes have been.
 """
 
 from dataclasses import dataclass

@@ -48,9 +48,11 @@ from .operands import DTYPE_CODES, admit, disjoint, extents, on_device, stream_o
 
 EXACT_MAX_AUTO_TOKENS = 0
 MFMA_MAX_TOKENS = 32
-# The dense route decodes and writes 4 bytes per weight before its GEMM, so it
-# pays only at large token counts: config-2 shapes against the fused GEMM at
-# 1024 tokens 0.87-1.28x (gate+up and down slower), at 2048 1.13-1.21x.
+# From this token count plans take the dense route when they are given its
+# workspace. It decodes and writes 4 bytes per weight before its GEMM, and the
+# fused GEMM has since passed it: config-2 shapes at 2048 tokens, dense / fused
+# us: QKV 283 / 272, o_proj 246 / 235, gate+up 1186 / 1051, down 703 / 567. The
+# route and its workspace size are part of what a plan promises and stay.
 DENSE_TOKENS = 2048
 DENSE_MAX_SCALE = 516.0  # 127 * 516 rounds past the fp16 range
 RESIDENCIES = ("row-major", "tiled", "tiled-paired")
